@@ -299,9 +299,9 @@ int kivi_packed_decode_attention_noalloc(
  * positions 0 .. kv_start[b]-1, quantised or in the window); each must leave
  * every query token at least one visible position (for causal queries:
  * kv_start[b] <= num_chunks*G + res_len - q_len).
- * When q_len * (q_heads / kv_heads) exceeds 8 the tokens are split over
- * several launches (and more than 8 query heads per kv head into groups of
- * 8), each streaming the store once.  No reference counterpart
+ * When q_len * (q_heads / kv_heads) exceeds 8, a matrix-core store is
+ * dequantised once for up to 256 query rows of a kv head at a time; a
+ * plain-layout store is streamed once per 8 rows.  No reference counterpart
  * beyond that math (the reference runs HF attention on the CPU,
  * src/kivi_sycl/cache/manager.py:251-290). */
 size_t kivi_packed_attention_workspace_size(int32_t batch, int32_t q_len, int32_t q_heads,

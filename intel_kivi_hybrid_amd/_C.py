@@ -450,11 +450,16 @@ def quant_dequant_roundtrip_values_async(input, output, head_dim, group_size):
 # include/kivi_hip.h).  Not part of the reference's twelve ops.
 # --------------------------------------------------------------------------
 _ws_cache = {}
+_WS_KEPT = 16 << 20      # largest workspace kept per stream (a decode step's take a few MB)
 
 
 def _workspace(device, nbytes: int):
     if nbytes == 0:
         return None
+    if nbytes > _WS_KEPT:
+        # (many query rows over several splits; torch's allocator reuses the
+        # block in stream order)
+        return torch.empty(nbytes, dtype=torch.uint8, device=device)
     key = (device_index(device), stream_handle(device))
     buf = _ws_cache.get(key)
     if buf is None or buf.numel() < nbytes:

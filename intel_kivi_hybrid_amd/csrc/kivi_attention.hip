@@ -672,20 +672,38 @@ int tokens_per_launch(int hg, int q_len, bool mfma, int D, int G, int Gv) {
     return t;
 }
 
+// Calls with more query rows per kv head than one launch of the decode kernel
+// takes run the many-row kernel (kivi_attention_rows.hip), where the store
+// has its layout.
+bool takes_rows(int q_len, int hg, int D, int G, int Gv) {
+    return q_len > 1 && (int64_t)q_len * hg > 8 && code_layout_for(D, G, Gv) == kLayoutMfma;
+}
+
 size_t workspace_for(int batch, int q_len, int q_heads, int kv_heads, int head_dim,
                      int group_size_k, int group_size_v, int num_chunks, int res_len,
                      int num_splits) {
     if (batch <= 0 || kv_heads <= 0 || q_heads <= 0 || head_dim <= 0 || group_size_k <= 0 ||
         group_size_v <= 0 || q_len <= 0 || q_heads % kv_heads)
         return 0;
+    size_t rows_need = 0;
+    if (takes_rows(q_len, q_heads / kv_heads, head_dim, group_size_k, group_size_v) &&
+        num_chunks >= 0 && res_len >= 0 && num_chunks + res_len > 0) {
+        const int rows = q_len * (q_heads / kv_heads);
+        const RowsPlan r = rows_plan(batch, kv_heads, rows, head_dim, group_size_k, num_chunks,
+                                     res_len, num_splits);
+        if (r.n_splits > 1)
+            rows_need = (size_t)batch * kv_heads * rows * r.n_splits * (head_dim + 2) *
+                        sizeof(float);
+    }
     const Plan p = make_plan(batch, kv_heads, head_dim, group_size_k, group_size_v, num_chunks,
                              res_len, num_splits);
-    if (!needs_workspace(p)) return 0;
+    if (!needs_workspace(p)) return rows_need;
     const int hl = heads_per_launch(q_heads / kv_heads,
                                     max_rows(p.mfma, head_dim, group_size_k, group_size_v));
     const int rows = rows_for(
         tokens_per_launch(hl, q_len, p.mfma, head_dim, group_size_k, group_size_v) * hl);
-    return (size_t)batch * kv_heads * rows * p.n_splits * (head_dim + 2) * sizeof(float);
+    return max(rows_need,
+               (size_t)batch * kv_heads * rows * p.n_splits * (head_dim + 2) * sizeof(float));
 }
 
 // Attention of q_len query tokens per sequence (q [batch][q_len][q_heads]
@@ -756,6 +774,26 @@ int attention_impl(const float* q, int32_t q_len, int32_t causal, const int32_t*
             return set_error(kErrInvalidArgument,
                              "residual window (start %d, len %d) outside capacity %d",
                              res_start, res_len, res_capacity);
+    }
+    // (its loads and stores of queries, outputs and partials are 16 bytes wide;
+    // buffers off that alignment take the decode kernel's launches)
+    if (takes_rows(q_len, hg, head_dim, group_size_k, group_size_v) &&
+        ((uintptr_t)q | (uintptr_t)out | (uintptr_t)workspace) % 16 == 0) {
+        const int rows = q_len * hg;
+        const RowsPlan r = rows_plan(batch, kv_heads, rows, head_dim, group_size_k, num_chunks,
+                                     res_len, num_splits);
+        const size_t n_part = (size_t)batch * kv_heads * rows * r.n_splits;
+        if (r.n_splits > 1 && (!workspace || workspace_bytes < n_part * (head_dim + 2) * sizeof(float)))
+            return set_error(kErrInvalidArgument, "workspace of %zu bytes needed, got %zu",
+                             n_part * (head_dim + 2) * sizeof(float), workspace_bytes);
+        RowsLaunch L{q, k_codes, k_scale, k_zero, v_codes, v_scale, v_zero, k_res, v_res, out,
+                     (float*)workspace, (float*)workspace + n_part * head_dim, batch, q_heads,
+                     kv_heads, head_dim, group_size_k, group_size_v, chunk_capacity, num_chunks,
+                     res_capacity, res_start, res_len, res_dtype, q_len, hg, rows,
+                     causal ? res_len - (q_len - 1) : res_len, r.block_rows, r.row_blocks,
+                     r.n_units, r.n_splits, r.weight_per_split, softmax_scale * kLog2e, kv_start,
+                     hidden, hidden_stride};
+        return launch_attention_rows(L, (hipStream_t)stream);
     }
     const bool empty_ok = chunk_capacity >= 1 && k_codes && k_scale && k_zero && v_codes &&
                           v_scale && v_zero;

@@ -101,6 +101,41 @@ int launch_attention_mfma_hg2_r16(const AttnLaunch& a, hipStream_t stream);
 int launch_attention_mfma_hg4_r16(const AttnLaunch& a, hipStream_t stream);
 int launch_attention_mfma_hg8_r16(const AttnLaunch& a, hipStream_t stream);
 
+// Attention of many query rows per kv head (kivi_attention_rows.hip): query
+// row r of a kv head is query token r / hg, head r % hg, r < rows = q_len *
+// hg.  Contexts are walked in units of 32 tokens, the packed chunks' first,
+// then the window's; split s takes weight [s, s+1) * weight_per_split
+// (a packed unit 1, a window unit 2).  Query
+// token i sees every packed token and the first min(res_len, vis0 + i) of the
+// window.
+struct RowsLaunch {
+    const float* q;          // [B, q_len, Hq, D]
+    const uint8_t* k_codes;  // as AttnLaunch
+    const float* k_scale;
+    const float* k_zero;
+    const uint8_t* v_codes;
+    const float* v_scale;
+    const float* v_zero;
+    const void* k_res;
+    const void* v_res;
+    float* out;              // [B, q_len, Hq, D]
+    float* part_o;           // [B, Hkv, rows, n_splits, D] (n_splits > 1 only)
+    float* part_ml;          // [B, Hkv, rows, n_splits, 2]
+    int B, Hq, Hkv, D, G, Gv, Cmax, n_chunks, Rcap, res_start, res_len, res_dt;
+    int q_len, hg, rows, vis0;
+    int block_rows, row_blocks, n_units, n_splits, weight_per_split;
+    float qscale;            // softmax scale * log2(e)
+    const int32_t* kv_start;
+    const uint32_t* hidden;
+    int64_t hidden_stride;
+};
+struct RowsPlan {
+    int block_rows, row_blocks, n_units, n_splits, weight_per_split;
+};
+RowsPlan rows_plan(int B, int Hkv, int rows, int D, int G, int n_chunks, int res_len,
+                   int splits_hint);
+int launch_attention_rows(const RowsLaunch& a, hipStream_t stream);
+
 // LDS bytes per workgroup of the matrix-core kernel for HG query heads per
 // kv head, head_dim D, key group G and NG value groups per token (-1 for a
 // shape it has no instance of).

@@ -59,14 +59,10 @@
 
 #include "kivi_common.hpp"
 #include "kivi_attention.hpp"
+#include "kivi_mfma.hpp"
 
 namespace kivi {
 namespace {
-
-typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
-typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
-typedef float f32x4_t __attribute__((ext_vector_type(4)));
-typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
 
 constexpr int kWaves = 4;
 
@@ -100,61 +96,6 @@ __device__ __forceinline__ void wave_sync() {
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-__device__ __forceinline__ uint32_t pack_bf16x2(float a, float b) {
-    bf16x2_t v = {(__bf16)a, (__bf16)b};   // round to nearest even
-    return __builtin_bit_cast(uint32_t, v);
-}
-
-// The bf16 pairs (-1, 0) and (0, -1), held in VGPRs: split_pair's v_dot2
-// reads them as register operands.  (As literals, the compiler's encoding of
-// the (-1, 0) pair made the instruction read the pair's high half -- measured
-// on gfx950 -- so the values are hidden from it.)
-struct SplitConsts {
-    uint32_t neg_x, neg_y;
-};
-__device__ __forceinline__ SplitConsts split_consts() {
-    SplitConsts c{0x0000bf80u, 0xbf800000u};
-    asm("" : "+v"(c.neg_x));
-    asm("" : "+v"(c.neg_y));
-    return c;
-}
-
-// (a, b) -> hi and lo bf16 pairs with a ~ hi.x + lo.x, b ~ hi.y + lo.y.
-// a - hi.x is exact in fp32 (hi.x is a rounded to 8 significant bits), so
-// one v_dot2_f32_bf16 of hi with (-1, 0) accumulated onto a forms it: two
-// ops instead of widening hi's halves and subtracting (bit-identical over
-// 8.4 M random pairs on gfx950, tiny normals included).
-__device__ __forceinline__ void split_pair(float a, float b, uint32_t& hi, uint32_t& lo,
-                                           SplitConsts k) {
-    hi = pack_bf16x2(a, b);
-    const bf16x2_t h2 = __builtin_bit_cast(bf16x2_t, hi);
-    const float la = __builtin_amdgcn_fdot2_f32_bf16(h2, __builtin_bit_cast(bf16x2_t, k.neg_x), a,
-                                                     false);
-    const float lb = __builtin_amdgcn_fdot2_f32_bf16(h2, __builtin_bit_cast(bf16x2_t, k.neg_y), b,
-                                                     false);
-    lo = pack_bf16x2(la, lb);
-}
-
-// Three pieces: a ~ hi.x + mid.x + lo.x, b likewise (~2^-25 relative).  Each
-// residual is exact in fp32 (the piece taken off is the value rounded to 8
-// significant bits), so only lo's rounding remains.
-__device__ __forceinline__ void split3_pair(float a, float b, uint32_t& hi, uint32_t& mid,
-                                            uint32_t& lo, SplitConsts k) {
-    hi = pack_bf16x2(a, b);
-    const bf16x2_t h2 = __builtin_bit_cast(bf16x2_t, hi);
-    const float ra = __builtin_amdgcn_fdot2_f32_bf16(h2, __builtin_bit_cast(bf16x2_t, k.neg_x), a,
-                                                     false);
-    const float rb = __builtin_amdgcn_fdot2_f32_bf16(h2, __builtin_bit_cast(bf16x2_t, k.neg_y), b,
-                                                     false);
-    mid = pack_bf16x2(ra, rb);
-    const bf16x2_t m2 = __builtin_bit_cast(bf16x2_t, mid);
-    const float sa = __builtin_amdgcn_fdot2_f32_bf16(m2, __builtin_bit_cast(bf16x2_t, k.neg_x), ra,
-                                                     false);
-    const float sb = __builtin_amdgcn_fdot2_f32_bf16(m2, __builtin_bit_cast(bf16x2_t, k.neg_y), rb,
-                                                     false);
-    lo = pack_bf16x2(sa, sb);
-}
-
 // Code word -> B operand of tile M (four dwords of two bf16 each).  Element j
 // of the tile sits at bit 8M + 2(j/2) of the low (j even) or high (j odd)
 // half of the word; dword k keeps bits 2k..2k+1 of each half of the word
@@ -180,10 +121,6 @@ constexpr int kProdExp = 64;
 constexpr float kProdUnit = 0x1p-64f;      // 2^-kProdExp
 constexpr float kProdScale = 0x1p64f;      // 2^kProdExp
 static_assert(kCodeExp - kProdExp == 69, "code scale constants below");
-
-__device__ __forceinline__ f32x4_t mfma(bf16x8_t a, bf16x8_t b, f32x4_t c) {
-    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
-}
 
 template <int CTRL>
 __device__ __forceinline__ float dpp(float v) {
@@ -220,8 +157,6 @@ __device__ __forceinline__ float wave_sum(float v) {
     v = row_sum16(v);
     return (lane_f(v, 0) + lane_f(v, 16)) + (lane_f(v, 32) + lane_f(v, 48));
 }
-
-__device__ __forceinline__ float exp2_fast(float x) { return __builtin_amdgcn_exp2f(x); }
 
 // A per-lane LDS address, computed once and kept in a VGPR (PIN).  Left to
 // itself the compiler rebuilds such addresses (a multiply and an add of the

@@ -1,0 +1,1264 @@
+// Packed-KV attention for many query rows per kv head (gfx950 matrix cores).
+//
+// Causal or full attention of q_len query tokens per sequence over [packed
+// chunks ; residual window] (kivi_packed_attention) when q_len * (q_heads /
+// kv_heads) exceeds the 8 rows that one launch of the decode kernel
+// (kivi_attention_mfma.hpp) takes: the verification pass of drafted tokens, a
+// chunk of a long prompt.  The decode kernel multiplies the codes themselves,
+// which needs the query folded with each chunk's key scales, work per row and
+// chunk; with many rows the other order is cheaper: dequantise each 32 tokens
+// once and let every row use them.
+//
+// * Row r of a kv head is query token r / hg, head r % hg.  Rows are held in
+//   tiles of 16, and the context is walked in units of 32 tokens: the packed
+//   chunks' (a G = 64 chunk is two units), then the window's.
+// * K_hat and V_hat are expanded into MFMA A operands as bf16 pieces (hi + mid
+//   + lo for keys and for the fp32 window's values, hi + lo for packed
+//   values): a packed code word already holds one lane's codes of two tiles.
+// * Scores are formed transposed, S^T = K_hat Q^T, so a lane holds the scores
+//   of one query row (its l % 16) for 8 of the unit's tokens, and the output
+//   transposed too, O^T = V_hat^T P^T: a row's softmax state and rescale are
+//   per-lane scalars, and the probabilities go from the score registers into
+//   the second product's B operand without moving between lanes.
+// * Precision: products of pieces are accumulated in fp32.  A query whose
+//   values are all bf16 (a bf16 model's, widened) takes one piece and three
+//   products per key tile, any other query three pieces and six products
+//   (~2^-24 relative); packed values take three products of two pieces
+//   (~2^-17 per weight, averaged over the context), window values six of
+//   three.  The softmax is online in fp32, in the log2 domain; its maximum
+//   moves only when exceeded by more than 8 (weights <= 256).
+//
+// Two kernels (few_rows(): which rows take which):
+// * attn_rows_shared_kernel (many rows): eight waves with up to 32 rows each
+//   expand every unit together into LDS and read it from there.
+// * attn_rows_wave_kernel (few rows): each wave takes units of its own and
+//   expands them straight into its operand registers.
+//
+// Measured (MI355X, 32/8 heads, head_dim 128, bf16 ring and queries; the decode
+// kernel's launches before, this file's after): 512 query tokens over 8.1K
+// packed tokens, B=1: 256 launches, 4.84 ms -> 229 us; 5 tokens over 4K, B=8: 3
+// launches, 85.6 -> 52.7 us.
+#include <math.h>
+
+#include "kivi_attention.hpp"
+#include "kivi_common.hpp"
+#include "kivi_mfma.hpp"
+
+namespace kivi {
+namespace {
+
+constexpr int kUnit = 32;                   // tokens per step
+constexpr float kMoveMax = 8.0f;            // log2 units
+constexpr int kWindowWeight = 2;            // cost of a window unit in packed units
+constexpr int kKP = 3;                      // key pieces
+constexpr int kVPWin = 3, kVPChunk = 2;     // value pieces: window, packed chunks
+constexpr int kTile = kWave * 16;           // bytes of one operand tile
+
+constexpr uint32_t kNotFinite = 0x7f7f8000u;  // |x| from here on rounds to infinity as bf16
+
+typedef const __attribute__((address_space(1))) char* gptr;
+template <class T>
+__device__ __forceinline__ T gload(gptr base, uint32_t off) {
+    return *reinterpret_cast<const __attribute__((address_space(1))) T*>(base + off);
+}
+
+template <bool V>
+struct BoolC {
+    static constexpr bool value = V;
+};
+
+// max / sum over the four lanes that share a query row (l % 16)
+__device__ __forceinline__ float row4_max(float v) {
+    v = fmaxf(v, __shfl_xor(v, 16));
+    return fmaxf(v, __shfl_xor(v, 32));
+}
+__device__ __forceinline__ float row4_sum(float v) {
+    v += __shfl_xor(v, 16);
+    return v + __shfl_xor(v, 32);
+}
+
+__device__ __forceinline__ int64_t row_offset(const RowsLaunch& a, int b, int kvh, int r) {
+    return (((int64_t)b * a.q_len + r / a.hg) * a.Hq + (int64_t)kvh * a.hg + r % a.hg) * a.D;
+}
+
+// Piece operands of 8 fp32 values.
+template <int NP>
+__device__ __forceinline__ void split8(const float* x, u32x4_t* p, SplitConsts k) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        uint32_t h, m, lo;
+        if constexpr (NP == 3) {
+            split3_pair(x[2 * j], x[2 * j + 1], h, m, lo, k);
+            p[2][j] = lo;
+            p[1][j] = m;
+        } else if constexpr (NP == 2) {
+            split_pair(x[2 * j], x[2 * j + 1], h, m, k);
+            p[1][j] = m;
+        } else {
+            h = pack_bf16x2(x[2 * j], x[2 * j + 1]);
+        }
+        p[0][j] = h;
+    }
+}
+
+// acc[rt] += (sum of A pieces) * (sum of B pieces of rt): the products of
+// pieces i and j with i + j < max(NA, NB), smallest first (LAST 1: all but the
+// product of the first pieces).
+template <int NA, int NB, int RT, int LAST = 0, class B>
+__device__ __forceinline__ void mul_pieces(f32x4_t (&acc)[RT], const bf16x8_t* A, const B& b_of) {
+    constexpr int N = NA > NB ? NA : NB;
+#pragma unroll
+    for (int d = N - 1; d >= LAST; --d) {
+#pragma unroll
+        for (int j = 0; j < NB; ++j) {
+            if (d - j < 0 || d - j >= NA) continue;
+#pragma unroll
+            for (int rt = 0; rt < RT; ++rt) acc[rt] = mfma(A[d - j], b_of(rt, j), acc[rt]);
+        }
+    }
+}
+
+// A 16-bit ring element (in bits 15:0) widened: fp16 where half_mask is all
+// ones, bf16 where it is 0 (see load4_16).
+__device__ __forceinline__ float widen16(uint32_t h, uint32_t half_mask) {
+    const uint32_t f = __float_as_uint((float)__builtin_bit_cast(_Float16, (uint16_t)h));
+    return __uint_as_float((f & half_mask) | ((h << 16) & ~half_mask));
+}
+template <bool R16>
+__device__ __forceinline__ uint32_t ring_word(gptr p, uint32_t off) {
+    if constexpr (R16) return gload<uint16_t>(p, off);
+    else return gload<uint32_t>(p, off);
+}
+
+// Ring slot of window token t (clamped to the window: tokens past its end
+// repeat the last one and take no weight).
+__device__ __forceinline__ int window_slot(const RowsLaunch& a, int t) {
+    const int s = a.res_start + min(t, a.res_len - 1);
+    return s >= a.Rcap ? s - a.Rcap : s;
+}
+
+// Is an element (R16: one of the two) of this ring dword not finite as bf16?
+template <bool R16>
+__device__ __forceinline__ bool ring_bad(uint32_t d, uint32_t half_mask) {
+    if constexpr (!R16) return (d & 0x7fffffffu) >= kNotFinite;
+    const uint32_t lim = half_mask ? 0x7c00u : 0x7f80u;
+    return (d & 0x7fffu) >= lim || ((d >> 16) & 0x7fffu) >= lim;
+}
+
+// What the wave's query values of rows row0 + 16 rt + l % 16 need: kWide if
+// some are not bf16 (three pieces), kSlow if some are not finite as bf16.
+constexpr int kWide = 1, kSlow = 2;
+template <int D, int RT>
+__device__ __forceinline__ int query_kind(const RowsLaunch& a, int row0, int b, int kvh) {
+    const int lane = threadIdx.x % kWave;
+    uint32_t low = 0, top = 0;
+#pragma unroll
+    for (int rt = 0; rt < RT; ++rt) {
+        const int r = min(row0 + 16 * rt + lane % 16, a.rows - 1);
+        const float4* q = reinterpret_cast<const float4*>(a.q + row_offset(a, b, kvh, r) +
+                                                          8 * (lane / 16));
+#pragma unroll
+        for (int ks = 0; ks < D / 32; ++ks) {
+#pragma unroll
+            for (int j = 0; j < 2; ++j) {
+                const float4 x = q[8 * ks + j];
+                const uint32_t w[4] = {__float_as_uint(x.x), __float_as_uint(x.y),
+                                       __float_as_uint(x.z), __float_as_uint(x.w)};
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    low |= w[i];
+                    top = max(top, w[i] & 0x7fffffffu);
+                }
+            }
+        }
+    }
+    return (__builtin_amdgcn_ballot_w64((low & 0xffffu) != 0) != 0 ? kWide : 0) |
+           (__builtin_amdgcn_ballot_w64(top >= kNotFinite) != 0 ? kSlow : 0);
+}
+
+// A wave's RT tiles of 16 query rows: operands, softmax state and output.
+template <int D, int RT, int NQ>
+struct Rows {
+    static constexpr int KS = D / 32, NBV = D / 16;
+    bf16x8_t qf[RT][KS][NQ];
+    f32x4_t O[RT][NBV];
+    float m[RT], l[RT];
+    int vis[RT];                    // window tokens the lane's row sees
+    float qs;                       // |softmax scale * log2 e| (its sign is in the query)
+    SplitConsts spc;
+
+    // rows row0 .. (those past the end repeat the last; they are not stored)
+    __device__ __forceinline__ void init(const RowsLaunch& a, int row0, int b, int kvh) {
+        const int lane = threadIdx.x % kWave, col = lane % 16, gq = lane / 16;
+        spc = split_consts();
+        qs = fabsf(a.qscale);
+        const float sign = a.qscale < 0.f ? -1.f : 1.f;
+#pragma unroll
+        for (int rt = 0; rt < RT; ++rt) {
+            const int r = min(row0 + 16 * rt + col, a.rows - 1);
+            vis[rt] = min(a.vis0 + r / a.hg, a.res_len);
+            const float4* q = reinterpret_cast<const float4*>(a.q + row_offset(a, b, kvh, r) +
+                                                              8 * gq);
+#pragma unroll
+            for (int ks = 0; ks < KS; ++ks) {
+                const float4 x0 = q[8 * ks], x1 = q[8 * ks + 1];
+                const float x[8] = {x0.x * sign, x0.y * sign, x0.z * sign, x0.w * sign,
+                                    x1.x * sign, x1.y * sign, x1.z * sign, x1.w * sign};
+                u32x4_t p[3];
+                split8<NQ>(x, p, spc);
+#pragma unroll
+                for (int i = 0; i < NQ; ++i) qf[rt][ks][i] = __builtin_bit_cast(bf16x8_t, p[i]);
+            }
+            m[rt] = -INFINITY;
+            l[rt] = 0.f;
+#pragma unroll
+            for (int nb = 0; nb < NBV; ++nb) O[rt][nb] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+        }
+    }
+
+    // s[rt] += key tile (kKP pieces) x query at k-step ks
+    __device__ __forceinline__ void keys(f32x4_t (&s)[RT], const bf16x8_t* kf, int ks) {
+        mul_pieces<kKP, NQ, RT>(s, kf, [&](int rt, int j) { return qf[rt][ks][j]; });
+    }
+    // The same for the window's fp32 keys, the small products in a sum of their
+    // own: s then rounds once per k-step at its full size, as plain fp32 sums
+    // over that many channels at most do.
+    __device__ __forceinline__ void window_keys(f32x4_t (&s)[RT], f32x4_t (&small)[RT],
+                                                const bf16x8_t* kf, int ks) {
+        mul_pieces<kKP, NQ, RT, 1>(small, kf, [&](int rt, int j) { return qf[rt][ks][j]; });
+#pragma unroll
+        for (int rt = 0; rt < RT; ++rt) s[rt] = mfma(kf[0], qf[rt][ks][0], s[rt]);
+    }
+
+    // Online softmax of a unit's scores s[nb][rt] (unscaled), leaving the
+    // weights in p.  Score i of tile nb is the unit's token 4gq + 16nb + i.
+    // `hid`: bit t hides token t from every row; WIN: the unit is window
+    // tokens t0.., of which row tile rt sees those below vis.
+    template <bool WIN>
+    __device__ __forceinline__ void softmax(const f32x4_t (&s)[2][RT], uint32_t hid, int t0,
+                                            float (&p)[RT][8]) {
+        const int gq = (threadIdx.x % kWave) / 16;
+#pragma unroll
+        for (int rt = 0; rt < RT; ++rt) {
+            float x[8];
+#pragma unroll
+            for (int i = 0; i < 8; ++i) x[i] = s[i / 4][rt][i % 4];
+            uint32_t off = 0;                  // bit i: score i takes no weight
+            if (WIN || hid) {
+#pragma unroll
+                for (int i = 0; i < 8; ++i) {
+                    const int t = 4 * gq + 16 * (i / 4) + i % 4;
+                    off |= ((hid >> t) & 1u) << i;
+                    if (WIN) off |= t >= vis[rt] - t0 ? 1u << i : 0u;
+                }
+#pragma unroll
+                for (int i = 0; i < 8; ++i) x[i] = (off >> i) & 1u ? -INFINITY : x[i];
+            }
+            float top = x[0];
+#pragma unroll
+            for (int i = 1; i < 8; ++i) top = fmaxf(top, x[i]);
+            top *= qs;
+            if (__builtin_expect(__builtin_amdgcn_ballot_w64(top > m[rt] + kMoveMax) != 0, 0)) {
+                const float cm = row4_max(top);
+                if (cm > m[rt] + kMoveMax) {
+                    const float f = exp2_fast(m[rt] - cm);
+                    m[rt] = cm;
+                    l[rt] *= f;
+#pragma unroll
+                    for (int nb = 0; nb < NBV; ++nb) O[rt][nb] *= f;
+                }
+            }
+            float sum = 0.f;
+#pragma unroll
+            for (int i = 0; i < 8; ++i) p[rt][i] = exp2_fast(fmaf(x[i], qs, -m[rt]));
+            if (WIN || hid) {                  // (0 also while the maximum is -inf)
+#pragma unroll
+                for (int i = 0; i < 8; ++i) p[rt][i] = (off >> i) & 1u ? 0.f : p[rt][i];
+            }
+#pragma unroll
+            for (int i = 0; i < 8; ++i) sum += p[rt][i];
+            l[rt] += sum;
+        }
+    }
+    // The weights as VP operand pieces.
+    template <int VP, bool WIN>
+    __device__ __forceinline__ void weights(const f32x4_t (&s)[2][RT], uint32_t hid, int t0,
+                                            bf16x8_t (&pf)[RT][VP]) {
+        float p[RT][8];
+        softmax<WIN>(s, hid, t0, p);
+#pragma unroll
+        for (int rt = 0; rt < RT; ++rt) {
+            u32x4_t w[3];
+            split8<VP>(p[rt], w, spc);
+#pragma unroll
+            for (int i = 0; i < VP; ++i) pf[rt][i] = __builtin_bit_cast(bf16x8_t, w[i]);
+        }
+    }
+    // O[.][nb] += value tile nb (VP pieces) x weights.  A window unit's sum is
+    // formed apart and rounds O once.
+    template <int VP>
+    __device__ __forceinline__ void values(const bf16x8_t* vf, const bf16x8_t (&pf)[RT][VP], int nb) {
+        constexpr bool WIN = VP == kVPWin;
+        f32x4_t o[RT];
+#pragma unroll
+        for (int rt = 0; rt < RT; ++rt) o[rt] = WIN ? f32x4_t{0.f, 0.f, 0.f, 0.f} : O[rt][nb];
+        mul_pieces<VP, VP, RT>(o, vf, [&](int rt, int j) { return pf[rt][j]; });
+#pragma unroll
+        for (int rt = 0; rt < RT; ++rt) O[rt][nb] = WIN ? O[rt][nb] + o[rt] : o[rt];
+    }
+};
+
+// The unnormalised state of row r -> its partial, or the output when the
+// context has one split (a row that sees no position gives 0).
+struct RowDst {
+    float* p;
+    float f;
+};
+__device__ __forceinline__ RowDst row_dst(const RowsLaunch& a, int b, int kvh, int64_t bh, int r,
+                                          int split, float m, float l, bool first) {
+    if (a.n_splits == 1) return {a.out + row_offset(a, b, kvh, r), l > 0.f || l != l ? 1.f / l : 0.f};
+    const int64_t row = (bh * a.rows + r) * a.n_splits + split;
+    if (first) {
+        a.part_ml[row * 2] = m;
+        a.part_ml[row * 2 + 1] = l;
+    }
+    return {a.part_o + row * a.D, 1.f};
+}
+
+// A workgroup's range of units, and which of a unit's tokens are hidden.
+struct Range {
+    int n_cu;                      // packed units of the context
+    int begin, c_end, end;         // packed units [begin, c_end), then window units [.., end)
+    int kv_lo;
+    const uint32_t* hid_row;
+    int vis_most;                  // window tokens that some row of the workgroup sees
+
+    __device__ __forceinline__ Range(const RowsLaunch& a, int split, int b, int last_row) {
+        n_cu = a.n_chunks * (a.G / kUnit);
+        // splits are even in weight: a window unit counts kWindowWeight
+        const int nu = n_cu, all = a.n_units;
+        auto at = [nu, all](int x) {
+            return x <= nu ? x : min(nu + (x - nu + kWindowWeight - 1) / kWindowWeight, all);
+        };
+        begin = at(split * a.weight_per_split);
+        end = at((split + 1) * a.weight_per_split);
+        c_end = min(end, n_cu);
+        kv_lo = __builtin_amdgcn_readfirstlane(a.kv_start ? a.kv_start[b] : 0);
+        hid_row = a.hidden ? a.hidden + b * a.hidden_stride : nullptr;
+        vis_most = min(a.vis0 + min(last_row, a.rows - 1) / a.hg, a.res_len);
+    }
+    __device__ __forceinline__ uint32_t hidden(int u) const {       // wave-uniform
+        const int n = kv_lo - kUnit * u;
+        uint32_t h = n >= kUnit ? ~0u : n > 0 ? (1u << n) - 1u : 0u;
+        if (hid_row) h |= hid_row[u];
+        return h;
+    }
+    // one past the last window unit that some row sees
+    __device__ __forceinline__ int w_end() const {
+        return min(end, n_cu + (vis_most + kUnit - 1) / kUnit);
+    }
+};
+
+// Rows row0 .. row0+n-1 of a workgroup's range in plain fp32, a wave per row,
+// lanes over channels: for keys, values or queries that are not finite as
+// bf16.  The pieces of an infinity are no sum (inf - inf), and a score of -inf
+// has to give its token no weight.  Runs after the walk has found such an
+// element (nothing of the walk is live then) and writes over its result.
+template <int D, bool R16>
+__device__ __forceinline__ void slow_rows(const RowsLaunch& a, const Range& rg, int row0, int n,
+                                          int64_t bh, int b, int kvh, int split) {
+    constexpr int C = D / kWave, E = R16 ? 2 : 4;         // channels per lane: lane + 64 c
+    const int lane = threadIdx.x % kWave, waves = blockDim.x / kWave;
+    const gptr kr = (gptr)a.k_res + bh * a.Rcap * D * E, vr = (gptr)a.v_res + bh * a.Rcap * D * E;
+    const uint32_t half_mask = a.res_dt == kSrcF16 ? ~0u : 0u;
+    const int np = a.G * D / 1024, ng = D / a.Gv;
+    for (int r = row0 + (int)threadIdx.x / kWave; r < min(row0 + n, a.rows); r += waves) {
+        const int vis = min(a.vis0 + r / a.hg, a.res_len);
+        const gptr q = (gptr)(a.q + row_offset(a, b, kvh, r));
+        float o[C] = {}, m = -INFINITY, l = 0.f;
+#pragma unroll 1
+        for (int u = rg.begin; u < rg.end; ++u) {
+            const uint32_t hid = rg.hidden(u);
+            const bool win = u >= rg.n_cu;
+            const int t0 = kUnit * (u - rg.n_cu);
+            if (win && t0 >= rg.vis_most) break;
+            const int64_t cid = bh * a.Cmax + (win ? 0 : u * kUnit / a.G);
+            const int tc = win ? 0 : u * kUnit % a.G;     // the unit's first token in its chunk
+#pragma unroll 1
+            for (int t = 0; t < kUnit; ++t) {
+                if (win && t0 + t >= a.res_len) break;
+                float part = 0.f, v[C];
+#pragma unroll
+                for (int c = 0; c < C; ++c) {
+                    const int d = lane + kWave * c;
+                    float kx;
+                    if (win) {
+                        const uint32_t at = E * ((uint32_t)window_slot(a, t0 + t) * D + d);
+                        const uint32_t kw = ring_word<R16>(kr, at), vw = ring_word<R16>(vr, at);
+                        kx = R16 ? widen16(kw, half_mask) : __uint_as_float(kw);
+                        v[c] = R16 ? widen16(vw, half_mask) : __uint_as_float(vw);
+                    } else {
+                        const int tt = tc + t;            // see kLayoutMfma
+                        const int ktile = d / 32 * (a.G / 16) + tt / 16;
+                        const int vtile = tt / 32 * (D / 16) + d / 16;
+                        const gptr kc = (gptr)a.k_codes + cid * (a.G * D / 4);
+                        const gptr vc = (gptr)a.v_codes + cid * (a.G * D / 4);
+                        const uint32_t kw = gload<uint32_t>(
+                            kc, 4 * ((16 * (d % 32 / 8) + tt % 16) * np + ktile / 2));
+                        const uint32_t vw = gload<uint32_t>(
+                            vc, 4 * ((16 * (tt % 32 / 8) + d % 16) * np + vtile / 2));
+                        const int64_t km = cid * D + d, vm = (cid * ng + d / a.Gv) * a.G + tt;
+                        kx = fmaf((float)((kw >> mfma_code_bit(ktile % 2, d % 8)) & 3u),
+                                  a.k_scale[km], a.k_zero[km]);
+                        v[c] = fmaf((float)((vw >> mfma_code_bit(vtile % 2, tt % 8)) & 3u),
+                                    a.v_scale[vm], a.v_zero[vm]);
+                    }
+                    part = fmaf(gload<float>(q, 4 * d), kx, part);
+                }
+#pragma unroll
+                for (int x = 1; x < kWave; x *= 2) part += __shfl_xor(part, x);
+                const bool off = ((hid >> t) & 1u) || (win && t0 + t >= vis);
+                const float s = off ? -INFINITY : part * a.qscale;
+                if (s > m + kMoveMax) {
+                    const float f = exp2_fast(m - s);
+                    m = s;
+                    l *= f;
+#pragma unroll
+                    for (int c = 0; c < C; ++c) o[c] *= f;
+                }
+                const float w = off ? 0.f : exp2_fast(s - m);
+                l += w;
+#pragma unroll
+                for (int c = 0; c < C; ++c) o[c] = fmaf(w, v[c], o[c]);
+            }
+        }
+        const RowDst dst = row_dst(a, b, kvh, bh, r, split, m, l, lane == 0);
+#pragma unroll
+        for (int c = 0; c < C; ++c) dst.p[lane + kWave * c] = o[c] * dst.f;
+    }
+}
+
+// ---------------------------------------------------------------------------
+// Many rows: units expanded into LDS by the whole workgroup.
+//
+// What bounds it: a wave's step is 96 matrix products (1536 cycles) of two row
+// tiles, ~270 vector instructions and 40 KB of LDS reads; two waves per SIMD
+// take ~6100 cycles per step, the products 3100 of them, the LDS reads 2600
+// (each 1 KB operand feeds two row tiles).  Also measured for 512 query
+// tokens (215 us kernel time): 4 waves with 128 rows and two workgroups per
+// CU 264 us; 4 waves with four row tiles each (half the LDS reads, one wave
+// per SIMD, 66 registers spilled) 295 us; a raised priority for half of the
+// waves 224 us.
+// ---------------------------------------------------------------------------
+template <int D>
+struct SharedShape {
+    static constexpr int KS = D / 32, NBV = D / 16;
+    static constexpr int WAVES = D <= 128 ? 8 : 4, BLOCK = WAVES * kWave;
+    // code words of a unit that each wave expands (a word: one lane-word of
+    // the key or value operands, two tiles); at head_dim 64 the last four
+    // waves have none
+    static constexpr int WORDS = 2 * KS / WAVES > 0 ? 2 * KS / WAVES : 1;
+    static constexpr int RT = D <= 128 ? 2 : 1;   // most row tiles per wave
+    // value tiles are spaced for three pieces where LDS allows (packed values
+    // then write a third piece nobody reads, instead of branching)
+    static constexpr int VSTR = WORDS > 1 ? 2 : 3;
+    static constexpr int K_BYTES = KS * 2 * kKP * kTile;
+    static constexpr int BUF = K_BYTES + NBV * VSTR * kTile;
+    static constexpr int LDS = 2 * BUF;
+    static_assert(K_BYTES + NBV * kVPWin * kTile <= LDS, "a window unit fits");
+};
+
+// Word i of a wave: key word or value word w.  At head_dim 256 a wave has two
+// of each, keys first; below, one word.
+struct Word {
+    bool key;
+    int w;
+};
+// (at head_dim 64 the last four waves have none)
+template <int D>
+__device__ __forceinline__ bool has_word(int wave) {
+    return 2 * (D / 32) >= SharedShape<D>::WAVES || wave < 2 * (D / 32);
+}
+template <int D>
+__device__ __forceinline__ Word word_of(int i, int wave) {
+    constexpr int KS = D / 32;
+    constexpr int HALF = SharedShape<D>::WORDS / 2;
+    if constexpr (HALF > 0) return {i < HALF, wave + SharedShape<D>::WAVES * (i % HALF)};
+    return {wave < KS, wave % KS};
+}
+
+// Where a thread stores its words' pieces: byte offset in a buffer of (tile 2w,
+// piece 0)'s first half, distance of the second half, of the tiles 2w + 1, of
+// the pieces (kTile).  Key operands are lane-major.  Value operands: this
+// lane's 8 tokens 8(l/16)..+7 of a channel go to the operand slots (g, j) of
+// tokens 4g + j%4 + 16(j/4), the order the scores lie in.
+template <int D>
+struct Dst {
+    uint32_t at[SharedShape<D>::WORDS], half[SharedShape<D>::WORDS], tile[SharedShape<D>::WORDS];
+    __device__ __forceinline__ Dst(int wave, int lane, int vstr) {
+        const int gq = lane / 16, col = lane % 16;
+#pragma unroll
+        for (int i = 0; i < SharedShape<D>::WORDS; ++i) {
+            const Word x = word_of<D>(i, wave);
+            at[i] = x.key ? (2 * x.w * kKP) * kTile + lane * 16
+                          : SharedShape<D>::K_BYTES + (2 * x.w * vstr) * kTile +
+                                ((2 * (gq % 2)) * 16 + col) * 16 + 8 * (gq / 2);
+            half[i] = x.key ? 8 : 256;
+            tile[i] = (x.key ? kKP : vstr) * kTile;
+        }
+    }
+};
+
+// Stores the pieces of one tile's 8 values.
+template <int NP>
+__device__ __forceinline__ void put_tile(unsigned char* at, uint32_t half, const float* x,
+                                         SplitConsts k) {
+    u32x4_t p[3];
+    split8<NP>(x, p, k);
+#pragma unroll
+    for (int i = 0; i < NP; ++i) {
+        *reinterpret_cast<uint2*>(at + i * kTile) = make_uint2(p[i][0], p[i][1]);
+        *reinterpret_cast<uint2*>(at + i * kTile + half) = make_uint2(p[i][2], p[i][3]);
+    }
+}
+
+// A thread's words of a packed unit with the 8 scales and zeros of their 8
+// channels (keys) or 8 tokens (values), and where they come from.
+template <int D>
+struct PackedUnit {
+    static constexpr int N = SharedShape<D>::WORDS;
+    uint32_t word[N];
+    kivi_f4v sc[N][2], zr[N][2];
+    // at chunk 0 of the (batch, kv head): wave-uniform bases (global pointers:
+    // a load through a selected generic pointer would count as an LDS access
+    // too, and every LDS wait would wait for it), bytes per chunk and per
+    // second unit of a G = 64 chunk, and this lane's bytes
+    gptr code[N], scale[N], zero[N];
+    uint32_t code_step[N], code_half[N], meta_step[N], meta_half[N], code_off[N], meta_off[N];
+
+    __device__ __forceinline__ void init(const RowsLaunch& a, int64_t bh, int wave, int lane) {
+        const int two = a.G == 64 ? 2 : 1;    // units per chunk
+        const int64_t c0 = bh * a.Cmax;
+#pragma unroll
+        for (int i = 0; i < N; ++i) {
+            const Word x = word_of<D>(i, wave);
+            code_step[i] = a.G * D / 4;
+            code_half[i] = x.key ? 4 : D / 8;
+            meta_step[i] = 4 * (x.key ? D : D / a.Gv * a.G);
+            meta_half[i] = x.key ? 0 : 4 * kUnit;
+            code[i] = (gptr)(x.key ? a.k_codes : a.v_codes) + c0 * code_step[i];
+            scale[i] = (gptr)(x.key ? a.k_scale : a.v_scale) + c0 * meta_step[i];
+            zero[i] = (gptr)(x.key ? a.k_zero : a.v_zero) + c0 * meta_step[i];
+            code_off[i] = 4u * (lane * (two * (D / 32)) + (x.key ? x.w * two : x.w));
+            meta_off[i] = 4u * ((x.key ? 32 * x.w : 32 * x.w / a.Gv * a.G) + 8 * (lane / 16));
+        }
+    }
+    __device__ __forceinline__ void load(int two, int u) {
+        const uint32_t chunk = two ? u >> 1 : u, half = two ? u & 1 : 0;
+#pragma unroll
+        for (int i = 0; i < N; ++i) {
+            const gptr c = code[i] + (chunk * code_step[i] + half * code_half[i]);
+            const uint32_t m = chunk * meta_step[i] + half * meta_half[i];
+            word[i] = gload<uint32_t>(c, code_off[i]);
+            sc[i][0] = gload<kivi_f4v>(scale[i] + m, meta_off[i]);
+            sc[i][1] = gload<kivi_f4v>(scale[i] + m, meta_off[i] + 16);
+            zr[i][0] = gload<kivi_f4v>(zero[i] + m, meta_off[i]);
+            zr[i][1] = gload<kivi_f4v>(zero[i] + m, meta_off[i] + 16);
+        }
+    }
+    // Expands tile m of every word into buffer `buf`.
+    template <int M>
+    __device__ __forceinline__ void expand(unsigned char* buf, const Dst<D>& d, int wave,
+                                           SplitConsts k) const {
+#pragma unroll
+        for (int i = 0; i < N; ++i) {
+            const Word w = word_of<D>(i, wave);
+            const float s[8] = {sc[i][0].x, sc[i][0].y, sc[i][0].z, sc[i][0].w,
+                                sc[i][1].x, sc[i][1].y, sc[i][1].z, sc[i][1].w};
+            const float z[8] = {zr[i][0].x, zr[i][0].y, zr[i][0].z, zr[i][0].w,
+                                zr[i][1].x, zr[i][1].y, zr[i][1].z, zr[i][1].w};
+            float x[8];
+#pragma unroll
+            for (int c = 0; c < 4; ++c) {     // elements 2c and 2c + 1: bytes M and 2 + M
+                const uint32_t y = (word[i] >> (2 * c)) & 0x03030303u;
+                x[2 * c] = fmaf((float)((y >> (8 * M)) & 0xffu), s[2 * c], z[2 * c]);
+                x[2 * c + 1] = fmaf((float)((y >> (16 + 8 * M)) & 0xffu), s[2 * c + 1],
+                                    z[2 * c + 1]);
+            }
+            unsigned char* at = buf + d.at[i] + M * d.tile[i];
+            if constexpr (N > 1) {            // (the kind of word is known)
+                if (w.key) put_tile<kKP>(at, d.half[i], x, k);
+                else put_tile<kVPChunk>(at, d.half[i], x, k);
+            } else if (has_word<D>(wave)) {
+                put_tile<kKP>(at, d.half[i], x, k);
+            }
+        }
+    }
+};
+
+// A thread's words of a window unit, as the ring holds them (widened when
+// they are expanded, so that nothing waits for the loads before).
+template <int D, bool R16>
+struct WindowUnit {
+    static constexpr int N = SharedShape<D>::WORDS, E = R16 ? 2 : 4;
+    uint32_t raw[N][16];
+
+    __device__ __forceinline__ void load(const RowsLaunch& a, int64_t bh, int t0, int wave,
+                                         int lane) {
+        const int gq = lane / 16, col = lane % 16;
+        const int64_t base = bh * a.Rcap * D * E;
+        const gptr kr = (gptr)a.k_res + base, vr = (gptr)a.v_res + base;
+        if (!has_word<D>(wave)) return;
+#pragma unroll
+        for (int i = 0; i < N; ++i) {
+            const Word w = word_of<D>(i, wave);
+            if (w.key) {
+#pragma unroll
+                for (int m = 0; m < 2; ++m) {
+                    const uint32_t o = E * ((uint32_t)window_slot(a, t0 + 16 * m + col) * D +
+                                            32 * w.w + 8 * gq);
+#pragma unroll
+                    for (int q = 0; q < E / 2; ++q) {
+                        const u32x4_t x = gload<u32x4_t>(kr, o + 16 * q);
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) raw[i][8 * m + 4 * q + e] = x[e];
+                    }
+                }
+            } else {
+#pragma unroll
+                for (int j = 0; j < 8; ++j) {
+                    const uint32_t o = E * ((uint32_t)window_slot(a, t0 + 8 * gq + j) * D +
+                                            32 * w.w + col);
+#pragma unroll
+                    for (int m = 0; m < 2; ++m) raw[i][8 * m + j] = ring_word<R16>(vr, o + 16 * E * m);
+                }
+            }
+        }
+    }
+    // (returns whether some element is not finite as bf16)
+    __device__ __forceinline__ bool expand(unsigned char* buf, const Dst<D>& d, int wave,
+                                           uint32_t half_mask, SplitConsts k) const {
+        bool bad = false;
+        if (!has_word<D>(wave)) return bad;
+#pragma unroll
+        for (int i = 0; i < N; ++i) {
+            const bool key = word_of<D>(i, wave).key;
+#pragma unroll
+            for (int j = 0; j < 16; ++j)
+                if (!R16 || !key || j % 8 < 4) bad = bad || ring_bad<R16>(raw[i][j], half_mask);
+#pragma unroll
+            for (int m = 0; m < 2; ++m) {
+                float x[8];
+#pragma unroll
+                for (int j = 0; j < 8; ++j) {
+                    if constexpr (!R16) x[j] = __uint_as_float(raw[i][8 * m + j]);
+                    else if (key) x[j] = widen16((raw[i][8 * m + j / 2] >> (16 * (j % 2))) & 0xffffu, half_mask);
+                    else x[j] = widen16(raw[i][8 * m + j], half_mask);
+                }
+                put_tile<3>(buf + d.at[i] + m * d.tile[i], d.half[i], x, k);
+            }
+        }
+        return bad;
+    }
+};
+
+// Scheduling order of a product phase of TILES operand tiles, READS LDS reads
+// and MFMAS products each: the reads run two tiles ahead of the products.  Left
+// to itself the compiler reads a tile right before its products and waits
+// out the LDS latency each time.
+template <int TILES, int READS, int MFMAS>
+__device__ __forceinline__ void order_products() {
+    constexpr int kMfma = 0x8, kDsRead = 0x100;
+    constexpr int AHEAD = TILES < 2 ? TILES : 2;
+    __builtin_amdgcn_sched_group_barrier(kDsRead, AHEAD * READS, 0);
+#pragma unroll
+    for (int t = 0; t < TILES; ++t) {
+        __builtin_amdgcn_sched_group_barrier(kMfma, MFMAS, 0);
+        if (t + AHEAD < TILES) __builtin_amdgcn_sched_group_barrier(kDsRead, READS, 0);
+    }
+}
+
+// Returns whether this thread met a window element that is not finite as bf16.
+template <int D, int RT, int NQ, bool R16>
+__device__ bool walk_shared(const RowsLaunch& a, unsigned char* smem, const Range& rg, int row0,
+                            int64_t bh, int b, int kvh, int split) {
+    using S = SharedShape<D>;
+    const int lane = threadIdx.x % kWave;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+    const bool active = row0 < a.rows;         // wave-uniform
+    Rows<D, RT, NQ> rows;
+    rows.init(a, row0, b, kvh);
+
+    // One unit from LDS buffer `buf`; after_k and after_v run behind the reads
+    // of the key and of the value tiles: the expansion of the next unit, whose
+    // vector work then sits among this unit's matrix products.
+    auto use_unit = [&](const unsigned char* buf, uint32_t hid, int t0, auto win_c, int vstr,
+                        auto&& after_k, auto&& after_v) {
+        constexpr bool WIN = decltype(win_c)::value;
+        constexpr int VP = WIN ? kVPWin : kVPChunk;
+        f32x4_t s[2][RT], small[2][RT];
+#pragma unroll
+        for (int rt = 0; rt < RT; ++rt)
+            s[0][rt] = s[1][rt] = small[0][rt] = small[1][rt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int ks = 0; ks < S::KS; ++ks) {
+#pragma unroll
+            for (int nb = 0; nb < 2; ++nb) {
+                bf16x8_t kf[kKP];
+#pragma unroll
+                for (int p = 0; p < kKP; ++p)
+                    kf[p] = *reinterpret_cast<const bf16x8_t*>(
+                        buf + ((2 * ks + nb) * kKP + p) * kTile + lane * 16);
+                if constexpr (WIN) rows.window_keys(s[nb], small[nb], kf, ks);
+                else rows.keys(s[nb], kf, ks);
+            }
+        }
+        if constexpr (WIN) {
+#pragma unroll
+            for (int rt = 0; rt < RT; ++rt) {
+                s[0][rt] += small[0][rt];
+                s[1][rt] += small[1][rt];
+            }
+        }
+        after_k();
+        order_products<2 * S::KS, kKP, (NQ == 1 ? 3 : 6) * RT>();
+        bf16x8_t pf[RT][VP];
+        rows.template weights<VP, WIN>(s, hid, t0, pf);
+#pragma unroll
+        for (int nb = 0; nb < S::NBV; ++nb) {
+            bf16x8_t vf[VP];
+#pragma unroll
+            for (int p = 0; p < VP; ++p)
+                vf[p] = *reinterpret_cast<const bf16x8_t*>(buf + S::K_BYTES +
+                                                           (nb * vstr + p) * kTile + lane * 16);
+            rows.template values<VP>(vf, pf, nb);
+        }
+        after_v();
+        order_products<S::NBV, VP, VP * (VP + 1) / 2 * RT>();
+    };
+
+    bool bad = false;
+    if (rg.begin < rg.c_end) {
+        PackedUnit<D> unit;
+        const Dst<D> dst(wave, lane, S::VSTR);
+        const int two = a.G == 64;
+        unit.init(a, bh, wave, lane);
+        unit.load(two, rg.begin);
+        lds_barrier();                         // an earlier walk has read its last unit
+        unit.template expand<0>(smem, dst, wave, rows.spc);
+        unit.template expand<1>(smem, dst, wave, rows.spc);
+        unit.load(two, min(rg.begin + 1, rg.c_end - 1));
+        for (int u = rg.begin; u < rg.c_end; ++u) {
+            const uint32_t hid = rg.hidden(u);
+            unsigned char* cur = smem + ((u - rg.begin) & 1) * S::BUF;
+            unsigned char* nxt = smem + ((u - rg.begin + 1) & 1) * S::BUF;
+            lds_barrier();                     // cur is written, nxt has been read
+            auto first = [&] { unit.template expand<0>(nxt, dst, wave, rows.spc); };
+            auto second = [&] {
+                unit.template expand<1>(nxt, dst, wave, rows.spc);
+                unit.load(two, min(u + 2, rg.c_end - 1));
+            };
+            if (active && hid != ~0u) {
+                use_unit(cur, hid, 0, BoolC<false>{}, S::VSTR, first, second);
+            } else {
+                first();
+                second();
+            }
+        }
+    }
+    const int w_begin = max(rg.begin, rg.n_cu), w_end = rg.w_end();
+    if (w_begin < w_end) {
+        WindowUnit<D, R16> unit;
+        const uint32_t half_mask = a.res_dt == kSrcF16 ? ~0u : 0u;
+        const Dst<D> dst(wave, lane, kVPWin);
+        unit.load(a, bh, kUnit * (w_begin - rg.n_cu), wave, lane);
+        for (int u = w_begin; u < w_end; ++u) {
+            const int t0 = kUnit * (u - rg.n_cu);
+            const uint32_t hid = rg.hidden(u);
+            lds_barrier();                     // the previous unit has been read
+            bad |= unit.expand(smem, dst, wave, half_mask, rows.spc);
+            unit.load(a, bh, t0 + kUnit, wave, lane);
+            lds_barrier();
+            if (active) use_unit(smem, hid, t0, BoolC<true>{}, kVPWin, [] {}, [] {});
+        }
+    }
+
+    if (!active) return bad;
+    const int gq = lane / 16;
+#pragma unroll
+    for (int rt = 0; rt < RT; ++rt) {
+        const float l = row4_sum(rows.l[rt]);
+        const int r = row0 + 16 * rt + lane % 16;
+        if (r >= a.rows) continue;
+        const RowDst d = row_dst(a, b, kvh, bh, r, split, rows.m[rt], l, gq == 0);
+#pragma unroll
+        for (int nb = 0; nb < S::NBV; ++nb) {
+            const f32x4_t o = rows.O[rt][nb];
+            *reinterpret_cast<float4*>(d.p + 16 * nb + 4 * gq) =
+                make_float4(o[0] * d.f, o[1] * d.f, o[2] * d.f, o[3] * d.f);
+        }
+    }
+    return bad;
+}
+
+template <int D, int RT, bool R16>
+__global__ __launch_bounds__(SharedShape<D>::BLOCK) __attribute__((amdgpu_waves_per_eu(D <= 128 ? 2 : 1)))
+void attn_rows_shared_kernel(RowsLaunch a) {
+    extern __shared__ __align__(16) unsigned char smem[];
+    const int split = blockIdx.x % a.n_splits, rblock = blockIdx.x / a.n_splits;
+    const int kvh = blockIdx.y, b = blockIdx.z;
+    const int64_t bh = (int64_t)b * a.Hkv + kvh;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+    const int block0 = rblock * a.block_rows, row0 = block0 + wave * 16 * RT;
+    const Range rg(a, split, b, block0 + a.block_rows - 1);
+    // OR of a value of each wave (before or after the units take the space)
+    int* word = reinterpret_cast<int*>(smem);
+    auto any_wave = [&](int mine) {
+        lds_barrier();
+        if (threadIdx.x % kWave == 0) word[wave] = mine;
+        lds_barrier();
+        int x = 0;
+#pragma unroll
+        for (int w = 0; w < SharedShape<D>::WAVES; ++w) x |= word[w];
+        lds_barrier();
+        return __builtin_amdgcn_readfirstlane(x);
+    };
+    // What the workgroup's queries need (uniform: both walks hold workgroup
+    // barriers).
+    const int kind = any_wave(query_kind<D, RT>(a, row0, b, kvh));
+    bool bad = kind & kSlow;
+    if (!(kind & kWide)) {
+        bad |= walk_shared<D, RT, 1, R16>(a, smem, rg, row0, bh, b, kvh, split);
+    } else {
+        // three query pieces: one row tile at a time (the pieces of two do not
+        // fit the registers)
+        for (int rt = 0; rt < RT; ++rt)
+            bad |= walk_shared<D, 1, 3, R16>(a, smem, rg, row0 + 16 * rt, bh, b, kvh, split);
+    }
+    if (__builtin_expect(any_wave(__builtin_amdgcn_ballot_w64(bad) != 0), 0)) {
+        __syncthreads();                       // the walk's results are written
+        slow_rows<D, R16>(a, rg, block0, a.block_rows, bh, b, kvh, split);
+    }
+}
+
+// ---------------------------------------------------------------------------
+// Few rows: each wave expands units of its own into its registers, with no
+// barrier and no LDS traffic but the scales.
+//
+// What bounds it: the expansion's vector work, ~800 instructions per unit
+// (4-5.5 cycles each) against 1536 cycles of matrix products for two row tiles;
+// a second wave per SIMD gains nothing (38 us against 37 us at B=8, 5 query
+// tokens over 4K), so a workgroup per CU is the plan's target.
+// ---------------------------------------------------------------------------
+constexpr int kWaveWaves = 4, kWaveBlock = kWaveWaves * kWave;
+
+template <int D>
+struct WaveShape {
+    static constexpr int KS = D / 32, NBV = D / 16;
+    static constexpr int RT = D <= 128 ? 2 : 1;
+    // a wave's staged scales and zeros: keys [2][D], values [2][D/Gv][32] (at
+    // most [2][D])
+    static constexpr int META = 4 * D * 4;
+    static constexpr int NMETA = (D + kWave - 1) / kWave;       // float4s per lane
+    // one wave's state of 16 RT rows: o [16 RT][D], m and l
+    static constexpr int STATE = 16 * RT * (D + 2) * 4;
+    static constexpr int LDS = kWaveWaves * (STATE > META ? STATE : META);
+};
+
+// Orders a wave's LDS writes before its own later reads (a wave's LDS
+// operations execute in order, so no wait is needed).
+__device__ __forceinline__ void wave_fence() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// A lane's loads of one packed unit.  A key word is used as it lies (two
+// tiles).  A lane's value operand holds tokens 4gq..+3 and 16+4gq..+3, half
+// of what the words of lane groups gq/2 (va) and 2 + gq/2 (vb) hold.
+template <int D>
+struct WaveUnit {
+    static constexpr int KS = D / 32;
+    uint32_t k[KS], va[KS], vb[KS];
+    kivi_f4v meta[WaveShape<D>::NMETA];
+
+    __device__ __forceinline__ void load_codes(const RowsLaunch& a, int64_t bh, int u, int lane) {
+        const int two = a.G == 64 ? 2 : 1;
+        const int chunk = two == 2 ? u >> 1 : u, half = two == 2 ? u & 1 : 0;
+        const int64_t c0 = (bh * a.Cmax + chunk) * (a.G * D / 4);
+        const uint32_t src = 16 * (lane / 32) + lane % 16;
+        const uint32_t np = two * KS;
+        const gptr kc = (gptr)a.k_codes + c0 + 4 * half, vc = (gptr)a.v_codes + c0 + 4 * half * KS;
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks) {
+            k[ks] = gload<uint32_t>(kc, 4u * (lane * np + ks * two));
+            va[ks] = gload<uint32_t>(vc, 4u * (src * np + ks));
+            vb[ks] = gload<uint32_t>(vc, 4u * ((src + 32) * np + ks));
+        }
+    }
+    // float4 e of [ks | kz | vs of the unit | vz of the unit]
+    __device__ __forceinline__ void load_meta(const RowsLaunch& a, int64_t bh, int u, int lane,
+                                              int ng) {
+        const int two = a.G == 64 ? 2 : 1;
+        const int chunk = two == 2 ? u >> 1 : u, half = two == 2 ? u & 1 : 0;
+        const int64_t cid = bh * a.Cmax + chunk;
+        const int kq = D / 4, vq = ng * 8;
+#pragma unroll
+        for (int i = 0; i < WaveShape<D>::NMETA; ++i) {
+            const int e = min(lane + kWave * i, 2 * kq + 2 * vq - 1);
+            gptr p;
+            if (e < 2 * kq) {
+                p = (gptr)(e < kq ? a.k_scale + 4 * e : a.k_zero + 4 * (e - kq)) + 4 * cid * D;
+            } else {
+                const int f = e - 2 * kq, g = f < vq ? f : f - vq;
+                p = (gptr)(f < vq ? a.v_scale : a.v_zero) +
+                    4 * ((cid * ng + g / 8) * a.G + kUnit * half + 4 * (g % 8));
+            }
+            meta[i] = gload<kivi_f4v>(p, 0);
+        }
+    }
+    __device__ __forceinline__ void stage_meta(float* mt, int lane, int ng) const {
+        const int n = D / 2 + 16 * ng;
+#pragma unroll
+        for (int i = 0; i < WaveShape<D>::NMETA; ++i) {
+            // (a lane past the end holds the last float4 and writes it again)
+            const int e = min(lane + kWave * i, n - 1);
+            reinterpret_cast<kivi_f4v*>(mt)[e] = meta[i];
+        }
+    }
+};
+
+// N elements, from 0 on, of both tiles of a code word.
+template <int N>
+__device__ __forceinline__ void expand_word(uint32_t word, const float* s, const float* z, float* x0,
+                                            float* x1) {
+#pragma unroll
+    for (int c = 0; c < N / 2; ++c) {
+        // bytes: tile 0 element 2c, tile 1 element 2c, tile 0 element 2c+1, tile 1 ...
+        const uint32_t y = (word >> (2 * c)) & 0x03030303u;
+        x0[2 * c] = fmaf((float)(y & 0xffu), s[2 * c], z[2 * c]);
+        x1[2 * c] = fmaf((float)((y >> 8) & 0xffu), s[2 * c], z[2 * c]);
+        x0[2 * c + 1] = fmaf((float)((y >> 16) & 0xffu), s[2 * c + 1], z[2 * c + 1]);
+        x1[2 * c + 1] = fmaf((float)(y >> 24), s[2 * c + 1], z[2 * c + 1]);
+    }
+}
+
+__device__ __forceinline__ void read4(const float* p, float* x) {
+    const float4 v = *reinterpret_cast<const float4*>(p);
+    x[0] = v.x; x[1] = v.y; x[2] = v.z; x[3] = v.w;
+}
+
+template <int NP>
+__device__ __forceinline__ void operands8(const float* x, bf16x8_t* f, SplitConsts k) {
+    u32x4_t p[3];
+    split8<NP>(x, p, k);
+#pragma unroll
+    for (int i = 0; i < NP; ++i) f[i] = __builtin_bit_cast(bf16x8_t, p[i]);
+}
+
+template <int D, int RT, int NQ, bool R16>
+__device__ bool walk_wave(const RowsLaunch& a, unsigned char* smem, const Range& rg, int row0,
+                          int64_t bh, int b, int kvh, int split) {
+    constexpr int KS = D / 32;
+    const int lane = threadIdx.x % kWave, gq = lane / 16, col = lane % 16;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+    Rows<D, RT, NQ> rows;
+    rows.init(a, row0, b, kvh);
+    bool bad = false;
+    const int ng = D / a.Gv;
+    float* mt = reinterpret_cast<float*>(smem + wave * WaveShape<D>::META);
+
+    // packed units begin + wave, + 4, ...
+    if (rg.begin + wave < rg.c_end) {
+        WaveUnit<D> unit;
+        unit.load_meta(a, bh, rg.begin + wave, lane, ng);
+        unit.load_codes(a, bh, rg.begin + wave, lane);
+        const int vshift = 4 * (gq % 2);       // the lane's half of its value words
+        for (int u = rg.begin + wave; u < rg.c_end; u += kWaveWaves) {
+            const uint32_t hid = rg.hidden(u);
+            const int next = min(u + kWaveWaves, rg.c_end - 1);
+            wave_fence();                      // the previous unit's reads come first
+            unit.stage_meta(mt, lane, ng);
+            wave_fence();
+            unit.load_meta(a, bh, next, lane, ng);
+            f32x4_t s[2][RT];
+#pragma unroll
+            for (int rt = 0; rt < RT; ++rt) s[0][rt] = s[1][rt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int ks = 0; ks < KS; ++ks) {
+                float sc[8], zr[8], x[2][8];
+                bf16x8_t kf[kKP];
+                const float* p = mt + 32 * ks + 8 * gq;
+                read4(p, sc);
+                read4(p + 4, sc + 4);
+                read4(p + D, zr);
+                read4(p + D + 4, zr + 4);
+                expand_word<8>(unit.k[ks], sc, zr, x[0], x[1]);
+#pragma unroll
+                for (int nb = 0; nb < 2; ++nb) {
+                    operands8<kKP>(x[nb], kf, rows.spc);
+                    rows.keys(s[nb], kf, ks);
+                }
+            }
+            bf16x8_t pf[RT][kVPChunk];
+            rows.template weights<kVPChunk, false>(s, hid, 0, pf);
+#pragma unroll
+            for (int w = 0; w < KS; ++w) {
+                float sc[8], zr[8], x[2][8];
+                bf16x8_t vf[kVPChunk];
+                const float* p = mt + 2 * D + kUnit * (32 * w / a.Gv) + 4 * gq;
+                read4(p, sc);
+                read4(p + 16, sc + 4);
+                read4(p + kUnit * ng, zr);
+                read4(p + kUnit * ng + 16, zr + 4);
+                expand_word<4>(unit.va[w] >> vshift, sc, zr, x[0], x[1]);
+                expand_word<4>(unit.vb[w] >> vshift, sc + 4, zr + 4, x[0] + 4, x[1] + 4);
+#pragma unroll
+                for (int m = 0; m < 2; ++m) {
+                    operands8<kVPChunk>(x[m], vf, rows.spc);
+                    rows.template values<kVPChunk>(vf, pf, 2 * w + m);
+                }
+            }
+            unit.load_codes(a, bh, next, lane);
+        }
+    }
+    // window units, dealt in the same turn
+    constexpr int E = R16 ? 2 : 4;
+    const gptr kr = (gptr)a.k_res + bh * a.Rcap * D * E, vr = (gptr)a.v_res + bh * a.Rcap * D * E;
+    const uint32_t half_mask = a.res_dt == kSrcF16 ? ~0u : 0u;
+    const int w_begin = max(rg.begin, rg.n_cu), w_end = rg.w_end();
+    for (int u = w_begin + (wave + rg.begin + 4 * kWaveWaves - w_begin % kWaveWaves) % kWaveWaves;
+         u < w_end; u += kWaveWaves) {
+        const int t0 = kUnit * (u - rg.n_cu);
+        const uint32_t hid = rg.hidden(u);
+        u32x4_t kq[2][KS][E / 2];
+#pragma unroll
+        for (int nb = 0; nb < 2; ++nb) {
+            const uint32_t o = E * ((uint32_t)window_slot(a, t0 + 16 * nb + col) * D + 8 * gq);
+#pragma unroll
+            for (int ks = 0; ks < KS; ++ks) {
+#pragma unroll
+                for (int q = 0; q < E / 2; ++q)
+                    kq[nb][ks][q] = gload<u32x4_t>(kr, o + 32 * E * ks + 16 * q);
+            }
+        }
+        uint32_t vo[8];
+#pragma unroll
+        for (int j = 0; j < 8; ++j)
+            vo[j] = E * ((uint32_t)window_slot(a, t0 + 4 * gq + 16 * (j / 4) + j % 4) * D + col);
+        f32x4_t s[2][RT], small[2][RT];
+#pragma unroll
+        for (int rt = 0; rt < RT; ++rt)
+            s[0][rt] = s[1][rt] = small[0][rt] = small[1][rt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks) {
+#pragma unroll
+            for (int nb = 0; nb < 2; ++nb) {
+                float x[8];
+                bf16x8_t kf[kKP];
+#pragma unroll
+                for (int j = 0; j < 8; ++j) {
+                    const uint32_t d = kq[nb][ks][R16 ? 0 : j / 4][R16 ? j / 2 : j % 4];
+                    bad = bad || ring_bad<R16>(d, half_mask);
+                    x[j] = R16 ? widen16((d >> (16 * (j % 2))) & 0xffffu, half_mask)
+                               : __uint_as_float(d);
+                }
+                operands8<kKP>(x, kf, rows.spc);
+                rows.window_keys(s[nb], small[nb], kf, ks);
+            }
+        }
+#pragma unroll
+        for (int rt = 0; rt < RT; ++rt) {
+            s[0][rt] += small[0][rt];
+            s[1][rt] += small[1][rt];
+        }
+        bf16x8_t pf[RT][kVPWin];
+        rows.template weights<kVPWin, true>(s, hid, t0, pf);
+#pragma unroll
+        for (int nb = 0; nb < D / 16; ++nb) {
+            float x[8];
+            bf16x8_t vf[kVPWin];
+#pragma unroll
+            for (int j = 0; j < 8; ++j) {
+                const uint32_t d = ring_word<R16>(vr, vo[j] + 16 * E * nb);
+                bad = bad || ring_bad<R16>(d, half_mask);
+                x[j] = R16 ? widen16(d, half_mask) : __uint_as_float(d);
+            }
+            operands8<kVPWin>(x, vf, rows.spc);
+            rows.template values<kVPWin>(vf, pf, nb);
+        }
+    }
+
+    // ---- merge the four waves' states through LDS -----------------------------
+    constexpr int NR = 16 * RT;
+    float* st = reinterpret_cast<float*>(smem);              // [4][NR][D], then [4][NR] m, l
+    float* sm = st + kWaveWaves * NR * D;
+    float* sl = sm + kWaveWaves * NR;
+    __syncthreads();                                         // every wave is done with its meta
+#pragma unroll
+    for (int rt = 0; rt < RT; ++rt) {
+        const float l = row4_sum(rows.l[rt]);
+        const int r = wave * NR + 16 * rt + col;
+#pragma unroll
+        for (int nb = 0; nb < D / 16; ++nb) {
+            const f32x4_t o = rows.O[rt][nb];
+            *reinterpret_cast<float4*>(st + r * D + 16 * nb + 4 * gq) =
+                make_float4(o[0], o[1], o[2], o[3]);
+        }
+        if (gq == 0) {
+            sm[r] = rows.m[rt];
+            sl[r] = l;
+        }
+    }
+    __syncthreads();
+    for (int e = threadIdx.x; e < NR * (D / 4); e += kWaveBlock) {
+        const int i = e / (D / 4), d = 4 * (e % (D / 4)), r = row0 + i;
+        if (r >= a.rows) continue;
+        float M = -INFINITY, L = 0.f;
+#pragma unroll
+        for (int w = 0; w < kWaveWaves; ++w) M = fmaxf(M, sm[w * NR + i]);
+        float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll
+        for (int w = 0; w < kWaveWaves; ++w) {
+            const float mw = sm[w * NR + i];
+            const float f = mw == -INFINITY ? 0.f : exp2_fast(mw - M);
+            const float4 o = *reinterpret_cast<const float4*>(st + (w * NR + i) * D + d);
+            L = fmaf(f, sl[w * NR + i], L);
+            acc.x = fmaf(f, o.x, acc.x);
+            acc.y = fmaf(f, o.y, acc.y);
+            acc.z = fmaf(f, o.z, acc.z);
+            acc.w = fmaf(f, o.w, acc.w);
+        }
+        const RowDst dst = row_dst(a, b, kvh, bh, r, split, M, L, d == 0);
+        *reinterpret_cast<float4*>(dst.p + d) =
+            make_float4(acc.x * dst.f, acc.y * dst.f, acc.z * dst.f, acc.w * dst.f);
+    }
+    __syncthreads();                                         // (another walk may follow)
+    return bad;
+}
+
+template <int D, int RT, bool R16>
+__global__ __launch_bounds__(kWaveBlock) __attribute__((amdgpu_waves_per_eu(D <= 128 ? 2 : 1)))
+void attn_rows_wave_kernel(RowsLaunch a) {
+    extern __shared__ __align__(16) unsigned char smem[];
+    const int split = blockIdx.x % a.n_splits, rblock = blockIdx.x / a.n_splits;
+    const int kvh = blockIdx.y, b = blockIdx.z;
+    const int64_t bh = (int64_t)b * a.Hkv + kvh;
+    const int row0 = rblock * a.block_rows;
+    const Range rg(a, split, b, row0 + a.block_rows - 1);
+    // (every wave holds the same rows, so the answer is the workgroup's)
+    const int kind = query_kind<D, RT>(a, row0, b, kvh);
+    bool bad = kind & kSlow;
+    if (!(kind & kWide)) {
+        bad |= walk_wave<D, RT, 1, R16>(a, smem, rg, row0, bh, b, kvh, split);
+    } else {
+        for (int rt = 0; rt < RT; ++rt)
+            bad |= walk_wave<D, 1, 3, R16>(a, smem, rg, row0 + 16 * rt, bh, b, kvh, split);
+    }
+    int* word = reinterpret_cast<int*>(smem);
+    bad = __builtin_amdgcn_ballot_w64(bad) != 0;
+    if (threadIdx.x % kWave == 0) word[threadIdx.x / kWave] = bad;
+    __syncthreads();
+    if (__builtin_expect(word[0] | word[1] | word[2] | word[3], 0))
+        slow_rows<D, R16>(a, rg, row0, a.block_rows, bh, b, kvh, split);
+}
+
+// Merges the split partials: one wave per query row, the sums in split order.
+__global__ __launch_bounds__(256) void attn_rows_merge_kernel(RowsLaunch a) {
+    const int64_t row = (int64_t)blockIdx.x * 4 + threadIdx.x / kWave;
+    const int lane = threadIdx.x % kWave;
+    if (row >= (int64_t)a.B * a.Hkv * a.rows) return;
+    const int S = a.n_splits, D = a.D;
+    const float* ml = a.part_ml + row * S * 2;
+    float M = -INFINITY;
+    for (int s = 0; s < S; ++s) M = fmaxf(M, ml[2 * s]);
+    const int64_t bh = row / a.rows;
+    float* out = a.out + row_offset(a, (int)(bh / a.Hkv), (int)(bh % a.Hkv), (int)(row % a.rows));
+    const float* po = a.part_o + row * S * D;
+    for (int d = 4 * lane; d < D; d += 4 * kWave) {
+        float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
+        float L = 0.f;
+#pragma unroll 4
+        for (int s = 0; s < S; ++s) {
+            const float m = ml[2 * s];
+            const float f = m == -INFINITY ? 0.f : exp2_fast(m - M);
+            const float4 o = *reinterpret_cast<const float4*>(po + (int64_t)s * D + d);
+            L = fmaf(f, ml[2 * s + 1], L);
+            acc.x = fmaf(f, o.x, acc.x);
+            acc.y = fmaf(f, o.y, acc.y);
+            acc.z = fmaf(f, o.z, acc.z);
+            acc.w = fmaf(f, o.w, acc.w);
+        }
+        const float f = L > 0.f || L != L ? 1.f / L : 0.f;      // 0: every position hidden
+        *reinterpret_cast<float4*>(out + d) =
+            make_float4(acc.x * f, acc.y * f, acc.z * f, acc.w * f);
+    }
+}
+
+// Rows per kv head that the wave kernel takes: those of one workgroup, and at
+// head_dim 64 of two.  Kernel times, wave / shared (rows, B): head_dim 128: 36
+// rows 71 / 55 us (B=8, 4K), 26 / 26 (B=1, 8K); 64 rows 70 / 58, 28 / 28;
+// head_dim 64 (B=8, 12 heads, 2K): 40 rows 36 / 46 us, 64 rows 37 / 47, 100
+// rows 59 / 54.
+int few_rows(int D) { return D <= 64 ? 64 : D <= 128 ? 32 : 16; }
+
+template <int D, bool R16>
+int launch_rows(const RowsLaunch& a, hipStream_t st) {
+    const dim3 grid(a.row_blocks * a.n_splits, a.Hkv, a.B);
+    if (a.rows <= few_rows(D)) {
+        using S = WaveShape<D>;
+        if (a.block_rows == 16)
+            attn_rows_wave_kernel<D, 1, R16><<<grid, kWaveBlock, S::LDS, st>>>(a);
+        else
+            attn_rows_wave_kernel<D, S::RT, R16><<<grid, kWaveBlock, S::LDS, st>>>(a);
+    } else {
+        using S = SharedShape<D>;
+        if (a.block_rows == 16 * S::WAVES)
+            attn_rows_shared_kernel<D, 1, R16><<<grid, S::BLOCK, S::LDS, st>>>(a);
+        else
+            attn_rows_shared_kernel<D, S::RT, R16><<<grid, S::BLOCK, S::LDS, st>>>(a);
+    }
+    int rc = check_launch("packed_attention (rows)");
+    if (rc || a.n_splits == 1) return rc;
+    const int64_t rows = (int64_t)a.B * a.Hkv * a.rows;
+    attn_rows_merge_kernel<<<(unsigned)((rows + 3) / 4), 256, 0, st>>>(a);
+    return check_launch("packed_attention (rows merge)");
+}
+
+}  // namespace
+
+// Rows per workgroup, row blocks and splits of a call: 16 or 32 rows per
+// workgroup of the wave kernel; 128 or 256 of the shared one (64 at head_dim
+// 256).  Splits then give every CU a workgroup while each split keeps at least
+// 12 units of 32 tokens.
+RowsPlan rows_plan(int B, int Hkv, int rows, int D, int G, int n_chunks, int res_len,
+                   int splits_hint) {
+    constexpr int kCUs = 256, kMinUnits = 12;
+    RowsPlan p;
+    const bool few = rows <= few_rows(D);
+    if (few) p.block_rows = rows > 16 && D <= 128 ? 32 : 16;
+    else p.block_rows = D > 128 ? 64 : rows > 128 ? 256 : 128;
+    p.row_blocks = (rows + p.block_rows - 1) / p.block_rows;
+    const int packed = n_chunks * (G / kUnit), window = (res_len + kUnit - 1) / kUnit;
+    p.n_units = packed + window;
+    const int weight = packed + kWindowWeight * window;
+    const int64_t groups = (int64_t)B * Hkv * p.row_blocks;
+    int64_t s = splits_hint;
+    if (s <= 0) s = min(kCUs / groups, (int64_t)p.n_units / kMinUnits);
+    s = max((int64_t)1, min(s, (int64_t)p.n_units));
+    p.weight_per_split = (int)((weight + s - 1) / s);
+    p.n_splits = (weight + p.weight_per_split - 1) / p.weight_per_split;
+    return p;
+}
+
+int launch_attention_rows(const RowsLaunch& a, hipStream_t st) {
+    const bool r16 = a.res_dt != kSrcF32;
+    switch (a.D) {
+        case 64: return r16 ? launch_rows<64, true>(a, st) : launch_rows<64, false>(a, st);
+        case 128: return r16 ? launch_rows<128, true>(a, st) : launch_rows<128, false>(a, st);
+        case 256: return r16 ? launch_rows<256, true>(a, st) : launch_rows<256, false>(a, st);
+        default: return set_error(kErrUnsupported, "head_dim %d", a.D);
+    }
+}
+
+}  // namespace kivi

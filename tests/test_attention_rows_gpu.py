@@ -1,0 +1,144 @@
+"""GPU parity of attention with more query rows per kv head than one decode
+launch takes (q_len * Hq / Hkv > 8, matrix-core stores): the kernels that
+dequantise each 32 tokens once for all rows.
+
+Rows per kv head sit at the edges of the row tiles (16), of the two kernels (16,
+32 or 64 by head_dim) and of the workgroups' row blocks (64, 128, 256); contexts end inside a 32-token
+unit, lie wholly in the window, and split.  Against float64 attention over the
+oracle's dequantised history, elementwise, with the bound that the arithmetic
+gives.  Weights and values are split into two bf16 pieces each (2^-18 relative)
+and their lo*lo product is dropped (2^-18): 3 * 2^-18 of sum_t p_t |v_t|.
+Keys carry three pieces; a score is then a fp32 sum of 6 D/32 matrix products
+(three-piece queries), off by at most 6 D/32 * 2^-24 of sum_d |q_d k_d| *
+scale, which moves a weight and the normaliser by as much each.
+"""
+
+import numpy as np
+import pytest
+import torch
+
+from oracle.attention import prefix_attention
+from tests.kv_helpers import make_kv, oracle_history
+
+pytestmark = pytest.mark.gpu
+
+def _store(hip_device, B, Hkv, D, G, Gv, R, T, L, ring):
+    from intel_kivi_hybrid_amd.store import PackedKVStore
+    dt = {"f32": torch.float32, "bf16": torch.bfloat16, "f16": torch.float16}[ring]
+    k, v = make_kv(B, Hkv, T + L, D, seed=T + L + D)
+    k, v = k.to(dt).float(), v.to(dt).float()
+    st = PackedKVStore(B, Hkv, D, G, R + L, "cuda:0", group_size_v=Gv, residual_dtype=dt,
+                       chunk_capacity=T // G + 1)
+    st.extend(k[:, :, :T].to("cuda", dt), v[:, :, :T].to("cuda", dt), flush_at=R)
+    st.append(k[:, :, T:].to("cuda", dt), v[:, :, T:].to("cuda", dt))
+    return st, k, v
+
+
+def _check(out, q, st, k, v, G, Gv, **mask):
+    kh, vh = oracle_history(k, v, st.n_chunks, G, Gv)
+    q0 = st.n_chunks * G
+    qn, kr, vr = q.transpose(1, 2).numpy(), k[:, :, q0:].numpy(), v[:, :, q0:].numpy()
+    ref = prefix_attention(qn, kh, vh, kr, vr, **mask)
+    size = prefix_attention(qn, kh, np.abs(vh), kr, np.abs(vr), **mask)
+    B, L, Hq, D = qn.shape
+    keys = np.abs(np.concatenate([kh, kr], 2))
+    qa = np.abs(qn).reshape(B, L, keys.shape[1], -1, D)
+    smax = max(float((qa[b, :, h].reshape(-1, D) @ keys[b, h].T).max())
+               for b in range(B) for h in range(keys.shape[1])) * D ** -0.5
+    bound = 3 * 2.0 ** -18 + 2 * (6 * D / 32) * 2.0 ** -24 * smax
+    err = np.abs(out.cpu().numpy().astype(np.float64) - ref) / np.maximum(size, 1e-30)
+    print(f"[rows]   largest error {err.max():.2e} of sum p|v| (bound {bound:.2e})", flush=True)
+    assert err.max() <= bound
+
+
+CASES = [
+    # B, Hq, Hkv, D, G, Gv, R, T, L, splits, ring, bf16 queries
+    (1, 3, 1, 128, 32, 32, 64, 300, 3, 0, "f32", False),      # 9 rows, 3 query pieces
+    (2, 4, 1, 128, 32, 32, 64, 777, 4, 0, "bf16", True),      # 16 rows: one tile
+    (1, 17, 1, 64, 32, 32, 64, 333, 2, 3, "f16", True),       # 34 rows, 3 splits
+    (1, 8, 1, 128, 32, 32, 64, 500, 4, 0, "f32", False),      # 32 rows
+    (1, 11, 1, 128, 32, 32, 64, 500, 3, 2, "bf16", True),     # 33 rows
+    (1, 4, 2, 128, 64, 64, 128, 1300, 32, 0, "f32", True),    # 64 rows, G = 64
+    (1, 13, 1, 128, 32, 128, 64, 500, 5, 0, "bf16", False),   # 65 rows, one value group
+    (1, 8, 2, 256, 64, 128, 128, 700, 4, 2, "f32", False),    # head_dim 256, 16 rows
+    (1, 17, 1, 256, 32, 256, 64, 400, 2, 0, "f16", False),    # head_dim 256, 34 rows
+    (1, 2, 1, 256, 32, 32, 64, 400, 50, 0, "bf16", True),     # head_dim 256, 100 rows
+    (1, 4, 1, 128, 32, 32, 128, 2100, 33, 0, "bf16", True),   # 132 rows: two row tiles
+    (2, 8, 4, 64, 64, 32, 64, 1000, 129, 2, "f16", False),    # 258 rows: two row blocks
+    (1, 2, 2, 128, 32, 32, 128, 40, 300, 0, "f32", True),     # no chunk yet: the window alone
+    (1, 4, 2, 64, 32, 32, 64, 20, 5, 0, "bf16", False),       # the same, few rows
+]
+
+
+@pytest.mark.parametrize("B,Hq,Hkv,D,G,Gv,R,T,L,splits,ring,half_q", CASES)
+def test_rows_match_oracle(hip_device, B, Hq, Hkv, D, G, Gv, R, T, L, splits, ring, half_q):
+    print(f"[rows] B={B} Hq={Hq} Hkv={Hkv} D={D} G={G} Gv={Gv} R={R} T={T} L={L} splits={splits} "
+          f"{ring} half_q={half_q}", flush=True)
+    st, k, v = _store(hip_device, B, Hkv, D, G, Gv, R, T, L, ring)
+    g = torch.Generator().manual_seed(L + D)
+    q = torch.randn(B, Hq, L, D, generator=g)
+    if half_q:
+        q = q.bfloat16().float()
+    out = st.attention(q.cuda(), num_splits=splits)
+    _check(out, q, st, k, v, G, Gv)
+    assert torch.equal(out, st.attention(q.cuda(), num_splits=splits))
+    # padding: a leading run, then holes (both kernels' masks, window included)
+    total = st.quantized_tokens + st.res_len
+    start = [min(37 * (b + 1), total - L) for b in range(B)]
+    out = st.attention(q.cuda(), num_splits=splits, kv_start=start)
+    _check(out, q, st, k, v, G, Gv, kv_start=np.array(start))
+    vis = torch.rand(B, total, generator=g) >= 0.2
+    vis[:, 0] = True
+    out = st.attention(q.cuda(), num_splits=splits, key_mask=vis)
+    _check(out, q, st, k, v, G, Gv, visible=vis.numpy())
+
+
+def test_unaligned_queries(hip_device):
+    """Queries and outputs off the 16-byte alignment of the wide loads."""
+    B, Hq, L, D = 1, 8, 6, 128
+    st, k, v = _store(hip_device, B, 2, D, 32, 32, 64, 300, L, "f32")
+    q = torch.randn(B, L, Hq, D, generator=torch.Generator().manual_seed(3))
+    base = torch.empty(q.numel() + 1, device="cuda")
+    base[1:] = q.flatten().cuda()
+    out = torch.empty(q.numel() + 1, device="cuda")[1:].view(B, L, Hq, D)
+    st.attention(base[1:].view(B, L, Hq, D).transpose(1, 2), out=out)
+    _check(out, q.transpose(1, 2), st, k, v, 32, 32)
+
+
+def test_negative_scale_and_hidden_rows(hip_device):
+    """A negative softmax scale turns the order of the scores; a sequence with
+    every position hidden gives zeros."""
+    st, k, v = _store(hip_device, 2, 1, 128, 32, 32, 64, 300, 8, "f32")
+    q = torch.randn(2, 4, 8, 128, generator=torch.Generator().manual_seed(1))
+    out = st.attention(q.cuda(), softmax_scale=-(128 ** -0.5))
+    _check(out, -q, st, k, v, 32, 32)
+    mask = torch.ones(2, st.quantized_tokens + st.res_len)
+    mask[1] = 0
+    out = st.attention(q.cuda(), key_mask=mask)
+    assert torch.equal(out[1], torch.zeros_like(out[1])) and bool((out[0] != 0).any())
+
+
+@pytest.mark.parametrize("ring,L", [("f32", 5), ("f32", 40), ("bf16", 5), ("bf16", 40)])
+def test_infinite_window_elements(hip_device, ring, L):
+    """An infinite key gives -inf scores (no weight) or poisons the rows that
+    see it, an infinite value makes its channel infinite: what fp32 sums give,
+    whatever the pieces."""
+    Hq, D, R, T = 4, 128, 64, 200
+    st, k, v = _store(hip_device, 1, 1, D, 32, 32, R, T, L, ring)
+    q = torch.rand(1, Hq, L, D, generator=torch.Generator().manual_seed(2)) + 0.5
+    q = q.bfloat16().float()
+    t = st.res_len - L - 3                     # a window token every query sees
+    slot = (st.res_start + t) % st.R
+    st.k_res[0, 0, slot, 7] = -float("inf")    # scores -inf: the token drops out
+    out = st.attention(q.cuda())
+    total = st.quantized_tokens + st.res_len
+    mask = torch.ones(1, total)
+    mask[0, st.quantized_tokens + t] = 0
+    kk = k.clone()
+    _check(out, q, st, kk, v, 32, 32, visible=mask.numpy().astype(bool))
+    st.k_res[0, 0, slot, 7] = 1.0
+    st.v_res[0, 0, slot, 9] = float("inf")
+    out = st.attention(q.cuda()).cpu()
+    assert bool(torch.isinf(out[..., 9]).all())
+    rest = torch.cat([out[..., :9], out[..., 10:]], -1)
+    assert bool(torch.isfinite(rest).all())

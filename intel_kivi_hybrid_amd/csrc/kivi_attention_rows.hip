@@ -56,12 +56,6 @@ constexpr int kTile = kWave * 16;           // bytes of one operand tile
 
 constexpr uint32_t kNotFinite = 0x7f7f8000u;  // |x| from here on rounds to infinity as bf16
 
-typedef const __attribute__((address_space(1))) char* gptr;
-template <class T>
-__device__ __forceinline__ T gload(gptr base, uint32_t off) {
-    return *reinterpret_cast<const __attribute__((address_space(1))) T*>(base + off);
-}
-
 template <bool V>
 struct BoolC {
     static constexpr bool value = V;
@@ -137,13 +131,26 @@ __device__ __forceinline__ int window_slot(const RowsLaunch& a, int t) {
     return s >= a.Rcap ? s - a.Rcap : s;
 }
 
-// Is an element (R16: one of the two) of this ring dword not finite as bf16?
+// The largest magnitudes of ring dwords (R16: of each half), and whether one of
+// them is not finite as bf16.
+typedef uint16_t u16x2_t __attribute__((ext_vector_type(2)));
 template <bool R16>
-__device__ __forceinline__ bool ring_bad(uint32_t d, uint32_t half_mask) {
-    if constexpr (!R16) return (d & 0x7fffffffu) >= kNotFinite;
-    const uint32_t lim = half_mask ? 0x7c00u : 0x7f80u;
-    return (d & 0x7fffu) >= lim || ((d >> 16) & 0x7fffu) >= lim;
-}
+struct RingTop {
+    uint32_t top = 0;
+    __device__ __forceinline__ void add(uint32_t d) {
+        if constexpr (R16)
+            top = __builtin_bit_cast(uint32_t, __builtin_elementwise_max(
+                      __builtin_bit_cast(u16x2_t, top),
+                      __builtin_bit_cast(u16x2_t, d & 0x7fff7fffu)));
+        else
+            top = max(top, d & 0x7fffffffu);
+    }
+    __device__ __forceinline__ bool bad(uint32_t half_mask) const {
+        if constexpr (!R16) return top >= kNotFinite;
+        const uint32_t lim = half_mask ? 0x7c00u : 0x7f80u;
+        return (top & 0xffffu) >= lim || (top >> 16) >= lim;
+    }
+};
 
 // What the wave's query values of rows row0 + 16 rt + l % 16 need: kWide if
 // some are not bf16 (three pieces), kSlow if some are not finite as bf16.
@@ -529,10 +536,8 @@ struct PackedUnit {
     static constexpr int N = SharedShape<D>::WORDS;
     uint32_t word[N];
     kivi_f4v sc[N][2], zr[N][2];
-    // at chunk 0 of the (batch, kv head): wave-uniform bases (global pointers:
-    // a load through a selected generic pointer would count as an LDS access
-    // too, and every LDS wait would wait for it), bytes per chunk and per
-    // second unit of a G = 64 chunk, and this lane's bytes
+    // at chunk 0 of the (batch, kv head): wave-uniform bases, bytes per chunk
+    // and per second unit of a G = 64 chunk, and this lane's bytes
     gptr code[N], scale[N], zero[N];
     uint32_t code_step[N], code_half[N], meta_step[N], meta_half[N], code_off[N], meta_off[N];
 
@@ -635,17 +640,16 @@ struct WindowUnit {
             }
         }
     }
-    // (returns whether some element is not finite as bf16)
-    __device__ __forceinline__ bool expand(unsigned char* buf, const Dst<D>& d, int wave,
-                                           uint32_t half_mask, SplitConsts k) const {
-        bool bad = false;
-        if (!has_word<D>(wave)) return bad;
+    __device__ __forceinline__ void expand(unsigned char* buf, const Dst<D>& d, int wave,
+                                           uint32_t half_mask, RingTop<R16>& top,
+                                           SplitConsts k) const {
+        if (!has_word<D>(wave)) return;
 #pragma unroll
         for (int i = 0; i < N; ++i) {
             const bool key = word_of<D>(i, wave).key;
 #pragma unroll
             for (int j = 0; j < 16; ++j)
-                if (!R16 || !key || j % 8 < 4) bad = bad || ring_bad<R16>(raw[i][j], half_mask);
+                if (!R16 || !key || j % 8 < 4) top.add(raw[i][j]);
 #pragma unroll
             for (int m = 0; m < 2; ++m) {
                 float x[8];
@@ -658,7 +662,6 @@ struct WindowUnit {
                 put_tile<3>(buf + d.at[i] + m * d.tile[i], d.half[i], x, k);
             }
         }
-        return bad;
     }
 };
 
@@ -769,6 +772,7 @@ __device__ bool walk_shared(const RowsLaunch& a, unsigned char* smem, const Rang
     const int w_begin = max(rg.begin, rg.n_cu), w_end = rg.w_end();
     if (w_begin < w_end) {
         WindowUnit<D, R16> unit;
+        RingTop<R16> top;
         const uint32_t half_mask = a.res_dt == kSrcF16 ? ~0u : 0u;
         const Dst<D> dst(wave, lane, kVPWin);
         unit.load(a, bh, kUnit * (w_begin - rg.n_cu), wave, lane);
@@ -776,11 +780,12 @@ __device__ bool walk_shared(const RowsLaunch& a, unsigned char* smem, const Rang
             const int t0 = kUnit * (u - rg.n_cu);
             const uint32_t hid = rg.hidden(u);
             lds_barrier();                     // the previous unit has been read
-            bad |= unit.expand(smem, dst, wave, half_mask, rows.spc);
+            unit.expand(smem, dst, wave, half_mask, top, rows.spc);
             unit.load(a, bh, t0 + kUnit, wave, lane);
             lds_barrier();
             if (active) use_unit(smem, hid, t0, BoolC<true>{}, kVPWin, [] {}, [] {});
         }
+        bad = top.bad(half_mask);
     }
 
     if (!active) return bad;
@@ -847,8 +852,8 @@ void attn_rows_shared_kernel(RowsLaunch a) {
 //
 // What bounds it: the expansion's vector work, ~800 instructions per unit
 // (4-5.5 cycles each) against 1536 cycles of matrix products for two row tiles;
-// a second wave per SIMD gains nothing (38 us against 37 us at B=8, 5 query
-// tokens over 4K), so a workgroup per CU is the plan's target.
+// two workgroups per CU gain little over one (39 against 42 us at B=8, 5 query
+// tokens over 4K).
 // ---------------------------------------------------------------------------
 constexpr int kWaveWaves = 4, kWaveBlock = kWaveWaves * kWave;
 
@@ -964,7 +969,7 @@ __device__ bool walk_wave(const RowsLaunch& a, unsigned char* smem, const Range&
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
     Rows<D, RT, NQ> rows;
     rows.init(a, row0, b, kvh);
-    bool bad = false;
+    RingTop<R16> top;
     const int ng = D / a.Gv;
     float* mt = reinterpret_cast<float*>(smem + wave * WaveShape<D>::META);
 
@@ -1059,7 +1064,7 @@ __device__ bool walk_wave(const RowsLaunch& a, unsigned char* smem, const Range&
 #pragma unroll
                 for (int j = 0; j < 8; ++j) {
                     const uint32_t d = kq[nb][ks][R16 ? 0 : j / 4][R16 ? j / 2 : j % 4];
-                    bad = bad || ring_bad<R16>(d, half_mask);
+                    top.add(d);
                     x[j] = R16 ? widen16((d >> (16 * (j % 2))) & 0xffffu, half_mask)
                                : __uint_as_float(d);
                 }
@@ -1081,7 +1086,7 @@ __device__ bool walk_wave(const RowsLaunch& a, unsigned char* smem, const Range&
 #pragma unroll
             for (int j = 0; j < 8; ++j) {
                 const uint32_t d = ring_word<R16>(vr, vo[j] + 16 * E * nb);
-                bad = bad || ring_bad<R16>(d, half_mask);
+                top.add(d);
                 x[j] = R16 ? widen16(d, half_mask) : __uint_as_float(d);
             }
             operands8<kVPWin>(x, vf, rows.spc);
@@ -1134,7 +1139,7 @@ __device__ bool walk_wave(const RowsLaunch& a, unsigned char* smem, const Range&
             make_float4(acc.x * dst.f, acc.y * dst.f, acc.z * dst.f, acc.w * dst.f);
     }
     __syncthreads();                                         // (another walk may follow)
-    return bad;
+    return top.bad(half_mask);
 }
 
 template <int D, int RT, bool R16>
@@ -1229,8 +1234,8 @@ int launch_rows(const RowsLaunch& a, hipStream_t st) {
 
 // Rows per workgroup, row blocks and splits of a call: 16 or 32 rows per
 // workgroup of the wave kernel; 128 or 256 of the shared one (64 at head_dim
-// 256).  Splits then give every CU a workgroup while each split keeps at least
-// 12 units of 32 tokens.
+// 256).  Splits then give every CU a workgroup (two of the wave kernel) while
+// each split keeps at least 12 units of 32 tokens.
 RowsPlan rows_plan(int B, int Hkv, int rows, int D, int G, int n_chunks, int res_len,
                    int splits_hint) {
     constexpr int kCUs = 256, kMinUnits = 12;
@@ -1244,7 +1249,7 @@ RowsPlan rows_plan(int B, int Hkv, int rows, int D, int G, int n_chunks, int res
     const int weight = packed + kWindowWeight * window;
     const int64_t groups = (int64_t)B * Hkv * p.row_blocks;
     int64_t s = splits_hint;
-    if (s <= 0) s = min(kCUs / groups, (int64_t)p.n_units / kMinUnits);
+    if (s <= 0) s = min((few ? 2 : 1) * kCUs / groups, (int64_t)p.n_units / kMinUnits);
     s = max((int64_t)1, min(s, (int64_t)p.n_units));
     p.weight_per_split = (int)((weight + s - 1) / s);
     p.n_splits = (weight + p.weight_per_split - 1) / p.weight_per_split;

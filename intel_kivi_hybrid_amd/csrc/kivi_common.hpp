@@ -302,6 +302,16 @@ __device__ __forceinline__ void store_stream(uint32_t* p, uint32_t v) {
     __builtin_nontemporal_store(v, p);
 }
 
+// Global-memory loads from a wave-uniform base and a per-lane byte offset (one
+// instruction, no 64-bit address per lane).  The pointer names its address
+// space: a load through a selected generic pointer would be a flat load, which
+// counts as an LDS access too, so that every LDS wait waits for it.
+typedef const __attribute__((address_space(1))) char* gptr;
+template <class T>
+__device__ __forceinline__ T gload(gptr base, uint32_t off) {
+    return *reinterpret_cast<const __attribute__((address_space(1))) T*>(base + off);
+}
+
 // Workgroup barrier that orders LDS accesses only.  __syncthreads() also
 // waits for every outstanding global load and store (s_waitcnt vmcnt(0)),
 // which would drain a prefetch issued before the barrier.  Only for kernels

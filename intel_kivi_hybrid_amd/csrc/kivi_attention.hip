@@ -87,6 +87,8 @@ __device__ __forceinline__ int ring_slot(int start, int t, int cap) {
     return s >= cap ? s - cap : s;
 }
 
+// The general kernel of plain-layout stores whose value factors ([D/Gv][G]
+// per chunk) are more than kivi_attention_plain.hip keeps (256).
 template <int HG>
 __global__ __launch_bounds__(kAttnBlock) void attn_generic_kernel(AttnArgs a) {
     extern __shared__ float smem[];
@@ -416,16 +418,18 @@ __global__ __launch_bounds__(kMaxD) void attn_merge_regs_kernel(const float* __r
 
 struct Plan {
     int layout;
-    bool mfma;                                // matrix-core kernel (else the generic one)
+    bool mfma;                                // matrix-core kernel
+    bool plain;                               // plain-layout kernel (else the generic one)
     int n_units, n_splits, units_per_split;   // generic kernel
     int n_qsplits, chunks_per_wave, res_waves, early_per_pass_x2;   // matrix-core kernel
 };
 
 // empty_ok: the caller can give the matrix-core kernel a readable chunk 0
 // (non-null chunk arrays with capacity for one chunk) when the context has
-// no chunk yet.
+// no chunk yet.  plain_rows: query rows per kv head of a launch of the
+// plain-layout kernel.
 Plan make_plan(int B, int Hkv, int D, int G, int Gv, int n_chunks, int res_len,
-               int splits_hint, bool empty_ok = true) {
+               int splits_hint, int plain_rows, bool empty_ok = true) {
     Plan p{};
     p.layout = code_layout_for(D, G, Gv);
     if (p.layout == kLayoutMfma && n_chunks == 0) {
@@ -437,6 +441,7 @@ Plan make_plan(int B, int Hkv, int D, int G, int Gv, int n_chunks, int res_len,
         // not depend on which.  B=1 and 16, 32/8 heads, 100-127 tokens: 32-43
         // us per call on the generic kernel.
         p.mfma = empty_ok;
+        p.plain = !empty_ok && plain_attention_supported(D, G, Gv);
         p.n_units = (res_len + kWave - 1) / kWave;
         p.units_per_split = p.n_units;
         p.n_qsplits = p.n_splits = 1;
@@ -507,6 +512,26 @@ Plan make_plan(int B, int Hkv, int D, int G, int Gv, int n_chunks, int res_len,
         p.n_splits = p.n_qsplits;
         return p;
     }
+    p.plain = plain_attention_supported(D, G, Gv);
+    if (p.plain) {
+        // The most splits whose workgroups fit the chip at once while every
+        // wave keeps at least 3 chunks.  head_dim 96, 4K context, us per call:
+        // B=4, 32/32 heads (four workgroups per CU fit): 6, 8, 15 splits 26.4,
+        // 25.6, 28.5; B=16, 32/8 heads (three fit): 4, 6, 7 splits 49.7, 46.5,
+        // 60.2; B=8, 64/8 heads at 8K (two fit): 6, 8, 10 splits 102, 81, 125.
+        constexpr int kWavesPerGroup = 4, kCUs = 256, kMinChunksPerWave = 3;
+        int S = splits_hint;
+        if (S <= 0)
+            S = min(kCUs * plain_attention_groups_per_cu(plain_rows, D, G, Gv) / (B * Hkv),
+                    n_chunks / (kWavesPerGroup * kMinChunksPerWave));
+        S = max(1, min(min(S, kMaxSplits), (n_chunks + kWavesPerGroup - 1) / kWavesPerGroup));
+        p.chunks_per_wave = (n_chunks + kWavesPerGroup * S - 1) / (kWavesPerGroup * S);
+        p.n_qsplits = n_chunks == 0 ? 1
+                                    : (n_chunks + kWavesPerGroup * p.chunks_per_wave - 1) /
+                                          (kWavesPerGroup * p.chunks_per_wave);
+        p.n_splits = p.n_qsplits;
+        return p;
+    }
     p.n_units = n_chunks + (res_len + kWave - 1) / kWave;
     int S = splits_hint;
     if (S <= 0) {
@@ -543,6 +568,12 @@ int rows_for(int n) { return n <= 1 ? 1 : n <= 2 ? 2 : n <= 4 ? 4 : 8; }
 // take 4 rows.
 int max_rows(bool mfma, int D, int G, int Gv) {
     return (mfma && D == 256 && G == 64 && Gv != 32 && Gv != D) ? 4 : 8;
+}
+
+// Rows per kv head of one launch of the plain-layout kernel.
+int plain_rows_for(int hg, int q_len) {
+    const int hl = hg < 8 ? hg : 8;
+    return rows_for(max(1, min(8 / hl, q_len)) * hl);
 }
 
 // Query heads per kv head that one launch covers: all of them up to
@@ -696,7 +727,7 @@ size_t workspace_for(int batch, int q_len, int q_heads, int kv_heads, int head_d
                         sizeof(float);
     }
     const Plan p = make_plan(batch, kv_heads, head_dim, group_size_k, group_size_v, num_chunks,
-                             res_len, num_splits);
+                             res_len, num_splits, plain_rows_for(q_heads / kv_heads, q_len));
     if (!needs_workspace(p)) return rows_need;
     const int hl = heads_per_launch(q_heads / kv_heads,
                                     max_rows(p.mfma, head_dim, group_size_k, group_size_v));
@@ -798,7 +829,7 @@ int attention_impl(const float* q, int32_t q_len, int32_t causal, const int32_t*
     const bool empty_ok = chunk_capacity >= 1 && k_codes && k_scale && k_zero && v_codes &&
                           v_scale && v_zero;
     const Plan p = make_plan(batch, kv_heads, head_dim, group_size_k, group_size_v, num_chunks,
-                             res_len, num_splits, empty_ok);
+                             res_len, num_splits, plain_rows_for(hg, q_len), empty_ok);
     const int hl = heads_per_launch(hg, max_rows(p.mfma, head_dim, group_size_k, group_size_v));
     const int tpl = tokens_per_launch(hl, q_len, p.mfma, head_dim, group_size_k, group_size_v);
     const int rows = rows_for(tpl * hl);
@@ -817,7 +848,7 @@ int attention_impl(const float* q, int32_t q_len, int32_t causal, const int32_t*
     hipStream_t st = (hipStream_t)stream;
     const int new_slot = k_new ? (res_start + res_len - 1) % res_capacity : 0;
     if (k_new && !p.mfma) {
-        // the generic kernel reads the ring only: file the token there first
+        // the other kernels read the ring only: file the token there first
         rc = kivi_store_append(k_new, v_new, res_dtype, new_sb, new_sh, 0, 1,
                                const_cast<void*>(k_res), const_cast<void*>(v_res), res_dtype,
                                batch, kv_heads, head_dim, res_capacity, new_slot, stream);
@@ -842,7 +873,7 @@ int attention_impl(const float* q, int32_t q_len, int32_t causal, const int32_t*
         qr.rows = rows;
         const float* qi = q + i0 * tok_stride;
         float* oi = out + i0 * tok_stride;
-        if (p.mfma) {
+        if (p.mfma || p.plain) {
             AttnLaunch L{qi, k_codes, k_scale, k_zero, v_codes, v_scale, v_zero, k_res, v_res,
                          oi, part_o, part_ml, batch, q_heads, kv_heads, head_dim, group_size_k,
                          group_size_v, chunk_capacity, num_chunks, res_capacity, res_start,
@@ -851,10 +882,10 @@ int attention_impl(const float* q, int32_t q_len, int32_t causal, const int32_t*
                          // context: 134.2 -> 130.6 us; 5 and 7 per pass
                          // 132.4 and 132.6 us)
                          p.early_per_pass_x2 * (rows >= 8 ? 2 : 1), p.n_splits,
-                         softmax_scale * kLog2e, k_new, v_new,
-                         new_sb, new_sh, new_slot, res_dtype, qr, kv_start, hidden,
+                         softmax_scale * kLog2e, p.mfma ? k_new : nullptr,
+                         p.mfma ? v_new : nullptr, new_sb, new_sh, new_slot, res_dtype, qr, kv_start, hidden,
                          hidden_stride};
-            rc = launch_attention_mfma(L, st);
+            rc = p.mfma ? launch_attention_mfma(L, st) : launch_attention_plain(L, st);
         } else {
             AttnArgs a{qi, k_codes, k_scale, k_zero, v_codes, v_scale, v_zero, k_res, v_res, oi,
                        part_o, part_ml, q_heads, kv_heads, head_dim, group_size_k, group_size_v,

@@ -101,6 +101,14 @@ int launch_attention_mfma_hg2_r16(const AttnLaunch& a, hipStream_t stream);
 int launch_attention_mfma_hg4_r16(const AttnLaunch& a, hipStream_t stream);
 int launch_attention_mfma_hg8_r16(const AttnLaunch& a, hipStream_t stream);
 
+// The fp32 kernel of plain-layout stores (kivi_attention_plain.hip), for up to
+// 8 rows per kv head: AttnLaunch without k_new (the ring holds the token
+// already), n_splits and chunks_per_wave as for the matrix-core kernel.
+bool plain_attention_supported(int D, int G, int Gv);
+int launch_attention_plain(const AttnLaunch& a, hipStream_t stream);
+// Workgroups of it that a CU holds (query rows per kv head of the launch).
+int plain_attention_groups_per_cu(int rows, int D, int G, int Gv);
+
 // Attention of many query rows per kv head (kivi_attention_rows.hip): query
 // row r of a kv head is query token r / hg, head r % hg, r < rows = q_len *
 // hg.  Contexts are walked in units of 32 tokens, the packed chunks' first,

@@ -426,10 +426,9 @@ struct Plan {
 
 // empty_ok: the caller can give the matrix-core kernel a readable chunk 0
 // (non-null chunk arrays with capacity for one chunk) when the context has
-// no chunk yet.  plain_rows: query rows per kv head of a launch of the
-// plain-layout kernel.
+// no chunk yet.  rows: query rows per kv head of a launch (rows_per_launch).
 Plan make_plan(int B, int Hkv, int D, int G, int Gv, int n_chunks, int res_len,
-               int splits_hint, int plain_rows, bool empty_ok = true) {
+               int splits_hint, int rows, bool empty_ok = true) {
     Plan p{};
     p.layout = code_layout_for(D, G, Gv);
     if (p.layout == kLayoutMfma && n_chunks == 0) {
@@ -457,7 +456,14 @@ Plan make_plan(int B, int Hkv, int D, int G, int Gv, int n_chunks, int res_len,
         // (a) the most splits whose workgroups still fit the chip at once
         //     (512: two per CU) while every wave keeps >= 16 chunks, so that
         //     one wave per workgroup takes the residual window alone;
-        // (b) enough splits for 256 workgroups (one per CU).
+        // (b) enough splits for 256 workgroups (one per CU);
+        // and in their place (c) the splits whose workgroups fill all 512
+        // places exactly, where every wave keeps >= 9 chunks (6 with 8 query
+        // rows, whose chunk steps cost twice): an unfilled chip leaves CUs with
+        // one workgroup idle while the others finish two.  B=16 sequences
+        // (bf16 ring), us per call: 64/8 heads at 7777 tokens 46.3 -> 41.8 (3 ->
+        // 4 splits), at 4000 35.2 -> 29.7 (2 -> 4); 32/8 heads at 7777 37.2 ->
+        // 33.6; B=32, 32/8 heads at 3000 39.3 -> 31.1 (1 -> 2).
         // Swept over B = 1-64 sequences at 2K-32K contexts (32/8 heads, the
         // best split count per shape against this rule's): B=12 at 8K takes
         // 4 splits (31.5 us; the 2048-wave target below took 6: 39.6 us, 576
@@ -482,6 +488,10 @@ Plan make_plan(int B, int Hkv, int D, int G, int Gv, int n_chunks, int res_len,
                         kMinChunksForOneResWave)
                         sa = s;
                 S = max(max(sa, kCUs / pairs), 1);
+                const int sc = kSlots / pairs;
+                if (sc > S && sc * pairs == kSlots &&
+                    n_chunks >= kWavesPerGroup * sc * (rows >= 8 ? 6 : 9))
+                    S = sc;
             } else {
                 S = (kTargetWaves + kWavesPerGroup * pairs - 1) / (kWavesPerGroup * pairs);
             }
@@ -522,7 +532,7 @@ Plan make_plan(int B, int Hkv, int D, int G, int Gv, int n_chunks, int res_len,
         constexpr int kWavesPerGroup = 4, kCUs = 256, kMinChunksPerWave = 3;
         int S = splits_hint;
         if (S <= 0)
-            S = min(kCUs * plain_attention_groups_per_cu(plain_rows, D, G, Gv) / (B * Hkv),
+            S = min(kCUs * plain_attention_groups_per_cu(rows, D, G, Gv) / (B * Hkv),
                     n_chunks / (kWavesPerGroup * kMinChunksPerWave));
         S = max(1, min(min(S, kMaxSplits), (n_chunks + kWavesPerGroup - 1) / kWavesPerGroup));
         p.chunks_per_wave = (n_chunks + kWavesPerGroup * S - 1) / (kWavesPerGroup * S);
@@ -570,8 +580,9 @@ int max_rows(bool mfma, int D, int G, int Gv) {
     return (mfma && D == 256 && G == 64 && Gv != 32 && Gv != D) ? 4 : 8;
 }
 
-// Rows per kv head of one launch of the plain-layout kernel.
-int plain_rows_for(int hg, int q_len) {
+// Rows per kv head of one launch where neither LDS nor registers allow fewer
+// than 8 (they do not for the plain-layout kernel and head_dim 128).
+int rows_per_launch(int hg, int q_len) {
     const int hl = hg < 8 ? hg : 8;
     return rows_for(max(1, min(8 / hl, q_len)) * hl);
 }
@@ -727,7 +738,7 @@ size_t workspace_for(int batch, int q_len, int q_heads, int kv_heads, int head_d
                         sizeof(float);
     }
     const Plan p = make_plan(batch, kv_heads, head_dim, group_size_k, group_size_v, num_chunks,
-                             res_len, num_splits, plain_rows_for(q_heads / kv_heads, q_len));
+                             res_len, num_splits, rows_per_launch(q_heads / kv_heads, q_len));
     if (!needs_workspace(p)) return rows_need;
     const int hl = heads_per_launch(q_heads / kv_heads,
                                     max_rows(p.mfma, head_dim, group_size_k, group_size_v));
@@ -829,7 +840,7 @@ int attention_impl(const float* q, int32_t q_len, int32_t causal, const int32_t*
     const bool empty_ok = chunk_capacity >= 1 && k_codes && k_scale && k_zero && v_codes &&
                           v_scale && v_zero;
     const Plan p = make_plan(batch, kv_heads, head_dim, group_size_k, group_size_v, num_chunks,
-                             res_len, num_splits, plain_rows_for(hg, q_len), empty_ok);
+                             res_len, num_splits, rows_per_launch(hg, q_len), empty_ok);
     const int hl = heads_per_launch(hg, max_rows(p.mfma, head_dim, group_size_k, group_size_v));
     const int tpl = tokens_per_launch(hl, q_len, p.mfma, head_dim, group_size_k, group_size_v);
     const int rows = rows_for(tpl * hl);

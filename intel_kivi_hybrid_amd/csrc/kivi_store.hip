@@ -617,6 +617,237 @@ bool launch_fast(FlushArgs a, int src, int mode, int first, int count, int bh, h
     return false;
 }
 
+// Plain layout with every value group in 1 to 64 adjacent lanes (Gv / 4 a
+// power of two) and at most TPT tokens per thread.  One workgroup per (b,
+// kv-head, chunk): thread (segment s, quad c) loads channels 4c..4c+3 of
+// tokens s, s + segments, .. of K and V at once and keeps them in registers,
+// so each tensor is read once and no tile passes through LDS.  Keys: a
+// segment's channel minima and maxima combine through LDS, one thread per
+// channel.  Values: a group is adjacent lanes of one row and combines with
+// DPP.  Codes go to LDS, a byte per token and quad, and leave in whole dwords:
+// keys in that order, values as [quad][token], whose dwords hold four tokens
+// of four channels and are transposed bit-wise.  Same codes, scales, zeros and
+// history as flush_kernel, which walks a channel or group per thread in LDS
+// with a divide per element.  Bound by the VALU, close to the loads:
+// 128 heads of 4000 tokens, head_dim 96, G = Gv = 32: fp32 196 -> 98 us (a copy
+// of its bytes takes 86), bf16 189 -> 85; 64 / 16 / 16, 128 heads of 4100, fp32
+// 169 -> 76.
+template <int TPT, int SRC>
+__global__ __launch_bounds__(kFlushBlock) void flush_plain_kernel(FlushArgs a, int segs) {
+    extern __shared__ __align__(16) unsigned char smem[];
+    const int D = a.D, G = a.G, D4 = D / 4, NG = D / a.Gv, N4 = G * D4;
+    const int group_lanes = a.Gv / 4;
+    float* const pmin = reinterpret_cast<float*>(smem);             // [segs][D]
+    float* const pmax = pmin + segs * D;
+    float* const kmin = pmax + segs * D;                            // [D]
+    float* const kscl = kmin + D;
+    float* const krcp = kscl + D;
+    float* const vscl = krcp + D;                                   // [NG][G]
+    float* const vzro = vscl + NG * G;
+    uint32_t* const kcodes = reinterpret_cast<uint32_t*>(vzro + NG * G);   // bytes [G][D4]
+    uint32_t* const vcodes = kcodes + N4 / 4;                       // bytes [D4][G]
+
+    const int tid = threadIdx.x, nthr = blockDim.x;
+    const int seg = tid / D4, quad = tid % D4;
+    const int bh = blockIdx.x;
+    const int chunk = a.chunk + (int)blockIdx.y;
+    const int vt0 = (int)blockIdx.y * G;
+    const int64_t chunk_id = (int64_t)bh * a.Cmax + chunk;
+    const int64_t hist_row0 = (int64_t)bh * a.hist_cap + (int64_t)chunk * G;
+
+    float4 kx[TPT], vx[TPT];
+    // (the last segments' tokens past the chunk repeat its last one: minima
+    // and maxima are the same, and their codes are not stored)
+    if (seg < segs) {
+        const int64_t new_base =
+            (int64_t)(bh / a.H) * a.new_sb + (int64_t)(bh % a.H) * a.new_sh + 4 * quad;
+        if (vt0 >= a.res_len) {
+#pragma unroll
+            for (int n = 0; n < TPT; ++n) {
+                const int t = min(seg + n * segs, G - 1);
+                const int64_t at = new_base + (int64_t)(vt0 + t - a.res_len) * a.new_st;
+                kx[n] = load4_vec<SRC>(a.k_new, at);
+                vx[n] = load4_vec<SRC>(a.v_new, at);
+            }
+        } else {
+            const int64_t res_base = (int64_t)bh * a.Rcap * D + 4 * quad;
+#pragma unroll
+            for (int n = 0; n < TPT; ++n) {
+                const int vt = vt0 + min(seg + n * segs, G - 1);
+                if (vt < a.res_len) {
+                    const int64_t at = res_base + (int64_t)ring(a.res_start, vt, a.Rcap) * D;
+                    kx[n] = load4_dt(a.k_res, at, a.res_dt);
+                    vx[n] = load4_dt(a.v_res, at, a.res_dt);
+                } else {
+                    const int64_t at = new_base + (int64_t)(vt - a.res_len) * a.new_st;
+                    kx[n] = load4_vec<SRC>(a.k_new, at);
+                    vx[n] = load4_vec<SRC>(a.v_new, at);
+                }
+            }
+        }
+
+        // ---- keys: this segment's part of the channels' minima and maxima ----
+        float4 mn = kx[0], mx = kx[0];
+#pragma unroll
+        for (int n = 0; n < TPT; ++n) {
+            mn.x = fmin_nan(mn.x, kx[n].x); mx.x = fmax_nan(mx.x, kx[n].x);
+            mn.y = fmin_nan(mn.y, kx[n].y); mx.y = fmax_nan(mx.y, kx[n].y);
+            mn.z = fmin_nan(mn.z, kx[n].z); mx.z = fmax_nan(mx.z, kx[n].z);
+            mn.w = fmin_nan(mn.w, kx[n].w); mx.w = fmax_nan(mx.w, kx[n].w);
+        }
+        *reinterpret_cast<float4*>(pmin + seg * D + 4 * quad) = mn;
+        *reinterpret_cast<float4*>(pmax + seg * D + 4 * quad) = mx;
+    }
+    auto encode = [&](const float (&x)[4], const float (&mn)[4], const float (&sc)[4],
+                      const float (&rc)[4], uint32_t (&q)[4]) {
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+            bool bad = false;
+            q[c] = code_fast(x[c], mn[c], rc[c], bad);
+            if (__builtin_expect(bad, 0)) q[c] = code_slow(x[c], mn[c], sc[c], rc[c]);
+        }
+    };
+
+    // ---- values: whole groups of adjacent lanes --------------------------------
+    if (seg < segs) {
+#pragma unroll
+        for (int n = 0; n < TPT; ++n) {
+            const int t = seg + n * segs;
+            const float x[4] = {vx[n].x, vx[n].y, vx[n].z, vx[n].w};
+            float mn = fmin_nan(fmin_nan(x[0], x[1]), fmin_nan(x[2], x[3]));
+            float mx = fmax_nan(fmax_nan(x[0], x[1]), fmax_nan(x[2], x[3]));
+            switch (group_lanes) {
+                case 2: seg_min_max<2>(mn, mx); break;
+                case 4: seg_min_max<4>(mn, mx); break;
+                case 8: seg_min_max<8>(mn, mx); break;
+                case 16: seg_min_max<16>(mn, mx); break;
+                case 32: seg_min_max<32>(mn, mx); break;
+                case 64: seg_min_max<64>(mn, mx); break;
+                default: break;
+            }
+            float scale;
+            finish_group(mn, mx, scale);
+            const float rc = crcp_or_nan(scale);
+            const float mn4[4] = {mn, mn, mn, mn}, sc4[4] = {scale, scale, scale, scale},
+                        rc4[4] = {rc, rc, rc, rc};
+            uint32_t q[4];
+            encode(x, mn4, sc4, rc4, q);
+            if (t < G) {
+                reinterpret_cast<uint8_t*>(vcodes)[quad * G + t] =
+                    (uint8_t)(q[0] | (q[1] << 2) | (q[2] << 4) | (q[3] << 6));
+                if (quad % group_lanes == 0) {
+                    vscl[quad / group_lanes * G + t] = scale;
+                    vzro[quad / group_lanes * G + t] = mn;
+                }
+                if (a.v_hist)
+                    *reinterpret_cast<float4*>(a.v_hist + (hist_row0 + t) * D + 4 * quad) =
+                        make_float4(decode1(q[0], scale, mn), decode1(q[1], scale, mn),
+                                    decode1(q[2], scale, mn), decode1(q[3], scale, mn));
+            }
+        }
+    }
+    lds_barrier();
+
+    // ---- keys: each channel's group ----------------------------------------------
+    for (int d = tid; d < D; d += nthr) {
+        float mn = 1e30f, mx = -1e30f, scale;
+        for (int s = 0; s < segs; ++s) {
+            mn = fmin_nan(mn, pmin[s * D + d]);
+            mx = fmax_nan(mx, pmax[s * D + d]);
+        }
+        finish_group(mn, mx, scale);
+        a.k_scale[chunk_id * D + d] = scale;
+        a.k_zero[chunk_id * D + d] = mn;
+        kmin[d] = mn;
+        kscl[d] = scale;
+        krcp[d] = crcp_or_nan(scale);
+    }
+    lds_barrier();
+    if (seg < segs) {
+        const float4 m = reinterpret_cast<const float4*>(kmin)[quad];
+        const float4 s = reinterpret_cast<const float4*>(kscl)[quad];
+        const float4 r = reinterpret_cast<const float4*>(krcp)[quad];
+        const float mn4[4] = {m.x, m.y, m.z, m.w}, sc4[4] = {s.x, s.y, s.z, s.w},
+                    rc4[4] = {r.x, r.y, r.z, r.w};
+#pragma unroll
+        for (int n = 0; n < TPT; ++n) {
+            const int t = seg + n * segs;
+            const float x[4] = {kx[n].x, kx[n].y, kx[n].z, kx[n].w};
+            uint32_t q[4];
+            encode(x, mn4, sc4, rc4, q);
+            if (t < G) {
+                reinterpret_cast<uint8_t*>(kcodes)[t * D4 + quad] =
+                    (uint8_t)(q[0] | (q[1] << 2) | (q[2] << 4) | (q[3] << 6));
+                if (a.k_hist)
+                    *reinterpret_cast<float4*>(a.k_hist + (hist_row0 + t) * D + 4 * quad) =
+                        make_float4(decode1(q[0], s.x, m.x), decode1(q[1], s.y, m.y),
+                                    decode1(q[2], s.z, m.z), decode1(q[3], s.w, m.w));
+            }
+        }
+    }
+    lds_barrier();
+
+    uint32_t* const kout = reinterpret_cast<uint32_t*>(a.k_codes + chunk_id * N4);
+    uint32_t* const vout = reinterpret_cast<uint32_t*>(a.v_codes + chunk_id * N4);
+    const int G4 = G / 4;
+    for (int e = tid; e < N4 / 4; e += nthr) {
+        kout[e] = kcodes[e];
+        // value byte 4e + b: channel d, tokens 4j..4j+3
+        int d = 4 * e / G4, j = 4 * e % G4;
+        uint32_t word = 0;
+#pragma unroll
+        for (int b = 0; b < 4; ++b) {
+            const uint32_t w = (vcodes[(d / 4) * G4 + j] >> (2 * (d % 4))) & 0x03030303u;
+            word |= ((w | (w >> 6) | (w >> 12) | (w >> 18)) & 0xffu) << (8 * b);
+            if (++j == G4) { j = 0; ++d; }
+        }
+        vout[e] = word;
+    }
+    for (int e = tid; e < NG * G; e += nthr) {
+        a.v_scale[chunk_id * NG * G + e] = vscl[e];
+        a.v_zero[chunk_id * NG * G + e] = vzro[e];
+    }
+}
+
+template <int TPT>
+void launch_plain2(const FlushArgs& a, int src, int segs, dim3 grid, int threads, size_t lds,
+                   hipStream_t st) {
+    switch (src) {
+        case kSrcBF16: flush_plain_kernel<TPT, kSrcBF16><<<grid, threads, lds, st>>>(a, segs); break;
+        case kSrcF16: flush_plain_kernel<TPT, kSrcF16><<<grid, threads, lds, st>>>(a, segs); break;
+        default: flush_plain_kernel<TPT, kSrcF32><<<grid, threads, lds, st>>>(a, segs); break;
+    }
+}
+
+// flush_plain_kernel where it applies (false: not launched, and flush_kernel
+// takes the call).  Its code stores are dwords, its rows at most one workgroup
+// wide, its tokens per thread at most 8 (K and V take 64 registers then); the
+// caller has checked the 16-byte accesses.  It is ahead at every size it takes
+// (fp32, before -> now: 80 / 16 / 16 213 -> 99 us, 96 / 64 / 32 with 8 tokens per
+// thread 60 -> 31, 256 / 16 / 16 102 -> 64), the smallest prompts being launches.
+bool launch_plain(const FlushArgs& a, int src, dim3 grid, hipStream_t st) {
+    const int lanes = a.Gv / 4, D4 = a.D / 4;
+    if ((lanes & (lanes - 1)) || lanes > 64 || D4 > kFlushBlock ||
+        (uintptr_t)a.k_codes % 4 || (uintptr_t)a.v_codes % 4)
+        return false;
+    const int most = kFlushBlock / D4;
+    const int need = (a.G + most - 1) / most;
+    const int tpt = need <= 1 ? 1 : need <= 2 ? 2 : need <= 4 ? 4 : 8;
+    if (need > tpt) return false;
+    const int segs = (a.G + tpt - 1) / tpt;        // <= most: tpt >= need
+    const int threads = (segs * D4 + 63) / 64 * 64;
+    const int ng = a.D / a.Gv;
+    const size_t lds = (size_t)(2 * segs * a.D + 3 * a.D + 2 * ng * a.G) * sizeof(float) +
+                       (size_t)a.G * a.D / 2;
+    switch (tpt) {
+        case 1: launch_plain2<1>(a, src, segs, grid, threads, lds, st); break;
+        case 2: launch_plain2<2>(a, src, segs, grid, threads, lds, st); break;
+        case 4: launch_plain2<4>(a, src, segs, grid, threads, lds, st); break;
+        default: launch_plain2<8>(a, src, segs, grid, threads, lds, st); break;
+    }
+    return true;
+}
+
 template <int LAYOUT, bool TILE>
 void launch_flush(const FlushArgs& a, int src, dim3 grid, size_t lds, hipStream_t st) {
     switch (src) {
@@ -810,7 +1041,7 @@ extern "C" int kivi_store_flush_chunks(
     if (layout == kLayoutMfma) {
         if (tile) launch_flush<kLayoutMfma, true>(a, new_dtype, grid, lds, st);
         else launch_flush<kLayoutMfma, false>(a, new_dtype, grid, lds, st);
-    } else {
+    } else if (!(tile && new_vec && launch_plain(a, new_dtype, grid, st))) {
         if (tile) launch_flush<kLayoutPlain, true>(a, new_dtype, grid, lds, st);
         else launch_flush<kLayoutPlain, false>(a, new_dtype, grid, lds, st);
     }

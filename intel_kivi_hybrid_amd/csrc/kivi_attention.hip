@@ -751,10 +751,11 @@ size_t workspace_for(int batch, int q_len, int q_heads, int kv_heads, int head_d
 // Attention of q_len query tokens per sequence (q [batch][q_len][q_heads]
 // [head_dim], out likewise) over [packed history ; residual window]; causal:
 // the queries are the window's last q_len tokens and token i sees the window
-// up to itself, else every token sees the whole context.  Tokens are split
-// across launches when q_len * (q_heads / kv_heads) exceeds 8 rows, and the
-// query heads of a kv head in groups of 8 when there are more; each launch
-// streams the store once.
+// up to itself, else every token sees the whole context.  Several tokens of
+// more than 8 rows (q_len * (q_heads / kv_heads)) take the many-row kernels
+// where takes_rows() says so; else tokens are split across launches of 8 rows,
+// and the query heads of a kv head in groups of 8 when there are more; each
+// launch streams the store once.
 int attention_impl(const float* q, int32_t q_len, int32_t causal, const int32_t* kv_start,
                    const uint32_t* hidden, int64_t hidden_stride, const uint8_t* k_codes,
                    const float* k_scale, const float* k_zero, const uint8_t* v_codes,

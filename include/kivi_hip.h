@@ -348,6 +348,30 @@ int kivi_packed_attention_masked(const float* q, int32_t q_len, int32_t causal,
                                  int32_t res_len, float softmax_scale, int32_t num_splits,
                                  void* stream);
 
+/* kivi_packed_attention_masked for queries in the model's own type and layout:
+ * q_dtype and out's type are 0 (f32), 1 (bf16) or 2 (f16), element (b, i, h, d)
+ * of q lies at b*q_stride_b + i*q_stride_t + h*q_stride_h + d (strides in
+ * elements, multiples of 4); out is [batch][q_len][q_heads][head_dim].  Queries
+ * widen exactly, the fp32 result is rounded once to nearest even: the bits are
+ * those of the fp32 call on converted buffers.  Only for q_len > 1 with
+ * q_len * (q_heads / kv_heads) > 8 on a matrix-core store, and 16-byte-aligned
+ * q, out and workspace (else an error, and nothing is launched).  No reference
+ * counterpart. */
+int kivi_packed_attention_typed(const void* q, int32_t q_dtype, int64_t q_stride_b,
+                                int64_t q_stride_t, int64_t q_stride_h, int32_t q_len,
+                                int32_t causal, const int32_t* kv_start, const uint32_t* hidden,
+                                int64_t hidden_stride, const uint8_t* k_codes,
+                                const float* k_scale, const float* k_zero,
+                                const uint8_t* v_codes, const float* v_scale,
+                                const float* v_zero, const void* k_res, const void* v_res,
+                                int32_t res_dtype, void* out, void* workspace,
+                                size_t workspace_bytes, int32_t batch, int32_t q_heads,
+                                int32_t kv_heads, int32_t head_dim, int32_t group_size_k,
+                                int32_t group_size_v, int32_t chunk_capacity,
+                                int32_t num_chunks, int32_t res_capacity, int32_t res_start,
+                                int32_t res_len, float softmax_scale, int32_t num_splits,
+                                void* stream);
+
 /* kivi_packed_decode_attention with this step's new token appended in the
  * same launch: the window (res_start, res_len) already counts the new token
  * as its last (index res_len - 1, ring slot (res_start + res_len - 1) %

@@ -640,3 +640,60 @@ def packed_attention(q, store, causal=True, softmax_scale=None, out=None, num_sp
             store.res_start, store.res_len, scale, int(num_splits),
             ctypes.c_void_p(_stream_of(q.device))), "packed_attention")
     return out
+
+
+_IO_DTYPES = {torch.float32: 0, torch.bfloat16: 1, torch.float16: 2}
+
+
+def takes_typed_queries(q, store):
+    """Whether :func:`packed_attention_typed` takes these queries: more than 8
+    query rows per kv head of several tokens on a matrix-core store, on the
+    store's device, channels contiguous and aligned for 4-element loads."""
+    return (q.dim() == 4 and q.shape[2] > 1 and q.dtype in _IO_DTYPES and q.is_cuda
+            and store.code_layout != 0 and q.device == store.device
+            and q.shape[0] == store.B and q.shape[3] == store.D and q.numel() > 0
+            and q.shape[1] % store.H == 0 and q.shape[2] * (q.shape[1] // store.H) > 8
+            and q.stride(3) == 1 and q.data_ptr() % 16 == 0
+            and not any(s % 4 for s in q.stride()[:3]))
+
+
+def packed_attention_typed(q, store, softmax_scale=None, kv_start=None, hidden=None):
+    """:func:`packed_attention` (causal) of queries ``q [B, Hq, L, D]`` in the
+    model's own type and strides, returning ``[B, L, Hq, D]`` of that type: the
+    bits of the fp32 call on converted tensors, without the conversions.  Only
+    where :func:`takes_typed_queries`.  ``kv_start`` and ``hidden``: tensors on
+    the store's device."""
+    _check(takes_typed_queries(q, store), "these queries need packed_attention")
+    B, Hq, L, D = q.shape
+    store._commit()
+    _check(L <= store.res_len, "causal attention of ", L, " query tokens needs them in "
+           "the residual window (", store.res_len, " tokens)")
+    if kv_start is not None:
+        _check(kv_start.dtype == torch.int32 and kv_start.numel() == B and
+               kv_start.is_contiguous() and kv_start.device == q.device,
+               "kv_start must be a contiguous int32 tensor of ", B, " positions")
+    if hidden is not None:
+        W = (store.quantized_tokens + store.res_len + 31) // 32
+        _check(hidden.dtype == torch.int32 and hidden.dim() == 2 and hidden.shape[0] == B and
+               hidden.shape[1] >= W and hidden.stride(1) == 1 and hidden.device == q.device,
+               "hidden must be an int32 [B, >=", W, "] tensor with contiguous rows on the "
+               "query's device")
+    out = torch.empty(B, L, Hq, D, dtype=q.dtype, device=q.device)
+    need = int(_lib.kivi_packed_attention_workspace_size(
+        B, L, Hq, store.H, D, store.G, store.Gv, store.n_chunks, store.res_len, 0))
+    ws = _workspace(q.device, need)
+    with on_device(q.device):
+        _native.check(_lib.kivi_packed_attention_typed(
+            q.data_ptr(), _IO_DTYPES[q.dtype], q.stride(0), q.stride(2), q.stride(1), L, 1,
+            0 if kv_start is None else kv_start.data_ptr(),
+            0 if hidden is None else hidden.data_ptr(),
+            0 if hidden is None else hidden.stride(0),
+            store.k_codes.data_ptr(), store.k_scale.data_ptr(), store.k_zero.data_ptr(),
+            store.v_codes.data_ptr(), store.v_scale.data_ptr(), store.v_zero.data_ptr(),
+            store.k_res.data_ptr(), store.v_res.data_ptr(), store.res_dtype_code, out.data_ptr(),
+            0 if ws is None else ws.data_ptr(), 0 if ws is None else ws.numel(),
+            B, Hq, store.H, D, store.G, store.Gv, store.capacity, store.n_chunks, store.R,
+            store.res_start, store.res_len,
+            D ** -0.5 if softmax_scale is None else float(softmax_scale), 0,
+            _stream_of(q.device)), "packed_attention")
+    return out

@@ -222,6 +222,13 @@ class KiviPackedLayer(CacheLayerMixin):
         update."""
         st = self.store
         B, Hq, L, D = query.shape
+        if (L > 1 and isinstance(st, PackedKVStore) and _C.takes_typed_queries(query, st)
+                and (kv_start is None
+                     or (torch.is_tensor(kv_start) and kv_start.device == query.device))):
+            o = _C.packed_attention_typed(query, st, softmax_scale=scaling, kv_start=kv_start,
+                                          hidden=hidden)
+            self._awaiting_attention = False
+            return o
         # (each decode step calls this once per layer: no-op conversions are
         # skipped, since each costs about a microsecond of host time)
         native = query.dtype is torch.float32 and query.get_device() == st.device.index

@@ -748,6 +748,12 @@ size_t workspace_for(int batch, int q_len, int q_heads, int kv_heads, int head_d
                (size_t)batch * kv_heads * rows * p.n_splits * (head_dim + 2) * sizeof(float));
 }
 
+// Type of queries and output, and the queries' strides in elements.
+struct QueryForm {
+    int dtype;
+    int64_t sb, st, sh;
+};
+
 // Attention of q_len query tokens per sequence (q [batch][q_len][q_heads]
 // [head_dim], out likewise) over [packed history ; residual window]; causal:
 // the queries are the window's last q_len tokens and token i sees the window
@@ -766,7 +772,7 @@ int attention_impl(const float* q, int32_t q_len, int32_t causal, const int32_t*
                    int32_t chunk_capacity, int32_t num_chunks, int32_t res_capacity,
                    int32_t res_start, int32_t res_len, float softmax_scale, int32_t num_splits,
                    const void* k_new, const void* v_new, int64_t new_sb, int64_t new_sh,
-                   void* stream) {
+                   void* stream, const QueryForm* form = nullptr) {
     if (!q || !out)
         return set_error(kErrInvalidArgument, "null q/out pointer");
     if (batch <= 0)
@@ -820,8 +826,23 @@ int attention_impl(const float* q, int32_t q_len, int32_t causal, const int32_t*
     }
     // (its loads and stores of queries, outputs and partials are 16 bytes wide;
     // buffers off that alignment take the decode kernel's launches)
-    if (takes_rows(q_len, hg, head_dim, group_size_k, group_size_v) &&
-        ((uintptr_t)q | (uintptr_t)out | (uintptr_t)workspace) % 16 == 0) {
+    const bool takes = takes_rows(q_len, hg, head_dim, group_size_k, group_size_v);
+    if (form) {
+        if (form->dtype < kSrcF32 || form->dtype > kSrcF16)
+            return set_error(kErrInvalidArgument, "q_dtype %d is not 0 (f32), 1 (bf16) or 2 (f16)",
+                             form->dtype);
+        if (!takes)
+            return set_error(kErrUnsupported,
+                             "typed queries need more than 8 rows per kv head of several tokens "
+                             "on a matrix-core store");
+        if (((uintptr_t)q | (uintptr_t)out | (uintptr_t)workspace) % 16 || form->sb % 4 ||
+            form->st % 4 || form->sh % 4)
+            return set_error(kErrInvalidArgument,
+                             "typed queries need 16-byte-aligned buffers and strides of whole "
+                             "4 elements");
+    }
+    if (takes && ((uintptr_t)q | (uintptr_t)out | (uintptr_t)workspace) % 16 == 0) {
+        const int64_t sh = head_dim, stok = sh * q_heads, sb = stok * q_len;
         const int rows = q_len * hg;
         const RowsPlan r = rows_plan(batch, kv_heads, rows, head_dim, group_size_k, num_chunks,
                                      res_len, num_splits);
@@ -835,7 +856,8 @@ int attention_impl(const float* q, int32_t q_len, int32_t causal, const int32_t*
                      res_capacity, res_start, res_len, res_dtype, q_len, hg, rows,
                      causal ? res_len - (q_len - 1) : res_len, r.block_rows, r.row_blocks,
                      r.n_units, r.n_splits, r.weight_per_split, softmax_scale * kLog2e, kv_start,
-                     hidden, hidden_stride};
+                     hidden, hidden_stride, form ? form->dtype : kSrcF32, form ? form->sb : sb,
+                     form ? form->st : stok, form ? form->sh : sh};
         return launch_attention_rows(L, (hipStream_t)stream);
     }
     const bool empty_ok = chunk_capacity >= 1 && k_codes && k_scale && k_zero && v_codes &&
@@ -999,6 +1021,29 @@ int kivi_packed_attention_masked(const float* q, int32_t q_len, int32_t causal,
                           group_size_k, group_size_v, chunk_capacity, num_chunks, res_capacity,
                           res_start, res_len, softmax_scale, num_splits, nullptr, nullptr, 0, 0,
                           stream);
+}
+
+int kivi_packed_attention_typed(const void* q, int32_t q_dtype, int64_t q_stride_b,
+                                int64_t q_stride_t, int64_t q_stride_h, int32_t q_len,
+                                int32_t causal, const int32_t* kv_start, const uint32_t* hidden,
+                                int64_t hidden_stride, const uint8_t* k_codes,
+                                const float* k_scale, const float* k_zero,
+                                const uint8_t* v_codes, const float* v_scale,
+                                const float* v_zero, const void* k_res, const void* v_res,
+                                int32_t res_dtype, void* out, void* workspace,
+                                size_t workspace_bytes, int32_t batch, int32_t q_heads,
+                                int32_t kv_heads, int32_t head_dim, int32_t group_size_k,
+                                int32_t group_size_v, int32_t chunk_capacity,
+                                int32_t num_chunks, int32_t res_capacity, int32_t res_start,
+                                int32_t res_len, float softmax_scale, int32_t num_splits,
+                                void* stream) {
+    const QueryForm form{q_dtype, q_stride_b, q_stride_t, q_stride_h};
+    return attention_impl((const float*)q, q_len, causal, kv_start, hidden, hidden_stride,
+                          k_codes, k_scale, k_zero, v_codes, v_scale, v_zero, k_res, v_res,
+                          res_dtype, (float*)out, workspace, workspace_bytes, batch, q_heads,
+                          kv_heads, head_dim, group_size_k, group_size_v, chunk_capacity,
+                          num_chunks, res_capacity, res_start, res_len, softmax_scale,
+                          num_splits, nullptr, nullptr, 0, 0, stream, &form);
 }
 
 int kivi_packed_decode_attention(const float* q, const uint8_t* k_codes, const float* k_scale,

@@ -117,7 +117,7 @@ int plain_attention_groups_per_cu(int rows, int D, int G, int Gv);
 // token i sees every packed token and the first min(res_len, vis0 + i) of the
 // window.
 struct RowsLaunch {
-    const float* q;          // [B, q_len, Hq, D]
+    const void* q;           // element (b, i, h, d) at b q_sb + i q_st + h q_sh + d, of type io_dt
     const uint8_t* k_codes;  // as AttnLaunch
     const float* k_scale;
     const float* k_zero;
@@ -126,7 +126,7 @@ struct RowsLaunch {
     const float* v_zero;
     const void* k_res;
     const void* v_res;
-    float* out;              // [B, q_len, Hq, D]
+    void* out;               // [B, q_len, Hq, D] of type io_dt
     float* part_o;           // [B, Hkv, rows, n_splits, D] (n_splits > 1 only)
     float* part_ml;          // [B, Hkv, rows, n_splits, 2]
     int B, Hq, Hkv, D, G, Gv, Cmax, n_chunks, Rcap, res_start, res_len, res_dt;
@@ -136,6 +136,8 @@ struct RowsLaunch {
     const int32_t* kv_start;
     const uint32_t* hidden;
     int64_t hidden_stride;
+    int io_dt;               // kSrc* of q and out
+    int64_t q_sb, q_st, q_sh;
 };
 struct RowsPlan {
     int block_rows, row_blocks, n_units, n_splits, weight_per_split;

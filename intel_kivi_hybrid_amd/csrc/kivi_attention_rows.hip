@@ -71,8 +71,47 @@ __device__ __forceinline__ float row4_sum(float v) {
     return v + __shfl_xor(v, 32);
 }
 
-__device__ __forceinline__ int64_t row_offset(const RowsLaunch& a, int b, int kvh, int r) {
+__device__ __forceinline__ int64_t out_offset(const RowsLaunch& a, int b, int kvh, int r) {
     return (((int64_t)b * a.q_len + r / a.hg) * a.Hq + (int64_t)kvh * a.hg + r % a.hg) * a.D;
+}
+__device__ __forceinline__ int64_t query_offset(const RowsLaunch& a, int b, int kvh, int r) {
+    return b * a.q_sb + r / a.hg * a.q_st + ((int64_t)kvh * a.hg + r % a.hg) * a.q_sh;
+}
+
+// Queries and outputs are in the caller's type, read and written here: a bf16
+// model's step otherwise pays up to three more launches (q widened, q made
+// token-major, the output rounded).  A layer's step, 32/8 heads, head_dim 128:
+// 5 query tokens, 4K context, B=8 51.2 -> 44.0 us; 512 tokens, 8.1K, B=1
+// 227.9 -> 217.5 us.
+// f(load) with load(i): elements i .. i + 3 of the queries, widened exactly.
+// (one branch around all loads: a branch per load would wait for each)
+template <class F>
+__device__ __forceinline__ void with_query(const RowsLaunch& a, F f) {
+    if (a.io_dt == kSrcF32) {
+        f([&](int64_t i) {
+            return *reinterpret_cast<const float4*>(static_cast<const float*>(a.q) + i);
+        });
+    } else {
+        const uint32_t half_mask = a.io_dt == kSrcF16 ? ~0u : 0u;
+        f([&, half_mask](int64_t i) { return load4_16(a.q, i, half_mask); });
+    }
+}
+__device__ __forceinline__ uint16_t round16(float x, int dt) {
+    return dt == kSrcBF16 ? __builtin_bit_cast(uint16_t, (__bf16)x)
+                          : __builtin_bit_cast(uint16_t, (_Float16)x);
+}
+__device__ __forceinline__ void store4_as(void* p, int64_t i, float4 x, int dt) {
+    if (dt == kSrcF32) {
+        *reinterpret_cast<float4*>(static_cast<float*>(p) + i) = x;
+    } else {
+        const uint32_t lo = round16(x.x, dt) | (uint32_t)round16(x.y, dt) << 16;
+        const uint32_t hi = round16(x.z, dt) | (uint32_t)round16(x.w, dt) << 16;
+        *reinterpret_cast<uint2*>(static_cast<uint16_t*>(p) + i) = make_uint2(lo, hi);
+    }
+}
+__device__ __forceinline__ void store1_as(void* p, int64_t i, float x, int dt) {
+    if (dt == kSrcF32) static_cast<float*>(p)[i] = x;
+    else static_cast<uint16_t*>(p)[i] = round16(x, dt);
 }
 
 // Piece operands of 8 fp32 values.
@@ -159,16 +198,16 @@ template <int D, int RT>
 __device__ __forceinline__ int query_kind(const RowsLaunch& a, int row0, int b, int kvh) {
     const int lane = threadIdx.x % kWave;
     uint32_t low = 0, top = 0;
+    with_query(a, [&](auto load) {
 #pragma unroll
     for (int rt = 0; rt < RT; ++rt) {
         const int r = min(row0 + 16 * rt + lane % 16, a.rows - 1);
-        const float4* q = reinterpret_cast<const float4*>(a.q + row_offset(a, b, kvh, r) +
-                                                          8 * (lane / 16));
+        const int64_t q = query_offset(a, b, kvh, r) + 8 * (lane / 16);
 #pragma unroll
         for (int ks = 0; ks < D / 32; ++ks) {
 #pragma unroll
             for (int j = 0; j < 2; ++j) {
-                const float4 x = q[8 * ks + j];
+                const float4 x = load(q + 32 * ks + 4 * j);
                 const uint32_t w[4] = {__float_as_uint(x.x), __float_as_uint(x.y),
                                        __float_as_uint(x.z), __float_as_uint(x.w)};
 #pragma unroll
@@ -179,6 +218,7 @@ __device__ __forceinline__ int query_kind(const RowsLaunch& a, int row0, int b, 
             }
         }
     }
+    });
     return (__builtin_amdgcn_ballot_w64((low & 0xffffu) != 0) != 0 ? kWide : 0) |
            (__builtin_amdgcn_ballot_w64(top >= kNotFinite) != 0 ? kSlow : 0);
 }
@@ -204,11 +244,19 @@ struct Rows {
         for (int rt = 0; rt < RT; ++rt) {
             const int r = min(row0 + 16 * rt + col, a.rows - 1);
             vis[rt] = min(a.vis0 + r / a.hg, a.res_len);
-            const float4* q = reinterpret_cast<const float4*>(a.q + row_offset(a, b, kvh, r) +
-                                                              8 * gq);
+            m[rt] = -INFINITY;
+            l[rt] = 0.f;
+#pragma unroll
+            for (int nb = 0; nb < NBV; ++nb) O[rt][nb] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+        }
+        with_query(a, [&](auto load) {
+#pragma unroll
+        for (int rt = 0; rt < RT; ++rt) {
+            const int r = min(row0 + 16 * rt + col, a.rows - 1);
+            const int64_t q = query_offset(a, b, kvh, r) + 8 * gq;
 #pragma unroll
             for (int ks = 0; ks < KS; ++ks) {
-                const float4 x0 = q[8 * ks], x1 = q[8 * ks + 1];
+                const float4 x0 = load(q + 32 * ks), x1 = load(q + 32 * ks + 4);
                 const float x[8] = {x0.x * sign, x0.y * sign, x0.z * sign, x0.w * sign,
                                     x1.x * sign, x1.y * sign, x1.z * sign, x1.w * sign};
                 u32x4_t p[3];
@@ -216,11 +264,8 @@ struct Rows {
 #pragma unroll
                 for (int i = 0; i < NQ; ++i) qf[rt][ks][i] = __builtin_bit_cast(bf16x8_t, p[i]);
             }
-            m[rt] = -INFINITY;
-            l[rt] = 0.f;
-#pragma unroll
-            for (int nb = 0; nb < NBV; ++nb) O[rt][nb] = f32x4_t{0.f, 0.f, 0.f, 0.f};
         }
+        });
     }
 
     // s[rt] += key tile (kKP pieces) x query at k-step ks
@@ -318,18 +363,24 @@ struct Rows {
 // The unnormalised state of row r -> its partial, or the output when the
 // context has one split (a row that sees no position gives 0).
 struct RowDst {
-    float* p;
+    void* p;
+    int64_t at;
+    int dt;
     float f;
+    __device__ __forceinline__ void store4(int d, float x, float y, float z, float w) const {
+        store4_as(p, at + d, make_float4(x * f, y * f, z * f, w * f), dt);
+    }
 };
 __device__ __forceinline__ RowDst row_dst(const RowsLaunch& a, int b, int kvh, int64_t bh, int r,
                                           int split, float m, float l, bool first) {
-    if (a.n_splits == 1) return {a.out + row_offset(a, b, kvh, r), l > 0.f || l != l ? 1.f / l : 0.f};
+    if (a.n_splits == 1)
+        return {a.out, out_offset(a, b, kvh, r), a.io_dt, l > 0.f || l != l ? 1.f / l : 0.f};
     const int64_t row = (bh * a.rows + r) * a.n_splits + split;
     if (first) {
         a.part_ml[row * 2] = m;
         a.part_ml[row * 2 + 1] = l;
     }
-    return {a.part_o + row * a.D, 1.f};
+    return {a.part_o, row * a.D, kSrcF32, 1.f};
 }
 
 // A workgroup's range of units, and which of a unit's tokens are hidden.
@@ -381,7 +432,10 @@ __device__ __forceinline__ void slow_rows(const RowsLaunch& a, const Range& rg, 
     const int np = a.G * D / 1024, ng = D / a.Gv;
     for (int r = row0 + (int)threadIdx.x / kWave; r < min(row0 + n, a.rows); r += waves) {
         const int vis = min(a.vis0 + r / a.hg, a.res_len);
-        const gptr q = (gptr)(a.q + row_offset(a, b, kvh, r));
+        float q[C];
+#pragma unroll
+        for (int c = 0; c < C; ++c)
+            q[c] = load1_dt(a.q, query_offset(a, b, kvh, r) + lane + kWave * c, a.io_dt);
         float o[C] = {}, m = -INFINITY, l = 0.f;
 #pragma unroll 1
         for (int u = rg.begin; u < rg.end; ++u) {
@@ -420,7 +474,7 @@ __device__ __forceinline__ void slow_rows(const RowsLaunch& a, const Range& rg, 
                         v[c] = fmaf((float)((vw >> mfma_code_bit(vtile % 2, tt % 8)) & 3u),
                                     a.v_scale[vm], a.v_zero[vm]);
                     }
-                    part = fmaf(gload<float>(q, 4 * d), kx, part);
+                    part = fmaf(q[c], kx, part);
                 }
 #pragma unroll
                 for (int x = 1; x < kWave; x *= 2) part += __shfl_xor(part, x);
@@ -441,7 +495,7 @@ __device__ __forceinline__ void slow_rows(const RowsLaunch& a, const Range& rg, 
         }
         const RowDst dst = row_dst(a, b, kvh, bh, r, split, m, l, lane == 0);
 #pragma unroll
-        for (int c = 0; c < C; ++c) dst.p[lane + kWave * c] = o[c] * dst.f;
+        for (int c = 0; c < C; ++c) store1_as(dst.p, dst.at + lane + kWave * c, o[c] * dst.f, dst.dt);
     }
 }
 
@@ -799,8 +853,7 @@ __device__ bool walk_shared(const RowsLaunch& a, unsigned char* smem, const Rang
 #pragma unroll
         for (int nb = 0; nb < S::NBV; ++nb) {
             const f32x4_t o = rows.O[rt][nb];
-            *reinterpret_cast<float4*>(d.p + 16 * nb + 4 * gq) =
-                make_float4(o[0] * d.f, o[1] * d.f, o[2] * d.f, o[3] * d.f);
+            d.store4(16 * nb + 4 * gq, o[0], o[1], o[2], o[3]);
         }
     }
     return bad;
@@ -1135,8 +1188,7 @@ __device__ bool walk_wave(const RowsLaunch& a, unsigned char* smem, const Range&
             acc.w = fmaf(f, o.w, acc.w);
         }
         const RowDst dst = row_dst(a, b, kvh, bh, r, split, M, L, d == 0);
-        *reinterpret_cast<float4*>(dst.p + d) =
-            make_float4(acc.x * dst.f, acc.y * dst.f, acc.z * dst.f, acc.w * dst.f);
+        dst.store4(d, acc.x, acc.y, acc.z, acc.w);
     }
     __syncthreads();                                         // (another walk may follow)
     return top.bad(half_mask);
@@ -1178,7 +1230,7 @@ __global__ __launch_bounds__(256) void attn_rows_merge_kernel(RowsLaunch a) {
     float M = -INFINITY;
     for (int s = 0; s < S; ++s) M = fmaxf(M, ml[2 * s]);
     const int64_t bh = row / a.rows;
-    float* out = a.out + row_offset(a, (int)(bh / a.Hkv), (int)(bh % a.Hkv), (int)(row % a.rows));
+    const int64_t out = out_offset(a, (int)(bh / a.Hkv), (int)(bh % a.Hkv), (int)(row % a.rows));
     const float* po = a.part_o + row * S * D;
     for (int d = 4 * lane; d < D; d += 4 * kWave) {
         float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
@@ -1195,8 +1247,8 @@ __global__ __launch_bounds__(256) void attn_rows_merge_kernel(RowsLaunch a) {
             acc.w = fmaf(f, o.w, acc.w);
         }
         const float f = L > 0.f || L != L ? 1.f / L : 0.f;      // 0: every position hidden
-        *reinterpret_cast<float4*>(out + d) =
-            make_float4(acc.x * f, acc.y * f, acc.z * f, acc.w * f);
+        store4_as(a.out, out + d, make_float4(acc.x * f, acc.y * f, acc.z * f, acc.w * f),
+                  a.io_dt);
     }
 }
 

@@ -487,7 +487,9 @@ __device__ __forceinline__ void slow_rows(const RowsLaunch& a, const Range& rg, 
 #pragma unroll
                     for (int c = 0; c < C; ++c) o[c] *= f;
                 }
-                const float w = off ? 0.f : exp2_fast(s - m);
+                // (by the score and not by `off`: a seen token's score can be -inf
+                // while the maximum still is)
+                const float w = s == -INFINITY ? 0.f : exp2_fast(s - m);
                 l += w;
 #pragma unroll
                 for (int c = 0; c < C; ++c) o[c] = fmaf(w, v[c], o[c]);

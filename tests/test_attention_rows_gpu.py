@@ -142,3 +142,34 @@ def test_infinite_window_elements(hip_device, ring, L):
     assert bool(torch.isinf(out[..., 9]).all())
     rest = torch.cat([out[..., :9], out[..., 10:]], -1)
     assert bool(torch.isfinite(rest).all())
+
+
+@pytest.mark.parametrize("Hq,D,G,Gv,T,L,splits,ring", [
+    (4, 128, 32, 32, 40, 5, 0, "f32"),        # the window alone, 20 rows
+    (4, 128, 32, 32, 40, 40, 0, "bf16"),      # the same, 160 rows
+    (3, 64, 64, 64, 333, 7, 3, "f16"),        # G = 64, three splits
+    (4, 64, 32, 64, 333, 30, 2, "f32"),       # 120 rows
+    (4, 128, 64, 128, 600, 40, 2, "f32"),     # one value group
+    (4, 256, 32, 256, 400, 3, 2, "f32"),      # head_dim 256, 12 rows
+    (4, 256, 64, 128, 400, 30, 2, "bf16"),    # 120 rows
+])
+def test_infinite_key_comes_first(hip_device, Hq, D, G, Gv, T, L, splits, ring):
+    """A token whose score is -inf takes no weight also where it is the first
+    that a row sees: at the start of the context, after left padding, behind
+    holes."""
+    print(f"[rows] first -inf: D={D} G={G} Gv={Gv} T={T} L={L} {splits} {ring}", flush=True)
+    st, k, v = _store(hip_device, 1, 1, D, G, Gv, 64, T, L, ring)
+    q = torch.rand(1, Hq, L, D, generator=torch.Generator().manual_seed(2)) + 0.5
+    q0 = st.quantized_tokens
+    j = 3 if q0 else 0                          # the window token, and its position
+    st.k_res[0, 0, (st.res_start + j) % st.R, 7] = -float("inf")
+    pos, total = q0 + j, q0 + st.res_len
+    vis = torch.ones(1, total, dtype=torch.bool)
+    vis[0, pos] = False
+    out = st.attention(q.cuda(), num_splits=splits)
+    _check(out, q, st, k, v, G, Gv, visible=vis.numpy())
+    out = st.attention(q.cuda(), num_splits=splits, kv_start=[pos])
+    _check(out, q, st, k, v, G, Gv, kv_start=np.array([pos + 1]))
+    holes = torch.arange(total)[None, :] >= pos
+    out = st.attention(q.cuda(), num_splits=splits, key_mask=holes)
+    _check(out, q, st, k, v, G, Gv, visible=(holes & vis).numpy())

@@ -27,6 +27,13 @@
 //   (~2^-17 per weight, averaged over the context), window values six of
 //   three.  The softmax is online in fp32, in the log2 domain; its maximum
 //   moves only when exceeded by more than 8 (weights <= 256).
+// * Elements that are not finite as bf16 have no pieces (inf - inf): every sum
+//   that they enter comes out NaN.  A workgroup whose window sums come out NaN
+//   walks its range again with the window in plain fp32 (Rows::plain_unit):
+//   an infinite value makes its channel infinite, a score of -inf gives its
+//   token no weight, and a token that a row does not see does not touch it.
+//   Packed chunks keep the same walk: non-finite factors make the rows that
+//   see them NaN.
 //
 // Two kernels (few_rows(): which rows take which):
 // * attn_rows_shared_kernel (many rows): eight waves with up to 32 rows each
@@ -38,6 +45,7 @@
 // kernel's launches before, this file's after): 512 query tokens over 8.1K
 // packed tokens, B=1: 256 launches, 4.84 ms -> 229 us; 5 tokens over 4K, B=8: 3
 // launches, 85.6 -> 52.7 us.
+#include <float.h>
 #include <math.h>
 
 #include "kivi_attention.hpp"
@@ -53,8 +61,6 @@ constexpr int kWindowWeight = 2;            // cost of a window unit in packed u
 constexpr int kKP = 3;                      // key pieces
 constexpr int kVPWin = 3, kVPChunk = 2;     // value pieces: window, packed chunks
 constexpr int kTile = kWave * 16;           // bytes of one operand tile
-
-constexpr uint32_t kNotFinite = 0x7f7f8000u;  // |x| from here on rounds to infinity as bf16
 
 template <bool V>
 struct BoolC {
@@ -108,10 +114,6 @@ __device__ __forceinline__ void store4_as(void* p, int64_t i, float4 x, int dt) 
         const uint32_t hi = round16(x.z, dt) | (uint32_t)round16(x.w, dt) << 16;
         *reinterpret_cast<uint2*>(static_cast<uint16_t*>(p) + i) = make_uint2(lo, hi);
     }
-}
-__device__ __forceinline__ void store1_as(void* p, int64_t i, float x, int dt) {
-    if (dt == kSrcF32) static_cast<float*>(p)[i] = x;
-    else static_cast<uint16_t*>(p)[i] = round16(x, dt);
 }
 
 // Piece operands of 8 fp32 values.
@@ -170,34 +172,12 @@ __device__ __forceinline__ int window_slot(const RowsLaunch& a, int t) {
     return s >= a.Rcap ? s - a.Rcap : s;
 }
 
-// The largest magnitudes of ring dwords (R16: of each half), and whether one of
-// them is not finite as bf16.
-typedef uint16_t u16x2_t __attribute__((ext_vector_type(2)));
-template <bool R16>
-struct RingTop {
-    uint32_t top = 0;
-    __device__ __forceinline__ void add(uint32_t d) {
-        if constexpr (R16)
-            top = __builtin_bit_cast(uint32_t, __builtin_elementwise_max(
-                      __builtin_bit_cast(u16x2_t, top),
-                      __builtin_bit_cast(u16x2_t, d & 0x7fff7fffu)));
-        else
-            top = max(top, d & 0x7fffffffu);
-    }
-    __device__ __forceinline__ bool bad(uint32_t half_mask) const {
-        if constexpr (!R16) return top >= kNotFinite;
-        const uint32_t lim = half_mask ? 0x7c00u : 0x7f80u;
-        return (top & 0xffffu) >= lim || (top >> 16) >= lim;
-    }
-};
-
-// What the wave's query values of rows row0 + 16 rt + l % 16 need: kWide if
-// some are not bf16 (three pieces), kSlow if some are not finite as bf16.
-constexpr int kWide = 1, kSlow = 2;
+// Whether some of the wave's query values of rows row0 + 16 rt + l % 16 are not
+// bf16 (they take three pieces).
 template <int D, int RT>
-__device__ __forceinline__ int query_kind(const RowsLaunch& a, int row0, int b, int kvh) {
+__device__ __forceinline__ bool wide_queries(const RowsLaunch& a, int row0, int b, int kvh) {
     const int lane = threadIdx.x % kWave;
-    uint32_t low = 0, top = 0;
+    uint32_t low = 0;
     with_query(a, [&](auto load) {
 #pragma unroll
     for (int rt = 0; rt < RT; ++rt) {
@@ -208,19 +188,13 @@ __device__ __forceinline__ int query_kind(const RowsLaunch& a, int row0, int b, 
 #pragma unroll
             for (int j = 0; j < 2; ++j) {
                 const float4 x = load(q + 32 * ks + 4 * j);
-                const uint32_t w[4] = {__float_as_uint(x.x), __float_as_uint(x.y),
-                                       __float_as_uint(x.z), __float_as_uint(x.w)};
-#pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    low |= w[i];
-                    top = max(top, w[i] & 0x7fffffffu);
-                }
+                low |= __float_as_uint(x.x) | __float_as_uint(x.y) | __float_as_uint(x.z) |
+                       __float_as_uint(x.w);
             }
         }
     }
     });
-    return (__builtin_amdgcn_ballot_w64((low & 0xffffu) != 0) != 0 ? kWide : 0) |
-           (__builtin_amdgcn_ballot_w64(top >= kNotFinite) != 0 ? kSlow : 0);
+    return __builtin_amdgcn_ballot_w64((low & 0xffffu) != 0) != 0;
 }
 
 // A wave's RT tiles of 16 query rows: operands, softmax state and output.
@@ -233,6 +207,7 @@ struct Rows {
     int vis[RT];                    // window tokens the lane's row sees
     float qs;                       // |softmax scale * log2 e| (its sign is in the query)
     SplitConsts spc;
+    bool bad = false;               // a window sum of this lane came out NaN
 
     // rows row0 .. (those past the end repeat the last; they are not stored)
     __device__ __forceinline__ void init(const RowsLaunch& a, int row0, int b, int kvh) {
@@ -244,7 +219,9 @@ struct Rows {
         for (int rt = 0; rt < RT; ++rt) {
             const int r = min(row0 + 16 * rt + col, a.rows - 1);
             vis[rt] = min(a.vis0 + r / a.hg, a.res_len);
-            m[rt] = -INFINITY;
+            // (the lowest finite value: a score of -inf then takes no weight
+            // also where it comes first, and any finite one moves it)
+            m[rt] = -FLT_MAX;
             l[rt] = 0.f;
 #pragma unroll
             for (int nb = 0; nb < NBV; ++nb) O[rt][nb] = f32x4_t{0.f, 0.f, 0.f, 0.f};
@@ -306,6 +283,10 @@ struct Rows {
 #pragma unroll
                 for (int i = 0; i < 8; ++i) x[i] = (off >> i) & 1u ? -INFINITY : x[i];
             }
+            if (WIN) {
+#pragma unroll
+                for (int i = 0; i < 8; ++i) bad |= x[i] != x[i];
+            }
             float top = x[0];
 #pragma unroll
             for (int i = 1; i < 8; ++i) top = fmaxf(top, x[i]);
@@ -323,7 +304,7 @@ struct Rows {
             float sum = 0.f;
 #pragma unroll
             for (int i = 0; i < 8; ++i) p[rt][i] = exp2_fast(fmaf(x[i], qs, -m[rt]));
-            if (WIN || hid) {                  // (0 also while the maximum is -inf)
+            if (WIN || hid) {                  // (0 also while the maximum is the lowest)
 #pragma unroll
                 for (int i = 0; i < 8; ++i) p[rt][i] = (off >> i) & 1u ? 0.f : p[rt][i];
             }
@@ -356,7 +337,77 @@ struct Rows {
         for (int rt = 0; rt < RT; ++rt) o[rt] = WIN ? f32x4_t{0.f, 0.f, 0.f, 0.f} : O[rt][nb];
         mul_pieces<VP, VP, RT>(o, vf, [&](int rt, int j) { return pf[rt][j]; });
 #pragma unroll
-        for (int rt = 0; rt < RT; ++rt) O[rt][nb] = WIN ? O[rt][nb] + o[rt] : o[rt];
+        for (int rt = 0; rt < RT; ++rt) {
+            O[rt][nb] = WIN ? O[rt][nb] + o[rt] : o[rt];
+            if (WIN) {
+#pragma unroll
+                for (int i = 0; i < 4; ++i) bad |= o[rt][i] != o[rt][i];
+            }
+        }
+    }
+
+    // A window unit (tokens t0 ..) in plain fp32 straight from the ring: dot
+    // products with a quarter of the channels per lane, four lanes per row, then
+    // the lane's channels' weighted sums over the tokens that the row sees.
+    template <bool R16>
+    __device__ __forceinline__ void plain_unit(const RowsLaunch& a, int64_t bh, int b, int kvh,
+                                               int row0, uint32_t hid, int t0) {
+        static_assert(RT == 1, "a row tile at a time");
+        const int lane = threadIdx.x % kWave, col = lane % 16, gq = lane / 16;
+        const float sign = a.qscale < 0.f ? -1.f : 1.f;
+        const uint32_t half_mask = a.res_dt == kSrcF16 ? ~0u : 0u;
+        auto ring4 = [&](const void* p, int64_t i) {
+            if constexpr (R16) return load4_16(p, i, half_mask);
+            else return load4_vec<kSrcF32>(p, i);
+        };
+        float4 q[D / 16];
+        with_query(a, [&](auto load) {
+            const int64_t at = query_offset(a, b, kvh, min(row0 + col, a.rows - 1)) + 4 * gq;
+#pragma unroll
+            for (int j = 0; j < D / 16; ++j) q[j] = load(at + 16 * j);
+        });
+        f32x4_t s[2][RT];
+#pragma unroll 2
+        for (int t = 0; t < kUnit; ++t) {
+            const int64_t k = (bh * a.Rcap + window_slot(a, t0 + t)) * D + 4 * gq;
+            float4 y[D / 16];
+#pragma unroll
+            for (int j = 0; j < D / 16; ++j) y[j] = ring4(a.k_res, k + 16 * j);
+            float sum = 0.f;
+#pragma unroll
+            for (int j = 0; j < D / 16; ++j) {
+                sum = fmaf(q[j].x, y[j].x, sum);
+                sum = fmaf(q[j].y, y[j].y, sum);
+                sum = fmaf(q[j].z, y[j].z, sum);
+                sum = fmaf(q[j].w, y[j].w, sum);
+            }
+            sum = row4_sum(sum) * sign;
+#pragma unroll
+            for (int i = 0; i < 8; ++i)
+                if (t == 4 * gq + 16 * (i / 4) + i % 4) s[i / 4][0][i % 4] = sum;
+        }
+        float p[RT][8];
+        softmax<true>(s, hid, t0, p);
+#pragma unroll 2
+        for (int t = 0; t < kUnit; ++t) {
+            const int64_t v = (bh * a.Rcap + window_slot(a, t0 + t)) * D + 4 * gq;
+            float4 y[NBV];
+#pragma unroll
+            for (int nb = 0; nb < NBV; ++nb) y[nb] = ring4(a.v_res, v + 16 * nb);
+            float w = 0.f;                     // the token's weight, where it lies
+#pragma unroll
+            for (int j = 0; j < 8; ++j)
+                if (j == 4 * (t / 16) + t % 4) w = p[0][j];
+            w = __shfl(w, 16 * (t % 16 / 4) + col);
+            if (((hid >> t) & 1u) || t >= vis[0] - t0) continue;
+#pragma unroll
+            for (int nb = 0; nb < NBV; ++nb) {
+                O[0][nb][0] = fmaf(w, y[nb].x, O[0][nb][0]);
+                O[0][nb][1] = fmaf(w, y[nb].y, O[0][nb][1]);
+                O[0][nb][2] = fmaf(w, y[nb].z, O[0][nb][2]);
+                O[0][nb][3] = fmaf(w, y[nb].w, O[0][nb][3]);
+            }
+        }
     }
 };
 
@@ -416,90 +467,6 @@ struct Range {
         return min(end, n_cu + (vis_most + kUnit - 1) / kUnit);
     }
 };
-
-// Rows row0 .. row0+n-1 of a workgroup's range in plain fp32, a wave per row,
-// lanes over channels: for keys, values or queries that are not finite as
-// bf16.  The pieces of an infinity are no sum (inf - inf), and a score of -inf
-// has to give its token no weight.  Runs after the walk has found such an
-// element (nothing of the walk is live then) and writes over its result.
-template <int D, bool R16>
-__device__ __forceinline__ void slow_rows(const RowsLaunch& a, const Range& rg, int row0, int n,
-                                          int64_t bh, int b, int kvh, int split) {
-    constexpr int C = D / kWave, E = R16 ? 2 : 4;         // channels per lane: lane + 64 c
-    const int lane = threadIdx.x % kWave, waves = blockDim.x / kWave;
-    const gptr kr = (gptr)a.k_res + bh * a.Rcap * D * E, vr = (gptr)a.v_res + bh * a.Rcap * D * E;
-    const uint32_t half_mask = a.res_dt == kSrcF16 ? ~0u : 0u;
-    const int np = a.G * D / 1024, ng = D / a.Gv;
-    for (int r = row0 + (int)threadIdx.x / kWave; r < min(row0 + n, a.rows); r += waves) {
-        const int vis = min(a.vis0 + r / a.hg, a.res_len);
-        float q[C];
-#pragma unroll
-        for (int c = 0; c < C; ++c)
-            q[c] = load1_dt(a.q, query_offset(a, b, kvh, r) + lane + kWave * c, a.io_dt);
-        float o[C] = {}, m = -INFINITY, l = 0.f;
-#pragma unroll 1
-        for (int u = rg.begin; u < rg.end; ++u) {
-            const uint32_t hid = rg.hidden(u);
-            const bool win = u >= rg.n_cu;
-            const int t0 = kUnit * (u - rg.n_cu);
-            if (win && t0 >= rg.vis_most) break;
-            const int64_t cid = bh * a.Cmax + (win ? 0 : u * kUnit / a.G);
-            const int tc = win ? 0 : u * kUnit % a.G;     // the unit's first token in its chunk
-#pragma unroll 1
-            for (int t = 0; t < kUnit; ++t) {
-                if (win && t0 + t >= a.res_len) break;
-                float part = 0.f, v[C];
-#pragma unroll
-                for (int c = 0; c < C; ++c) {
-                    const int d = lane + kWave * c;
-                    float kx;
-                    if (win) {
-                        const uint32_t at = E * ((uint32_t)window_slot(a, t0 + t) * D + d);
-                        const uint32_t kw = ring_word<R16>(kr, at), vw = ring_word<R16>(vr, at);
-                        kx = R16 ? widen16(kw, half_mask) : __uint_as_float(kw);
-                        v[c] = R16 ? widen16(vw, half_mask) : __uint_as_float(vw);
-                    } else {
-                        const int tt = tc + t;            // see kLayoutMfma
-                        const int ktile = d / 32 * (a.G / 16) + tt / 16;
-                        const int vtile = tt / 32 * (D / 16) + d / 16;
-                        const gptr kc = (gptr)a.k_codes + cid * (a.G * D / 4);
-                        const gptr vc = (gptr)a.v_codes + cid * (a.G * D / 4);
-                        const uint32_t kw = gload<uint32_t>(
-                            kc, 4 * ((16 * (d % 32 / 8) + tt % 16) * np + ktile / 2));
-                        const uint32_t vw = gload<uint32_t>(
-                            vc, 4 * ((16 * (tt % 32 / 8) + d % 16) * np + vtile / 2));
-                        const int64_t km = cid * D + d, vm = (cid * ng + d / a.Gv) * a.G + tt;
-                        kx = fmaf((float)((kw >> mfma_code_bit(ktile % 2, d % 8)) & 3u),
-                                  a.k_scale[km], a.k_zero[km]);
-                        v[c] = fmaf((float)((vw >> mfma_code_bit(vtile % 2, tt % 8)) & 3u),
-                                    a.v_scale[vm], a.v_zero[vm]);
-                    }
-                    part = fmaf(q[c], kx, part);
-                }
-#pragma unroll
-                for (int x = 1; x < kWave; x *= 2) part += __shfl_xor(part, x);
-                const bool off = ((hid >> t) & 1u) || (win && t0 + t >= vis);
-                const float s = off ? -INFINITY : part * a.qscale;
-                if (s > m + kMoveMax) {
-                    const float f = exp2_fast(m - s);
-                    m = s;
-                    l *= f;
-#pragma unroll
-                    for (int c = 0; c < C; ++c) o[c] *= f;
-                }
-                // (by the score and not by `off`: a seen token's score can be -inf
-                // while the maximum still is)
-                const float w = s == -INFINITY ? 0.f : exp2_fast(s - m);
-                l += w;
-#pragma unroll
-                for (int c = 0; c < C; ++c) o[c] = fmaf(w, v[c], o[c]);
-            }
-        }
-        const RowDst dst = row_dst(a, b, kvh, bh, r, split, m, l, lane == 0);
-#pragma unroll
-        for (int c = 0; c < C; ++c) store1_as(dst.p, dst.at + lane + kWave * c, o[c] * dst.f, dst.dt);
-    }
-}
 
 // ---------------------------------------------------------------------------
 // Many rows: units expanded into LDS by the whole workgroup.
@@ -697,15 +664,11 @@ struct WindowUnit {
         }
     }
     __device__ __forceinline__ void expand(unsigned char* buf, const Dst<D>& d, int wave,
-                                           uint32_t half_mask, RingTop<R16>& top,
-                                           SplitConsts k) const {
+                                           uint32_t half_mask, SplitConsts k) const {
         if (!has_word<D>(wave)) return;
 #pragma unroll
         for (int i = 0; i < N; ++i) {
             const bool key = word_of<D>(i, wave).key;
-#pragma unroll
-            for (int j = 0; j < 16; ++j)
-                if (!R16 || !key || j % 8 < 4) top.add(raw[i][j]);
 #pragma unroll
             for (int m = 0; m < 2; ++m) {
                 float x[8];
@@ -737,8 +700,9 @@ __device__ __forceinline__ void order_products() {
     }
 }
 
-// Returns whether this thread met a window element that is not finite as bf16.
-template <int D, int RT, int NQ, bool R16>
+// Returns whether a window sum of this thread came out NaN.  PLAIN: the window
+// in plain fp32.
+template <int D, int RT, int NQ, bool R16, bool PLAIN>
 __device__ bool walk_shared(const RowsLaunch& a, unsigned char* smem, const Range& rg, int row0,
                             int64_t bh, int b, int kvh, int split) {
     using S = SharedShape<D>;
@@ -796,7 +760,6 @@ __device__ bool walk_shared(const RowsLaunch& a, unsigned char* smem, const Rang
         order_products<S::NBV, VP, VP * (VP + 1) / 2 * RT>();
     };
 
-    bool bad = false;
     if (rg.begin < rg.c_end) {
         PackedUnit<D> unit;
         const Dst<D> dst(wave, lane, S::VSTR);
@@ -826,9 +789,11 @@ __device__ bool walk_shared(const RowsLaunch& a, unsigned char* smem, const Rang
         }
     }
     const int w_begin = max(rg.begin, rg.n_cu), w_end = rg.w_end();
-    if (w_begin < w_end) {
+    if constexpr (PLAIN) {
+        for (int u = w_begin; active && u < w_end; ++u)
+            rows.template plain_unit<R16>(a, bh, b, kvh, row0, rg.hidden(u), kUnit * (u - rg.n_cu));
+    } else if (w_begin < w_end) {
         WindowUnit<D, R16> unit;
-        RingTop<R16> top;
         const uint32_t half_mask = a.res_dt == kSrcF16 ? ~0u : 0u;
         const Dst<D> dst(wave, lane, kVPWin);
         unit.load(a, bh, kUnit * (w_begin - rg.n_cu), wave, lane);
@@ -836,15 +801,14 @@ __device__ bool walk_shared(const RowsLaunch& a, unsigned char* smem, const Rang
             const int t0 = kUnit * (u - rg.n_cu);
             const uint32_t hid = rg.hidden(u);
             lds_barrier();                     // the previous unit has been read
-            unit.expand(smem, dst, wave, half_mask, top, rows.spc);
+            unit.expand(smem, dst, wave, half_mask, rows.spc);
             unit.load(a, bh, t0 + kUnit, wave, lane);
             lds_barrier();
             if (active) use_unit(smem, hid, t0, BoolC<true>{}, kVPWin, [] {}, [] {});
         }
-        bad = top.bad(half_mask);
     }
 
-    if (!active) return bad;
+    if (!active) return false;
     const int gq = lane / 16;
 #pragma unroll
     for (int rt = 0; rt < RT; ++rt) {
@@ -858,7 +822,7 @@ __device__ bool walk_shared(const RowsLaunch& a, unsigned char* smem, const Rang
             d.store4(16 * nb + 4 * gq, o[0], o[1], o[2], o[3]);
         }
     }
-    return bad;
+    return rows.bad;
 }
 
 template <int D, int RT, bool R16>
@@ -885,19 +849,19 @@ void attn_rows_shared_kernel(RowsLaunch a) {
     };
     // What the workgroup's queries need (uniform: both walks hold workgroup
     // barriers).
-    const int kind = any_wave(query_kind<D, RT>(a, row0, b, kvh));
-    bool bad = kind & kSlow;
-    if (!(kind & kWide)) {
-        bad |= walk_shared<D, RT, 1, R16>(a, smem, rg, row0, bh, b, kvh, split);
+    bool bad = false;
+    if (!any_wave(wide_queries<D, RT>(a, row0, b, kvh))) {
+        bad = walk_shared<D, RT, 1, R16, false>(a, smem, rg, row0, bh, b, kvh, split);
     } else {
         // three query pieces: one row tile at a time (the pieces of two do not
         // fit the registers)
         for (int rt = 0; rt < RT; ++rt)
-            bad |= walk_shared<D, 1, 3, R16>(a, smem, rg, row0 + 16 * rt, bh, b, kvh, split);
+            bad |= walk_shared<D, 1, 3, R16, false>(a, smem, rg, row0 + 16 * rt, bh, b, kvh, split);
     }
     if (__builtin_expect(any_wave(__builtin_amdgcn_ballot_w64(bad) != 0), 0)) {
-        __syncthreads();                       // the walk's results are written
-        slow_rows<D, R16>(a, rg, block0, a.block_rows, bh, b, kvh, split);
+        __syncthreads();                       // the first results are written
+        for (int rt = 0; rt < RT; ++rt)
+            walk_shared<D, 1, 3, R16, true>(a, smem, rg, row0 + 16 * rt, bh, b, kvh, split);
     }
 }
 
@@ -1016,7 +980,7 @@ __device__ __forceinline__ void operands8(const float* x, bf16x8_t* f, SplitCons
     for (int i = 0; i < NP; ++i) f[i] = __builtin_bit_cast(bf16x8_t, p[i]);
 }
 
-template <int D, int RT, int NQ, bool R16>
+template <int D, int RT, int NQ, bool R16, bool PLAIN>
 __device__ bool walk_wave(const RowsLaunch& a, unsigned char* smem, const Range& rg, int row0,
                           int64_t bh, int b, int kvh, int split) {
     constexpr int KS = D / 32;
@@ -1024,7 +988,6 @@ __device__ bool walk_wave(const RowsLaunch& a, unsigned char* smem, const Range&
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
     Rows<D, RT, NQ> rows;
     rows.init(a, row0, b, kvh);
-    RingTop<R16> top;
     const int ng = D / a.Gv;
     float* mt = reinterpret_cast<float*>(smem + wave * WaveShape<D>::META);
 
@@ -1091,6 +1054,10 @@ __device__ bool walk_wave(const RowsLaunch& a, unsigned char* smem, const Range&
          u < w_end; u += kWaveWaves) {
         const int t0 = kUnit * (u - rg.n_cu);
         const uint32_t hid = rg.hidden(u);
+        if constexpr (PLAIN) {
+            rows.template plain_unit<R16>(a, bh, b, kvh, row0, hid, t0);
+            continue;
+        }
         u32x4_t kq[2][KS][E / 2];
 #pragma unroll
         for (int nb = 0; nb < 2; ++nb) {
@@ -1119,7 +1086,6 @@ __device__ bool walk_wave(const RowsLaunch& a, unsigned char* smem, const Range&
 #pragma unroll
                 for (int j = 0; j < 8; ++j) {
                     const uint32_t d = kq[nb][ks][R16 ? 0 : j / 4][R16 ? j / 2 : j % 4];
-                    top.add(d);
                     x[j] = R16 ? widen16((d >> (16 * (j % 2))) & 0xffffu, half_mask)
                                : __uint_as_float(d);
                 }
@@ -1141,7 +1107,6 @@ __device__ bool walk_wave(const RowsLaunch& a, unsigned char* smem, const Range&
 #pragma unroll
             for (int j = 0; j < 8; ++j) {
                 const uint32_t d = ring_word<R16>(vr, vo[j] + 16 * E * nb);
-                top.add(d);
                 x[j] = R16 ? widen16(d, half_mask) : __uint_as_float(d);
             }
             operands8<kVPWin>(x, vf, rows.spc);
@@ -1174,14 +1139,13 @@ __device__ bool walk_wave(const RowsLaunch& a, unsigned char* smem, const Range&
     for (int e = threadIdx.x; e < NR * (D / 4); e += kWaveBlock) {
         const int i = e / (D / 4), d = 4 * (e % (D / 4)), r = row0 + i;
         if (r >= a.rows) continue;
-        float M = -INFINITY, L = 0.f;
+        float M = -FLT_MAX, L = 0.f;
 #pragma unroll
         for (int w = 0; w < kWaveWaves; ++w) M = fmaxf(M, sm[w * NR + i]);
         float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
 #pragma unroll
         for (int w = 0; w < kWaveWaves; ++w) {
-            const float mw = sm[w * NR + i];
-            const float f = mw == -INFINITY ? 0.f : exp2_fast(mw - M);
+            const float f = exp2_fast(sm[w * NR + i] - M);
             const float4 o = *reinterpret_cast<const float4*>(st + (w * NR + i) * D + d);
             L = fmaf(f, sl[w * NR + i], L);
             acc.x = fmaf(f, o.x, acc.x);
@@ -1193,7 +1157,7 @@ __device__ bool walk_wave(const RowsLaunch& a, unsigned char* smem, const Range&
         dst.store4(d, acc.x, acc.y, acc.z, acc.w);
     }
     __syncthreads();                                         // (another walk may follow)
-    return top.bad(half_mask);
+    return rows.bad;
 }
 
 template <int D, int RT, bool R16>
@@ -1205,21 +1169,24 @@ void attn_rows_wave_kernel(RowsLaunch a) {
     const int64_t bh = (int64_t)b * a.Hkv + kvh;
     const int row0 = rblock * a.block_rows;
     const Range rg(a, split, b, row0 + a.block_rows - 1);
+    bool bad = false;
     // (every wave holds the same rows, so the answer is the workgroup's)
-    const int kind = query_kind<D, RT>(a, row0, b, kvh);
-    bool bad = kind & kSlow;
-    if (!(kind & kWide)) {
-        bad |= walk_wave<D, RT, 1, R16>(a, smem, rg, row0, bh, b, kvh, split);
+    if (!wide_queries<D, RT>(a, row0, b, kvh)) {
+        bad = walk_wave<D, RT, 1, R16, false>(a, smem, rg, row0, bh, b, kvh, split);
     } else {
         for (int rt = 0; rt < RT; ++rt)
-            bad |= walk_wave<D, 1, 3, R16>(a, smem, rg, row0 + 16 * rt, bh, b, kvh, split);
+            bad |= walk_wave<D, 1, 3, R16, false>(a, smem, rg, row0 + 16 * rt, bh, b, kvh, split);
     }
     int* word = reinterpret_cast<int*>(smem);
     bad = __builtin_amdgcn_ballot_w64(bad) != 0;
     if (threadIdx.x % kWave == 0) word[threadIdx.x / kWave] = bad;
     __syncthreads();
-    if (__builtin_expect(word[0] | word[1] | word[2] | word[3], 0))
-        slow_rows<D, R16>(a, rg, row0, a.block_rows, bh, b, kvh, split);
+    bad = word[0] | word[1] | word[2] | word[3];
+    if (__builtin_expect(__builtin_amdgcn_readfirstlane(bad), 0)) {
+        __syncthreads();                       // (every wave has read the words)
+        for (int rt = 0; rt < RT; ++rt)
+            walk_wave<D, 1, 3, R16, true>(a, smem, rg, row0 + 16 * rt, bh, b, kvh, split);
+    }
 }
 
 // Merges the split partials: one wave per query row, the sums in split order.
@@ -1229,7 +1196,7 @@ __global__ __launch_bounds__(256) void attn_rows_merge_kernel(RowsLaunch a) {
     if (row >= (int64_t)a.B * a.Hkv * a.rows) return;
     const int S = a.n_splits, D = a.D;
     const float* ml = a.part_ml + row * S * 2;
-    float M = -INFINITY;
+    float M = -FLT_MAX;
     for (int s = 0; s < S; ++s) M = fmaxf(M, ml[2 * s]);
     const int64_t bh = row / a.rows;
     const int64_t out = out_offset(a, (int)(bh / a.Hkv), (int)(bh % a.Hkv), (int)(row % a.rows));
@@ -1239,8 +1206,7 @@ __global__ __launch_bounds__(256) void attn_rows_merge_kernel(RowsLaunch a) {
         float L = 0.f;
 #pragma unroll 4
         for (int s = 0; s < S; ++s) {
-            const float m = ml[2 * s];
-            const float f = m == -INFINITY ? 0.f : exp2_fast(m - M);
+            const float f = exp2_fast(ml[2 * s] - M);
             const float4 o = *reinterpret_cast<const float4*>(po + (int64_t)s * D + d);
             L = fmaf(f, ml[2 * s + 1], L);
             acc.x = fmaf(f, o.x, acc.x);

@@ -34,18 +34,23 @@ def _store(hip_device, B, Hkv, D, G, Gv, R, T, L, ring):
     return st, k, v
 
 
+def _bound(q, kh, kr):
+    """The bound above for queries [B, L, Hq, D]."""
+    B, L, Hq, D = q.shape
+    keys = np.abs(np.concatenate([kh, kr], 2))
+    qa = np.abs(q).reshape(B, L, keys.shape[1], -1, D)
+    smax = max(float((qa[b, :, h].reshape(-1, D) @ keys[b, h].T).max())
+               for b in range(B) for h in range(keys.shape[1])) * D ** -0.5
+    return 3 * 2.0 ** -18 + 2 * (6 * D / 32) * 2.0 ** -24 * smax
+
+
 def _check(out, q, st, k, v, G, Gv, **mask):
     kh, vh = oracle_history(k, v, st.n_chunks, G, Gv)
     q0 = st.n_chunks * G
     qn, kr, vr = q.transpose(1, 2).numpy(), k[:, :, q0:].numpy(), v[:, :, q0:].numpy()
     ref = prefix_attention(qn, kh, vh, kr, vr, **mask)
     size = prefix_attention(qn, kh, np.abs(vh), kr, np.abs(vr), **mask)
-    B, L, Hq, D = qn.shape
-    keys = np.abs(np.concatenate([kh, kr], 2))
-    qa = np.abs(qn).reshape(B, L, keys.shape[1], -1, D)
-    smax = max(float((qa[b, :, h].reshape(-1, D) @ keys[b, h].T).max())
-               for b in range(B) for h in range(keys.shape[1])) * D ** -0.5
-    bound = 3 * 2.0 ** -18 + 2 * (6 * D / 32) * 2.0 ** -24 * smax
+    bound = _bound(qn, kh, kr)
     err = np.abs(out.cpu().numpy().astype(np.float64) - ref) / np.maximum(size, 1e-30)
     print(f"[rows]   largest error {err.max():.2e} of sum p|v| (bound {bound:.2e})", flush=True)
     assert err.max() <= bound
@@ -144,7 +149,8 @@ def test_infinite_window_elements(hip_device, ring, L):
     assert bool(torch.isfinite(rest).all())
 
 
-@pytest.mark.parametrize("Hq,D,G,Gv,T,L,splits,ring", [
+ODD_CASES = [
+    # Hq, D, G, Gv, T, L, splits, ring (B = Hkv = 1, R = 64)
     (4, 128, 32, 32, 40, 5, 0, "f32"),        # the window alone, 20 rows
     (4, 128, 32, 32, 40, 40, 0, "bf16"),      # the same, 160 rows
     (3, 64, 64, 64, 333, 7, 3, "f16"),        # G = 64, three splits
@@ -152,7 +158,10 @@ def test_infinite_window_elements(hip_device, ring, L):
     (4, 128, 64, 128, 600, 40, 2, "f32"),     # one value group
     (4, 256, 32, 256, 400, 3, 2, "f32"),      # head_dim 256, 12 rows
     (4, 256, 64, 128, 400, 30, 2, "bf16"),    # 120 rows
-])
+]
+
+
+@pytest.mark.parametrize("Hq,D,G,Gv,T,L,splits,ring", ODD_CASES)
 def test_infinite_key_comes_first(hip_device, Hq, D, G, Gv, T, L, splits, ring):
     """A token whose score is -inf takes no weight also where it is the first
     that a row sees: at the start of the context, after left padding, behind
@@ -173,3 +182,64 @@ def test_infinite_key_comes_first(hip_device, Hq, D, G, Gv, T, L, splits, ring):
     holes = torch.arange(total)[None, :] >= pos
     out = st.attention(q.cuda(), num_splits=splits, key_mask=holes)
     _check(out, q, st, k, v, G, Gv, visible=(holes & vis).numpy())
+
+
+@pytest.mark.parametrize("half_q", [False, True])
+@pytest.mark.parametrize("Hq,D,G,Gv,T,L,splits,ring", ODD_CASES)
+def test_window_elements_that_are_not_finite(hip_device, Hq, D, G, Gv, T, L, splits, ring, half_q):
+    """An infinite or NaN window element touches what sees it and nothing else:
+    not the rows it is hidden from (padding, or a token after theirs), nor, in a
+    value, the other channels."""
+    print(f"[rows] not finite: D={D} G={G} Gv={Gv} T={T} L={L} {splits} {ring} {half_q}", flush=True)
+    st, k, v = _store(hip_device, 1, 1, D, G, Gv, 64, T, L, ring)
+    q = torch.randn(1, Hq, L, D, generator=torch.Generator().manual_seed(L))
+    if half_q:
+        q = q.bfloat16().float()
+    q0, n = st.quantized_tokens, st.res_len
+    total = q0 + n
+    vis = torch.ones(1, total, dtype=torch.bool)
+    vis[0, q0 + 2] = False
+    plain = st.attention(q.cuda(), num_splits=splits)
+    inf, nan = float("inf"), float("nan")
+    # two results of the bound's size apart, at most
+    tol = 2 * _bound(q.transpose(1, 2).numpy(), k.numpy(), k.numpy()) * float(v.abs().max())
+
+    def poisoned(t, key, value, **kw):
+        slot = (st.res_start + t) % st.R
+        saved = st.k_res[0, 0, slot].clone(), st.v_res[0, 0, slot].clone()
+        if key is not None:
+            st.k_res[0, 0, slot, 5] = key
+        if value is not None:
+            st.v_res[0, 0, slot, D - 3] = value
+        out = st.attention(q.cuda(), num_splits=splits, **kw)
+        st.k_res[0, 0, slot], st.v_res[0, 0, slot] = saved
+        return out
+
+    # hidden by holes, or before the first visible position
+    for key, value in ((nan, nan), (inf, -inf), (-inf, inf)):
+        _check(poisoned(2, key, value, key_mask=vis), q, st, k, v, G, Gv, visible=vis.numpy())
+        _check(poisoned(2, key, value, kv_start=[q0 + 3]), q, st, k, v, G, Gv,
+               kv_start=np.array([q0 + 3]))
+    # the newest token: its own rows only
+    out = poisoned(n - 1, nan, nan)
+    assert bool(out[:, -1].isnan().all())
+    assert float((out - plain)[:, :-1].abs().max()) <= tol
+    # a value that every row sees: its channel only
+    for value in (nan, inf):
+        out = poisoned(0, None, value)
+        assert not bool(out[..., D - 3].isfinite().any())
+        out[..., D - 3] = plain[..., D - 3]
+        assert float((out - plain).abs().max()) <= tol
+    # a key: every row that sees it is NaN, or the token takes no weight
+    out = poisoned(0, nan, None)
+    assert bool(out.isnan().all())
+    # finite keys whose scores overflow to -inf, first in sight
+    if ring != "f16":
+        qq = q.clone()
+        qq[..., 5] = 1e3
+        slot = st.res_start
+        st.k_res[0, 0, slot, 5] = -3e38
+        out = st.attention(qq.cuda(), num_splits=splits, kv_start=[q0])
+        st.k_res[0, 0, slot, 5] = 0.0
+        kk = k.clone()
+        _check(out, qq, st, kk, v, G, Gv, kv_start=np.array([q0 + 1]))

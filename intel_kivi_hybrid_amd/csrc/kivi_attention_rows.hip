@@ -15,6 +15,9 @@
 // * K_hat and V_hat are expanded into MFMA A operands as bf16 pieces (hi + mid
 //   + lo for keys and for the fp32 window's values, hi + lo for packed
 //   values): a packed code word already holds one lane's codes of two tiles.
+//   Packed values enter as their offset (c - 1.5) vs from the middle of their
+//   group's range; the middles vz + 1.5 vs, one per token and group, are rows of
+//   a tile of their own, whose sums are added at the end (Rows::middles).
 // * Scores are formed transposed, S^T = K_hat Q^T, so a lane holds the scores
 //   of one query row (its l % 16) for 8 of the unit's tokens, and the output
 //   transposed too, O^T = V_hat^T P^T: a row's softmax state and rescale are
@@ -23,9 +26,10 @@
 // * Precision: products of pieces are accumulated in fp32.  A query whose
 //   values are all bf16 (a bf16 model's, widened) takes one piece and three
 //   products per key tile, any other query three pieces and six products
-//   (~2^-24 relative); packed values take three products of two pieces
-//   (~2^-17 per weight, averaged over the context), window values six of
-//   three.  The softmax is online in fp32, in the log2 domain; its maximum
+//   (~2^-24 relative); packed values' offsets take three products of two
+//   pieces (~2^-17 of p vs per token, averaged over the context), their
+//   groups' middles and window values six of three: a common part of the
+//   values, which does not average out, keeps fp32's precision.  The softmax is online in fp32, in the log2 domain; its maximum
 //   moves only when exceeded by more than 8 (weights <= 256).
 // * Elements that are not finite as bf16 have no pieces (inf - inf): every sum
 //   that they enter comes out NaN.  A workgroup whose window sums come out NaN
@@ -60,6 +64,7 @@ constexpr float kMoveMax = 8.0f;            // log2 units
 constexpr int kWindowWeight = 2;            // cost of a window unit in packed units
 constexpr int kKP = 3;                      // key pieces
 constexpr int kVPWin = 3, kVPChunk = 2;     // value pieces: window, packed chunks
+constexpr int kPP = 3;                      // weight pieces
 constexpr int kTile = kWave * 16;           // bytes of one operand tile
 
 template <bool V>
@@ -136,6 +141,24 @@ __device__ __forceinline__ void split8(const float* x, u32x4_t* p, SplitConsts k
     }
 }
 
+// The middles of packed values: row m of their operand tile is a block of 32
+// channels (which share a value group).
+__device__ __forceinline__ constexpr int middle_block(int m, int D) {
+    return D > 128 ? m % 8 : m % 4 % (D / 32);
+}
+// Up to four blocks: the same stacked in one operand, piece m / 4 in row m, the
+// last four rows ones, whose sum is the normaliser's: half of the products, and
+// one tile to keep in LDS, but the fold crosses lanes.
+__device__ __forceinline__ u32x4_t middle_stack(const float* mid, int lane, SplitConsts k) {
+    u32x4_t p[3], z;
+    split8<3>(mid, p, k);
+    const int i = lane % 16 / 4;
+#pragma unroll
+    for (int c = 0; c < 4; ++c)
+        z[c] = i == 0 ? p[0][c] : i == 1 ? p[1][c] : i == 2 ? p[2][c] : 0x3f803f80u;
+    return z;
+}
+
 // acc[rt] += (sum of A pieces) * (sum of B pieces of rt): the products of
 // pieces i and j with i + j < max(NA, NB), smallest first (LAST 1: all but the
 // product of the first pieces).
@@ -198,11 +221,13 @@ __device__ __forceinline__ bool wide_queries(const RowsLaunch& a, int row0, int 
 }
 
 // A wave's RT tiles of 16 query rows: operands, softmax state and output.
-template <int D, int RT, int NQ>
+// STACKED: the middles' pieces lie in one operand (middle_stack).
+template <int D, int RT, int NQ, bool STACKED>
 struct Rows {
     static constexpr int KS = D / 32, NBV = D / 16;
     bf16x8_t qf[RT][KS][NQ];
     f32x4_t O[RT][NBV];
+    f32x4_t Z[RT];                  // weighted middles (STACKED: and weights)
     float m[RT], l[RT];
     int vis[RT];                    // window tokens the lane's row sees
     float qs;                       // |softmax scale * log2 e| (its sign is in the query)
@@ -223,6 +248,7 @@ struct Rows {
             // also where it comes first, and any finite one moves it)
             m[rt] = -FLT_MAX;
             l[rt] = 0.f;
+            Z[rt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
             for (int nb = 0; nb < NBV; ++nb) O[rt][nb] = f32x4_t{0.f, 0.f, 0.f, 0.f};
         }
@@ -297,40 +323,78 @@ struct Rows {
                     const float f = exp2_fast(m[rt] - cm);
                     m[rt] = cm;
                     l[rt] *= f;
+                    Z[rt] *= f;
 #pragma unroll
                     for (int nb = 0; nb < NBV; ++nb) O[rt][nb] *= f;
                 }
             }
-            float sum = 0.f;
 #pragma unroll
             for (int i = 0; i < 8; ++i) p[rt][i] = exp2_fast(fmaf(x[i], qs, -m[rt]));
             if (WIN || hid) {                  // (0 also while the maximum is the lowest)
 #pragma unroll
                 for (int i = 0; i < 8; ++i) p[rt][i] = (off >> i) & 1u ? 0.f : p[rt][i];
             }
+            if (WIN || !STACKED) {
+                float sum = 0.f;
 #pragma unroll
-            for (int i = 0; i < 8; ++i) sum += p[rt][i];
-            l[rt] += sum;
+                for (int i = 0; i < 8; ++i) sum += p[rt][i];
+                l[rt] += sum;
+            }
         }
     }
-    // The weights as VP operand pieces.
-    template <int VP, bool WIN>
+    // The weights as operand pieces.
+    template <bool WIN>
     __device__ __forceinline__ void weights(const f32x4_t (&s)[2][RT], uint32_t hid, int t0,
-                                            bf16x8_t (&pf)[RT][VP]) {
+                                            bf16x8_t (&pf)[RT][kPP]) {
         float p[RT][8];
         softmax<WIN>(s, hid, t0, p);
 #pragma unroll
         for (int rt = 0; rt < RT; ++rt) {
             u32x4_t w[3];
-            split8<VP>(p[rt], w, spc);
+            split8<kPP>(p[rt], w, spc);
 #pragma unroll
-            for (int i = 0; i < VP; ++i) pf[rt][i] = __builtin_bit_cast(bf16x8_t, w[i]);
+            for (int i = 0; i < kPP; ++i) pf[rt][i] = __builtin_bit_cast(bf16x8_t, w[i]);
         }
     }
+    // Z += middles x weights, rounded once per unit.
+    static constexpr int MID_TILES = STACKED ? 1 : kPP, MID_PRODUCTS = (STACKED ? 3 : 6) * RT;
+    __device__ __forceinline__ void middles(const u32x4_t* zt, const bf16x8_t (&pf)[RT][kPP]) {
+        f32x4_t z[RT];
+        bf16x8_t zf[MID_TILES];
+#pragma unroll
+        for (int i = 0; i < MID_TILES; ++i) zf[i] = __builtin_bit_cast(bf16x8_t, zt[i]);
+#pragma unroll
+        for (int rt = 0; rt < RT; ++rt) z[rt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+        mul_pieces<MID_TILES, kPP, RT>(z, zf, [&](int rt, int j) { return pf[rt][j]; });
+#pragma unroll
+        for (int rt = 0; rt < RT; ++rt) Z[rt] += z[rt];
+    }
+    // O += Z (and l), after the packed units: the lane's Z[.][i] is row 4 gq + i.
+    __device__ __forceinline__ void fold_middles() {
+        const int gq = (threadIdx.x % kWave) / 16;
+#pragma unroll
+        for (int rt = 0; rt < RT; ++rt) {
+            if constexpr (STACKED) l[rt] += gq == 3 ? Z[rt][0] : 0.f;
+#pragma unroll
+            for (int w = 0; w < KS; ++w) {
+                float x = Z[rt][w % 4];
+                if constexpr (STACKED) {
+                    x = row4_sum(gq == 3 ? 0.f : x);
+                } else if constexpr (KS > 4) {         // half of the blocks are 16 lanes away
+                    const float other = __shfl_xor(x, 16);
+                    x = w / 4 == gq % 2 ? x : other;
+                }
+                O[rt][2 * w] += x;
+                O[rt][2 * w + 1] += x;
+            }
+            Z[rt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+        }
+    }
+
     // O[.][nb] += value tile nb (VP pieces) x weights.  A window unit's sum is
     // formed apart and rounds O once.
     template <int VP>
-    __device__ __forceinline__ void values(const bf16x8_t* vf, const bf16x8_t (&pf)[RT][VP], int nb) {
+    __device__ __forceinline__ void values(const bf16x8_t* vf, const bf16x8_t (&pf)[RT][kPP], int nb) {
         constexpr bool WIN = VP == kVPWin;
         f32x4_t o[RT];
 #pragma unroll
@@ -493,7 +557,11 @@ struct SharedShape {
     // then write a third piece nobody reads, instead of branching)
     static constexpr int VSTR = WORDS > 1 ? 2 : 3;
     static constexpr int K_BYTES = KS * 2 * kKP * kTile;
-    static constexpr int BUF = K_BYTES + NBV * VSTR * kTile;
+    // the middles' tile, stacked (at head_dim 256 LDS is full: each wave makes
+    // their operands itself)
+    static constexpr bool MID_LDS = D <= 128;
+    static constexpr int MID = K_BYTES + NBV * VSTR * kTile;
+    static constexpr int BUF = MID + (MID_LDS ? kTile : 0);
     static constexpr int LDS = 2 * BUF;
     static_assert(K_BYTES + NBV * kVPWin * kTile <= LDS, "a window unit fits");
 };
@@ -517,6 +585,13 @@ __device__ __forceinline__ Word word_of(int i, int wave) {
     return {wave < KS, wave % KS};
 }
 
+// Byte offset, in a value operand tile, of row lane % 16's tokens 8 (lane / 16) ..
+// + 3 (the next four lie 256 bytes on).
+__device__ __forceinline__ uint32_t value_slot(int lane) {
+    const int gq = lane / 16;
+    return ((2 * (gq % 2)) * 16 + lane % 16) * 16 + 8 * (gq / 2);
+}
+
 // Where a thread stores its words' pieces: byte offset in a buffer of (tile 2w,
 // piece 0)'s first half, distance of the second half, of the tiles 2w + 1, of
 // the pieces (kTile).  Key operands are lane-major.  Value operands: this
@@ -526,13 +601,11 @@ template <int D>
 struct Dst {
     uint32_t at[SharedShape<D>::WORDS], half[SharedShape<D>::WORDS], tile[SharedShape<D>::WORDS];
     __device__ __forceinline__ Dst(int wave, int lane, int vstr) {
-        const int gq = lane / 16, col = lane % 16;
 #pragma unroll
         for (int i = 0; i < SharedShape<D>::WORDS; ++i) {
             const Word x = word_of<D>(i, wave);
             at[i] = x.key ? (2 * x.w * kKP) * kTile + lane * 16
-                          : SharedShape<D>::K_BYTES + (2 * x.w * vstr) * kTile +
-                                ((2 * (gq % 2)) * 16 + col) * 16 + 8 * (gq / 2);
+                          : SharedShape<D>::K_BYTES + (2 * x.w * vstr) * kTile + value_slot(lane);
             half[i] = x.key ? 8 : 256;
             tile[i] = (x.key ? kKP : vstr) * kTile;
         }
@@ -594,6 +667,31 @@ struct PackedUnit {
             zr[i][1] = gload<kivi_f4v>(zero[i] + m, meta_off[i] + 16);
         }
     }
+    // Value words enter as offsets from the middle of their group's range, c vs -
+    // 1.5 vs: call once after load().
+    float mid[8];                  // N == 1: the word's middles
+    __device__ __forceinline__ void center(int wave) {
+#pragma unroll
+        for (int i = 0; i < N; ++i) {
+            const bool key = word_of<D>(i, wave).key;
+#pragma unroll
+            for (int c = 0; c < 8; ++c) {
+                if constexpr (N == 1) mid[c] = fmaf(1.5f, sc[i][c / 4][c % 4], zr[i][c / 4][c % 4]);
+                zr[i][c / 4][c % 4] = key ? zr[i][c / 4][c % 4] : -1.5f * sc[i][c / 4][c % 4];
+            }
+        }
+    }
+    // N == 1: a value word's rows of the middles' tile.
+    __device__ __forceinline__ void put_middles(unsigned char* buf, int wave, int lane,
+                                                SplitConsts k) const {
+        const Word w = word_of<D>(0, wave);
+        if (w.key || !has_word<D>(wave)) return;
+        const u32x4_t z = middle_stack(mid, lane, k);
+        if (middle_block(lane % 16, D) != w.w) return;
+        unsigned char* at = buf + SharedShape<D>::MID + value_slot(lane);
+        *reinterpret_cast<uint2*>(at) = make_uint2(z[0], z[1]);
+        *reinterpret_cast<uint2*>(at + 256) = make_uint2(z[2], z[3]);
+    }
     // Expands tile m of every word into buffer `buf`.
     template <int M>
     __device__ __forceinline__ void expand(unsigned char* buf, const Dst<D>& d, int wave,
@@ -621,6 +719,32 @@ struct PackedUnit {
                 put_tile<kKP>(at, d.half[i], x, k);
             }
         }
+    }
+};
+
+// The middles of the lane's row for the 8 tokens of its operand slots, from
+// global memory.
+template <int D>
+struct Middles {
+    kivi_f4v sc[2], zr[2];
+
+    __device__ __forceinline__ void load(const RowsLaunch& a, int64_t bh, int u, int lane) {
+        const int two = a.G == 64 ? 2 : 1, ng = D / a.Gv;
+        const int chunk = two == 2 ? u >> 1 : u, half = two == 2 ? u & 1 : 0;
+        const int64_t at = (bh * a.Cmax + chunk) * ng * a.G + kUnit * half;
+        const uint32_t off =
+            4u * (32 * middle_block(lane % 16, D) / a.Gv * a.G + 4 * (lane / 16));
+        const gptr s = (gptr)(a.v_scale + at), z = (gptr)(a.v_zero + at);
+        sc[0] = gload<kivi_f4v>(s, off);
+        sc[1] = gload<kivi_f4v>(s, off + 64);
+        zr[0] = gload<kivi_f4v>(z, off);
+        zr[1] = gload<kivi_f4v>(z, off + 64);
+    }
+    __device__ __forceinline__ void operands(u32x4_t* zf, SplitConsts k) const {
+        float x[8];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) x[j] = fmaf(1.5f, sc[j / 4][j % 4], zr[j / 4][j % 4]);
+        split8<kPP>(x, zf, k);
     }
 };
 
@@ -688,11 +812,14 @@ struct WindowUnit {
 // and MFMAS products each: the reads run two tiles ahead of the products.  Left
 // to itself the compiler reads a tile right before its products and waits
 // out the LDS latency each time.
-template <int TILES, int READS, int MFMAS>
+// LEAD products of LEAD_READS reads of their own come first, behind the first
+// reads.
+template <int TILES, int READS, int MFMAS, int LEAD = 0, int LEAD_READS = 0>
 __device__ __forceinline__ void order_products() {
     constexpr int kMfma = 0x8, kDsRead = 0x100;
     constexpr int AHEAD = TILES < 2 ? TILES : 2;
-    __builtin_amdgcn_sched_group_barrier(kDsRead, AHEAD * READS, 0);
+    __builtin_amdgcn_sched_group_barrier(kDsRead, AHEAD * READS + LEAD_READS, 0);
+    if constexpr (LEAD > 0) __builtin_amdgcn_sched_group_barrier(kMfma, LEAD, 0);
 #pragma unroll
     for (int t = 0; t < TILES; ++t) {
         __builtin_amdgcn_sched_group_barrier(kMfma, MFMAS, 0);
@@ -709,14 +836,14 @@ __device__ bool walk_shared(const RowsLaunch& a, unsigned char* smem, const Rang
     const int lane = threadIdx.x % kWave;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
     const bool active = row0 < a.rows;         // wave-uniform
-    Rows<D, RT, NQ> rows;
+    Rows<D, RT, NQ, S::MID_LDS> rows;
     rows.init(a, row0, b, kvh);
 
     // One unit from LDS buffer `buf`; after_k and after_v run behind the reads
     // of the key and of the value tiles: the expansion of the next unit, whose
     // vector work then sits among this unit's matrix products.
     auto use_unit = [&](const unsigned char* buf, uint32_t hid, int t0, auto win_c, int vstr,
-                        auto&& after_k, auto&& after_v) {
+                        const Middles<D>& mid, auto&& after_k, auto&& after_v) {
         constexpr bool WIN = decltype(win_c)::value;
         constexpr int VP = WIN ? kVPWin : kVPChunk;
         f32x4_t s[2][RT], small[2][RT];
@@ -745,8 +872,16 @@ __device__ bool walk_shared(const RowsLaunch& a, unsigned char* smem, const Rang
         }
         after_k();
         order_products<2 * S::KS, kKP, (NQ == 1 ? 3 : 6) * RT>();
-        bf16x8_t pf[RT][VP];
-        rows.template weights<VP, WIN>(s, hid, t0, pf);
+        bf16x8_t pf[RT][kPP];
+        rows.template weights<WIN>(s, hid, t0, pf);
+        if constexpr (!WIN) {
+            u32x4_t zf[decltype(rows)::MID_TILES];
+            if constexpr (S::MID_LDS)
+                zf[0] = *reinterpret_cast<const u32x4_t*>(buf + S::MID + lane * 16);
+            else
+                mid.operands(zf, rows.spc);
+            rows.middles(zf, pf);
+        }
 #pragma unroll
         for (int nb = 0; nb < S::NBV; ++nb) {
             bf16x8_t vf[VP];
@@ -757,7 +892,8 @@ __device__ bool walk_shared(const RowsLaunch& a, unsigned char* smem, const Rang
             rows.template values<VP>(vf, pf, nb);
         }
         after_v();
-        order_products<S::NBV, VP, VP * (VP + 1) / 2 * RT>();
+        order_products<S::NBV, VP, VP * (VP + 1) / 2 * RT, WIN ? 0 : decltype(rows)::MID_PRODUCTS,
+                       WIN || !S::MID_LDS ? 0 : 1>();
     };
 
     if (rg.begin < rg.c_end) {
@@ -767,26 +903,38 @@ __device__ bool walk_shared(const RowsLaunch& a, unsigned char* smem, const Rang
         unit.init(a, bh, wave, lane);
         unit.load(two, rg.begin);
         lds_barrier();                         // an earlier walk has read its last unit
+        unit.center(wave);
         unit.template expand<0>(smem, dst, wave, rows.spc);
         unit.template expand<1>(smem, dst, wave, rows.spc);
+        if constexpr (S::MID_LDS) unit.put_middles(smem, wave, lane, rows.spc);
         unit.load(two, min(rg.begin + 1, rg.c_end - 1));
         for (int u = rg.begin; u < rg.c_end; ++u) {
             const uint32_t hid = rg.hidden(u);
             unsigned char* cur = smem + ((u - rg.begin) & 1) * S::BUF;
             unsigned char* nxt = smem + ((u - rg.begin + 1) & 1) * S::BUF;
+            Middles<D> mid;
+            if constexpr (!S::MID_LDS) mid.load(a, bh, u, lane);
             lds_barrier();                     // cur is written, nxt has been read
-            auto first = [&] { unit.template expand<0>(nxt, dst, wave, rows.spc); };
+            auto first = [&] {
+                unit.center(wave);
+                unit.template expand<0>(nxt, dst, wave, rows.spc);
+            };
             auto second = [&] {
                 unit.template expand<1>(nxt, dst, wave, rows.spc);
-                unit.load(two, min(u + 2, rg.c_end - 1));
+                if constexpr (!S::MID_LDS) unit.load(two, min(u + 2, rg.c_end - 1));
             };
             if (active && hid != ~0u) {
-                use_unit(cur, hid, 0, BoolC<false>{}, S::VSTR, first, second);
+                use_unit(cur, hid, 0, BoolC<false>{}, S::VSTR, mid, first, second);
             } else {
                 first();
                 second();
             }
+            if constexpr (S::MID_LDS) {        // (a branch: it would break the order above)
+                unit.put_middles(nxt, wave, lane, rows.spc);
+                unit.load(two, min(u + 2, rg.c_end - 1));
+            }
         }
+        rows.fold_middles();
     }
     const int w_begin = max(rg.begin, rg.n_cu), w_end = rg.w_end();
     if constexpr (PLAIN) {
@@ -804,7 +952,7 @@ __device__ bool walk_shared(const RowsLaunch& a, unsigned char* smem, const Rang
             unit.expand(smem, dst, wave, half_mask, rows.spc);
             unit.load(a, bh, t0 + kUnit, wave, lane);
             lds_barrier();
-            if (active) use_unit(smem, hid, t0, BoolC<true>{}, kVPWin, [] {}, [] {});
+            if (active) use_unit(smem, hid, t0, BoolC<true>{}, kVPWin, {}, [] {}, [] {});
         }
     }
 
@@ -986,7 +1134,7 @@ __device__ bool walk_wave(const RowsLaunch& a, unsigned char* smem, const Range&
     constexpr int KS = D / 32;
     const int lane = threadIdx.x % kWave, gq = lane / 16, col = lane % 16;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
-    Rows<D, RT, NQ> rows;
+    Rows<D, RT, NQ, false> rows;
     rows.init(a, row0, b, kvh);
     const int ng = D / a.Gv;
     float* mt = reinterpret_cast<float*>(smem + wave * WaveShape<D>::META);
@@ -1023,8 +1171,21 @@ __device__ bool walk_wave(const RowsLaunch& a, unsigned char* smem, const Range&
                     rows.keys(s[nb], kf, ks);
                 }
             }
-            bf16x8_t pf[RT][kVPChunk];
-            rows.template weights<kVPChunk, false>(s, hid, 0, pf);
+            bf16x8_t pf[RT][kPP];
+            rows.template weights<false>(s, hid, 0, pf);
+            {
+                float sc[8], x[8];
+                u32x4_t zf[kPP];
+                const float* p = mt + 2 * D + kUnit * (32 * middle_block(col, D) / a.Gv) + 4 * gq;
+                read4(p, sc);
+                read4(p + 16, sc + 4);
+                read4(p + kUnit * ng, x);
+                read4(p + kUnit * ng + 16, x + 4);
+#pragma unroll
+                for (int j = 0; j < 8; ++j) x[j] = fmaf(1.5f, sc[j], x[j]);
+                split8<kPP>(x, zf, rows.spc);
+                rows.middles(zf, pf);
+            }
 #pragma unroll
             for (int w = 0; w < KS; ++w) {
                 float sc[8], zr[8], x[2][8];
@@ -1032,8 +1193,8 @@ __device__ bool walk_wave(const RowsLaunch& a, unsigned char* smem, const Range&
                 const float* p = mt + 2 * D + kUnit * (32 * w / a.Gv) + 4 * gq;
                 read4(p, sc);
                 read4(p + 16, sc + 4);
-                read4(p + kUnit * ng, zr);
-                read4(p + kUnit * ng + 16, zr + 4);
+#pragma unroll
+                for (int j = 0; j < 8; ++j) zr[j] = -1.5f * sc[j];
                 expand_word<4>(unit.va[w] >> vshift, sc, zr, x[0], x[1]);
                 expand_word<4>(unit.vb[w] >> vshift, sc + 4, zr + 4, x[0] + 4, x[1] + 4);
 #pragma unroll
@@ -1044,6 +1205,7 @@ __device__ bool walk_wave(const RowsLaunch& a, unsigned char* smem, const Range&
             }
             unit.load_codes(a, bh, next, lane);
         }
+        rows.fold_middles();
     }
     // window units, dealt in the same turn
     constexpr int E = R16 ? 2 : 4;
@@ -1098,8 +1260,8 @@ __device__ bool walk_wave(const RowsLaunch& a, unsigned char* smem, const Range&
             s[0][rt] += small[0][rt];
             s[1][rt] += small[1][rt];
         }
-        bf16x8_t pf[RT][kVPWin];
-        rows.template weights<kVPWin, true>(s, hid, t0, pf);
+        bf16x8_t pf[RT][kPP];
+        rows.template weights<true>(s, hid, t0, pf);
 #pragma unroll
         for (int nb = 0; nb < D / 16; ++nb) {
             float x[8];
@@ -1189,7 +1351,9 @@ void attn_rows_wave_kernel(RowsLaunch a) {
     }
 }
 
-// Merges the split partials: one wave per query row, the sums in split order.
+// Merges the split partials: one wave per query row.  Each sum runs as four, of
+// every fourth split: up to 64 splits of even weight, added one after the
+// other, would round at the sum's full size each time.
 __global__ __launch_bounds__(256) void attn_rows_merge_kernel(RowsLaunch a) {
     const int64_t row = (int64_t)blockIdx.x * 4 + threadIdx.x / kWave;
     const int lane = threadIdx.x % kWave;
@@ -1202,21 +1366,37 @@ __global__ __launch_bounds__(256) void attn_rows_merge_kernel(RowsLaunch a) {
     const int64_t out = out_offset(a, (int)(bh / a.Hkv), (int)(bh % a.Hkv), (int)(row % a.rows));
     const float* po = a.part_o + row * S * D;
     for (int d = 4 * lane; d < D; d += 4 * kWave) {
-        float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
-        float L = 0.f;
-#pragma unroll 4
-        for (int s = 0; s < S; ++s) {
+        float4 acc[4];
+        float L[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            acc[i] = make_float4(0.f, 0.f, 0.f, 0.f);
+            L[i] = 0.f;
+        }
+        auto add = [&](int i, int s) {
             const float f = exp2_fast(ml[2 * s] - M);
             const float4 o = *reinterpret_cast<const float4*>(po + (int64_t)s * D + d);
-            L = fmaf(f, ml[2 * s + 1], L);
-            acc.x = fmaf(f, o.x, acc.x);
-            acc.y = fmaf(f, o.y, acc.y);
-            acc.z = fmaf(f, o.z, acc.z);
-            acc.w = fmaf(f, o.w, acc.w);
+            L[i] = fmaf(f, ml[2 * s + 1], L[i]);
+            acc[i].x = fmaf(f, o.x, acc[i].x);
+            acc[i].y = fmaf(f, o.y, acc[i].y);
+            acc[i].z = fmaf(f, o.z, acc[i].z);
+            acc[i].w = fmaf(f, o.w, acc[i].w);
+        };
+        int s = 0;
+#pragma unroll 2
+        for (; s + 4 <= S; s += 4) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) add(i, s + i);
         }
-        const float f = L > 0.f || L != L ? 1.f / L : 0.f;      // 0: every position hidden
-        store4_as(a.out, out + d, make_float4(acc.x * f, acc.y * f, acc.z * f, acc.w * f),
-                  a.io_dt);
+        for (; s < S; ++s) add(0, s);
+        const float l = (L[0] + L[1]) + (L[2] + L[3]);
+        const float f = l > 0.f || l != l ? 1.f / l : 0.f;      // 0: every position hidden
+        auto sum = [&](float a0, float a1, float a2, float a3) { return ((a0 + a1) + (a2 + a3)) * f; };
+        store4_as(a.out, out + d,
+                  make_float4(sum(acc[0].x, acc[1].x, acc[2].x, acc[3].x),
+                              sum(acc[0].y, acc[1].y, acc[2].y, acc[3].y),
+                              sum(acc[0].z, acc[1].z, acc[2].z, acc[3].z),
+                              sum(acc[0].w, acc[1].w, acc[2].w, acc[3].w)), a.io_dt);
     }
 }
 

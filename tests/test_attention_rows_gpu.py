@@ -22,11 +22,11 @@ from tests.kv_helpers import make_kv, oracle_history
 
 pytestmark = pytest.mark.gpu
 
-def _store(hip_device, B, Hkv, D, G, Gv, R, T, L, ring):
+def _store(hip_device, B, Hkv, D, G, Gv, R, T, L, ring, v_offset=0.0):
     from intel_kivi_hybrid_amd.store import PackedKVStore
     dt = {"f32": torch.float32, "bf16": torch.bfloat16, "f16": torch.float16}[ring]
     k, v = make_kv(B, Hkv, T + L, D, seed=T + L + D)
-    k, v = k.to(dt).float(), v.to(dt).float()
+    k, v = k.to(dt).float(), (v + v_offset).to(dt).float()
     st = PackedKVStore(B, Hkv, D, G, R + L, "cuda:0", group_size_v=Gv, residual_dtype=dt,
                        chunk_capacity=T // G + 1)
     st.extend(k[:, :, :T].to("cuda", dt), v[:, :, :T].to("cuda", dt), flush_at=R)
@@ -243,3 +243,38 @@ def test_window_elements_that_are_not_finite(hip_device, Hq, D, G, Gv, T, L, spl
         st.k_res[0, 0, slot, 5] = 0.0
         kk = k.clone()
         _check(out, qq, st, kk, v, G, Gv, kv_start=np.array([q0 + 1]))
+
+
+@pytest.mark.parametrize("Hq,D,G,Gv,T,L,splits,ring", ODD_CASES[2:] + [
+    (4, 128, 32, 32, 600, 5, 0, "f32"),       # 20 rows, four value groups
+    (4, 256, 32, 32, 400, 30, 0, "f32"),      # eight value groups
+])
+def test_common_part_of_the_values(hip_device, Hq, D, G, Gv, T, L, splits, ring):
+    """Values with a common offset of 20: packed values lose 3 * 2^-18 of their
+    offset from the middle of their group's range (at most 1.5 scales), not of
+    themselves.  Queries of one channel, so that a score is one product (6
+    roundings of 2^-24, 2 more before the exponential): a weight is off by eps,
+    which moves the output by eps * sum p |v - o|.  The output's fp32 sums round
+    once per 32 tokens, and a few times at the end."""
+    print(f"[rows] offset: D={D} G={G} Gv={Gv} T={T} L={L} {splits} {ring}", flush=True)
+    st, k, v = _store(hip_device, 1, 1, D, G, Gv, 64, T, L, ring, v_offset=20.0)
+    g = torch.Generator().manual_seed(L)
+    q = torch.zeros(1, Hq, L, D)
+    q[..., 11] = 3 * D ** 0.5 * torch.randn(1, Hq, L, generator=g)
+    out = st.attention(q.cuda(), num_splits=splits).cpu().numpy().astype(np.float64)
+    kh, vh = oracle_history(k, v, st.n_chunks, G, Gv)
+    q0 = st.quantized_tokens
+    qn, kr, vr = q.transpose(1, 2).numpy(), k[:, :, q0:].numpy(), v[:, :, q0:].numpy()
+    ref = prefix_attention(qn, kh, vh, kr, vr)
+    groups = v[:, :, :q0].reshape(1, 1, q0, D // Gv, Gv)
+    scale = ((groups.amax(-1) - groups.amin(-1)) / 3).repeat_interleave(Gv, -1).numpy()
+    part = 1.5 * prefix_attention(qn, kh, scale, kr, 0 * vr)
+    square = prefix_attention(qn, kh, vh.astype(np.float64) ** 2, kr, vr.astype(np.float64) ** 2)
+    spread = np.sqrt(np.maximum(square - ref ** 2, 0))          # >= sum p |v - o|
+    smax = float(np.abs(qn).max() * np.abs(k.numpy()).max()) * D ** -0.5
+    eps = 2 * (8 * 2.0 ** -24 * smax + 2.0 ** -22)
+    units = (T + L) / 32 + 8
+    bound = 3 * 2.0 ** -18 * part + eps * spread + units * 2.0 ** -24 * np.abs(ref)
+    err = np.abs(out - ref) / bound
+    print(f"[rows]   largest error {err.max():.2f} of the bound", flush=True)
+    assert err.max() <= 1

@@ -225,7 +225,12 @@ __device__ __forceinline__ bool wide_queries(const RowsLaunch& a, int row0, int 
 template <int D, int RT, int NQ, bool STACKED>
 struct Rows {
     static constexpr int KS = D / 32, NBV = D / 16;
-    bf16x8_t qf[RT][KS][NQ];
+    // Three pieces of two tiles do not fit the registers: they lie in LDS, once
+    // for the waves of a workgroup that holds the same rows in all of them.
+    static constexpr bool Q_LDS = RT * NQ > 3;
+    static constexpr int Q_BYTES = RT * KS * NQ * kTile;
+    bf16x8_t qf[Q_LDS ? 1 : RT][Q_LDS ? 1 : KS][NQ];
+    unsigned char* ql;
     f32x4_t O[RT][NBV];
     f32x4_t Z[RT];                  // weighted middles (STACKED: and weights)
     float m[RT], l[RT];
@@ -235,8 +240,11 @@ struct Rows {
     bool bad = false;               // a window sum of this lane came out NaN
 
     // rows row0 .. (those past the end repeat the last; they are not stored)
-    __device__ __forceinline__ void init(const RowsLaunch& a, int row0, int b, int kvh) {
+    // q_lds (Q_LDS): Q_BYTES of LDS, which the workgroup may read after a barrier.
+    __device__ __forceinline__ void init(const RowsLaunch& a, int row0, int b, int kvh,
+                                         unsigned char* q_lds = nullptr) {
         const int lane = threadIdx.x % kWave, col = lane % 16, gq = lane / 16;
+        ql = q_lds + lane * 16;
         spc = split_consts();
         qs = fabsf(a.qscale);
         const float sign = a.qscale < 0.f ? -1.f : 1.f;
@@ -265,24 +273,44 @@ struct Rows {
                 u32x4_t p[3];
                 split8<NQ>(x, p, spc);
 #pragma unroll
-                for (int i = 0; i < NQ; ++i) qf[rt][ks][i] = __builtin_bit_cast(bf16x8_t, p[i]);
+                for (int i = 0; i < NQ; ++i) {
+                    if constexpr (Q_LDS) *q_at(rt, ks, i) = __builtin_bit_cast(bf16x8_t, p[i]);
+                    else qf[rt][ks][i] = __builtin_bit_cast(bf16x8_t, p[i]);
+                }
             }
         }
         });
     }
+    __device__ __forceinline__ bf16x8_t* q_at(int rt, int ks, int i) const {
+        return reinterpret_cast<bf16x8_t*>(ql + ((rt * KS + ks) * NQ + i) * kTile);
+    }
+    __device__ __forceinline__ void query(bf16x8_t (&q)[RT][NQ], int ks) const {
+#pragma unroll
+        for (int rt = 0; rt < RT; ++rt) {
+#pragma unroll
+            for (int i = 0; i < NQ; ++i) {
+                if constexpr (Q_LDS) q[rt][i] = *q_at(rt, ks, i);
+                else q[rt][i] = qf[rt][ks][i];
+            }
+        }
+    }
 
     // s[rt] += key tile (kKP pieces) x query at k-step ks
     __device__ __forceinline__ void keys(f32x4_t (&s)[RT], const bf16x8_t* kf, int ks) {
-        mul_pieces<kKP, NQ, RT>(s, kf, [&](int rt, int j) { return qf[rt][ks][j]; });
+        bf16x8_t q[RT][NQ];
+        query(q, ks);
+        mul_pieces<kKP, NQ, RT>(s, kf, [&](int rt, int j) { return q[rt][j]; });
     }
     // The same for the window's fp32 keys, the small products in a sum of their
     // own: s then rounds once per k-step at its full size, as plain fp32 sums
     // over that many channels at most do.
     __device__ __forceinline__ void window_keys(f32x4_t (&s)[RT], f32x4_t (&small)[RT],
                                                 const bf16x8_t* kf, int ks) {
-        mul_pieces<kKP, NQ, RT, 1>(small, kf, [&](int rt, int j) { return qf[rt][ks][j]; });
+        bf16x8_t q[RT][NQ];
+        query(q, ks);
+        mul_pieces<kKP, NQ, RT, 1>(small, kf, [&](int rt, int j) { return q[rt][j]; });
 #pragma unroll
-        for (int rt = 0; rt < RT; ++rt) s[rt] = mfma(kf[0], qf[rt][ks][0], s[rt]);
+        for (int rt = 0; rt < RT; ++rt) s[rt] = mfma(kf[0], q[rt][0], s[rt]);
     }
 
     // Online softmax of a unit's scores s[nb][rt] (unscaled), leaving the
@@ -1003,12 +1031,12 @@ void attn_rows_shared_kernel(RowsLaunch a) {
     } else {
         // three query pieces: one row tile at a time (the pieces of two do not
         // fit the registers)
-        for (int rt = 0; rt < RT; ++rt)
+        for (int rt = 0; rt < RT && block0 + 16 * rt < a.rows; ++rt)
             bad |= walk_shared<D, 1, 3, R16, false>(a, smem, rg, row0 + 16 * rt, bh, b, kvh, split);
     }
     if (__builtin_expect(any_wave(__builtin_amdgcn_ballot_w64(bad) != 0), 0)) {
         __syncthreads();                       // the first results are written
-        for (int rt = 0; rt < RT; ++rt)
+        for (int rt = 0; rt < RT && block0 + 16 * rt < a.rows; ++rt)
             walk_shared<D, 1, 3, R16, true>(a, smem, rg, row0 + 16 * rt, bh, b, kvh, split);
     }
 }
@@ -1135,7 +1163,11 @@ __device__ bool walk_wave(const RowsLaunch& a, unsigned char* smem, const Range&
     const int lane = threadIdx.x % kWave, gq = lane / 16, col = lane % 16;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
     Rows<D, RT, NQ, false> rows;
-    rows.init(a, row0, b, kvh);
+    static_assert(!decltype(rows)::Q_LDS ||
+                  kWaveWaves * WaveShape<D>::META + decltype(rows)::Q_BYTES <= WaveShape<D>::LDS,
+                  "the query's pieces lie behind the staged scales");
+    rows.init(a, row0, b, kvh, smem + kWaveWaves * WaveShape<D>::META);   // (by every wave alike)
+    if constexpr (decltype(rows)::Q_LDS) lds_barrier();
     const int ng = D / a.Gv;
     float* mt = reinterpret_cast<float*>(smem + wave * WaveShape<D>::META);
 
@@ -1333,12 +1365,10 @@ void attn_rows_wave_kernel(RowsLaunch a) {
     const Range rg(a, split, b, row0 + a.block_rows - 1);
     bool bad = false;
     // (every wave holds the same rows, so the answer is the workgroup's)
-    if (!wide_queries<D, RT>(a, row0, b, kvh)) {
+    if (!wide_queries<D, RT>(a, row0, b, kvh))
         bad = walk_wave<D, RT, 1, R16, false>(a, smem, rg, row0, bh, b, kvh, split);
-    } else {
-        for (int rt = 0; rt < RT; ++rt)
-            bad |= walk_wave<D, 1, 3, R16, false>(a, smem, rg, row0 + 16 * rt, bh, b, kvh, split);
-    }
+    else
+        bad = walk_wave<D, RT, 3, R16, false>(a, smem, rg, row0, bh, b, kvh, split);
     int* word = reinterpret_cast<int*>(smem);
     bad = __builtin_amdgcn_ballot_w64(bad) != 0;
     if (threadIdx.x % kWave == 0) word[threadIdx.x / kWave] = bad;
@@ -1346,7 +1376,7 @@ void attn_rows_wave_kernel(RowsLaunch a) {
     bad = word[0] | word[1] | word[2] | word[3];
     if (__builtin_expect(__builtin_amdgcn_readfirstlane(bad), 0)) {
         __syncthreads();                       // (every wave has read the words)
-        for (int rt = 0; rt < RT; ++rt)
+        for (int rt = 0; rt < RT && row0 + 16 * rt < a.rows; ++rt)
             walk_wave<D, 1, 3, R16, true>(a, smem, rg, row0 + 16 * rt, bh, b, kvh, split);
     }
 }

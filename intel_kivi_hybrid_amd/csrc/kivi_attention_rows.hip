@@ -836,23 +836,14 @@ struct WindowUnit {
     }
 };
 
-// Scheduling order of a product phase of TILES operand tiles, READS LDS reads
-// and MFMAS products each: the reads run two tiles ahead of the products.  Left
-// to itself the compiler reads a tile right before its products and waits
-// out the LDS latency each time.
-// LEAD products of LEAD_READS reads of their own come first, behind the first
-// reads.
-template <int TILES, int READS, int MFMAS, int LEAD = 0, int LEAD_READS = 0>
-__device__ __forceinline__ void order_products() {
-    constexpr int kMfma = 0x8, kDsRead = 0x100;
-    constexpr int AHEAD = TILES < 2 ? TILES : 2;
-    __builtin_amdgcn_sched_group_barrier(kDsRead, AHEAD * READS + LEAD_READS, 0);
-    if constexpr (LEAD > 0) __builtin_amdgcn_sched_group_barrier(kMfma, LEAD, 0);
-#pragma unroll
-    for (int t = 0; t < TILES; ++t) {
-        __builtin_amdgcn_sched_group_barrier(kMfma, MFMAS, 0);
-        if (t + AHEAD < TILES) __builtin_amdgcn_sched_group_barrier(kDsRead, READS, 0);
-    }
+// Between two operand tiles' products: the LDS reads and the products keep their
+// order, everything else may cross.  The reads run two tiles ahead of the
+// products; left to itself the compiler reads a tile right before its products
+// and waits out the LDS latency each time.
+__device__ __forceinline__ void keep_order() {
+    constexpr int kValu = 0x2, kSalu = 0x4, kVmem = 0x10 | 0x20 | 0x40, kDsWrite = 0x200,
+                  kTrans = 0x400;
+    __builtin_amdgcn_sched_barrier(kValu | kSalu | kVmem | kDsWrite | kTrans);
 }
 
 // Returns whether a window sum of this thread came out NaN.  PLAIN: the window
@@ -878,18 +869,22 @@ __device__ bool walk_shared(const RowsLaunch& a, unsigned char* smem, const Rang
 #pragma unroll
         for (int rt = 0; rt < RT; ++rt)
             s[0][rt] = s[1][rt] = small[0][rt] = small[1][rt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+        constexpr int AHEAD = D > 128 ? 1 : 2;
+        bf16x8_t kf[2 * S::KS][kKP];
+        auto read_keys = [&](int t) {
 #pragma unroll
-        for (int ks = 0; ks < S::KS; ++ks) {
+            for (int p = 0; p < kKP; ++p)
+                kf[t][p] = *reinterpret_cast<const bf16x8_t*>(buf + (t * kKP + p) * kTile + lane * 16);
+        };
 #pragma unroll
-            for (int nb = 0; nb < 2; ++nb) {
-                bf16x8_t kf[kKP];
+        for (int t = 0; t < AHEAD; ++t) read_keys(t);
+        keep_order();
 #pragma unroll
-                for (int p = 0; p < kKP; ++p)
-                    kf[p] = *reinterpret_cast<const bf16x8_t*>(
-                        buf + ((2 * ks + nb) * kKP + p) * kTile + lane * 16);
-                if constexpr (WIN) rows.window_keys(s[nb], small[nb], kf, ks);
-                else rows.keys(s[nb], kf, ks);
-            }
+        for (int t = 0; t < 2 * S::KS; ++t) {
+            if (t + AHEAD < 2 * S::KS) read_keys(t + AHEAD);
+            if constexpr (WIN) rows.window_keys(s[t % 2], small[t % 2], kf[t], t / 2);
+            else rows.keys(s[t % 2], kf[t], t / 2);
+            keep_order();
         }
         if constexpr (WIN) {
 #pragma unroll
@@ -899,29 +894,37 @@ __device__ bool walk_shared(const RowsLaunch& a, unsigned char* smem, const Rang
             }
         }
         after_k();
-        order_products<2 * S::KS, kKP, (NQ == 1 ? 3 : 6) * RT>();
         bf16x8_t pf[RT][kPP];
         rows.template weights<WIN>(s, hid, t0, pf);
+        bf16x8_t vf[S::NBV][VP];
+        auto read_values = [&](int nb) {
+#pragma unroll
+            for (int p = 0; p < VP; ++p)
+                vf[nb][p] = *reinterpret_cast<const bf16x8_t*>(buf + S::K_BYTES +
+                                                               (nb * vstr + p) * kTile + lane * 16);
+        };
         if constexpr (!WIN) {
             u32x4_t zf[decltype(rows)::MID_TILES];
             if constexpr (S::MID_LDS)
                 zf[0] = *reinterpret_cast<const u32x4_t*>(buf + S::MID + lane * 16);
             else
                 mid.operands(zf, rows.spc);
+#pragma unroll
+            for (int nb = 0; nb < AHEAD; ++nb) read_values(nb);
+            keep_order();
             rows.middles(zf, pf);
+        } else {
+#pragma unroll
+            for (int nb = 0; nb < AHEAD; ++nb) read_values(nb);
         }
+        keep_order();
 #pragma unroll
         for (int nb = 0; nb < S::NBV; ++nb) {
-            bf16x8_t vf[VP];
-#pragma unroll
-            for (int p = 0; p < VP; ++p)
-                vf[p] = *reinterpret_cast<const bf16x8_t*>(buf + S::K_BYTES +
-                                                           (nb * vstr + p) * kTile + lane * 16);
-            rows.template values<VP>(vf, pf, nb);
+            if (nb + AHEAD < S::NBV) read_values(nb + AHEAD);
+            rows.template values<VP>(vf[nb], pf, nb);
+            keep_order();
         }
         after_v();
-        order_products<S::NBV, VP, VP * (VP + 1) / 2 * RT, WIN ? 0 : decltype(rows)::MID_PRODUCTS,
-                       WIN || !S::MID_LDS ? 0 : 1>();
     };
 
     if (rg.begin < rg.c_end) {
@@ -954,8 +957,16 @@ __device__ bool walk_shared(const RowsLaunch& a, unsigned char* smem, const Rang
             if (active && hid != ~0u) {
                 use_unit(cur, hid, 0, BoolC<false>{}, S::VSTR, mid, first, second);
             } else {
-                first();
-                second();
+                // (as a loop: as plain code the compiler moves what both arms
+                // share above the branch, where it waits for unit's loads
+                // before any product: 36 rows, B=16 58 -> 68 us)
+                int once = 1;
+                asm volatile("" : "+s"(once));
+#pragma unroll 1
+                for (; once; --once) {
+                    first();
+                    second();
+                }
             }
             if constexpr (S::MID_LDS) {        // (a branch: it would break the order above)
                 unit.put_middles(nxt, wave, lane, rows.spc);

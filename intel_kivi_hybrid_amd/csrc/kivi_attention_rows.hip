@@ -1263,38 +1263,53 @@ __device__ bool walk_wave(const RowsLaunch& a, unsigned char* smem, const Range&
             rows.template plain_unit<R16>(a, bh, b, kvh, row0, hid, t0);
             continue;
         }
-        u32x4_t kq[2][KS][E / 2];
+        // (Key loads run up to four k-steps ahead of their use, and a value tile's
+        // are issued before the tile before it is used; left to itself the compiler
+        // waits for each load where registers are short.)
+        constexpr int AHEAD = KS < 4 ? KS : 4, kNoMemory = 0x1;
+        u32x4_t kq[AHEAD][2][E / 2];
+        uint32_t ko[2], vo[8];
 #pragma unroll
-        for (int nb = 0; nb < 2; ++nb) {
-            const uint32_t o = E * ((uint32_t)window_slot(a, t0 + 16 * nb + col) * D + 8 * gq);
-#pragma unroll
-            for (int ks = 0; ks < KS; ++ks) {
-#pragma unroll
-                for (int q = 0; q < E / 2; ++q)
-                    kq[nb][ks][q] = gload<u32x4_t>(kr, o + 32 * E * ks + 16 * q);
-            }
-        }
-        uint32_t vo[8];
+        for (int nb = 0; nb < 2; ++nb)
+            ko[nb] = E * ((uint32_t)window_slot(a, t0 + 16 * nb + col) * D + 8 * gq);
 #pragma unroll
         for (int j = 0; j < 8; ++j)
             vo[j] = E * ((uint32_t)window_slot(a, t0 + 4 * gq + 16 * (j / 4) + j % 4) * D + col);
+        auto load_keys = [&](int ks) {
+#pragma unroll
+            for (int nb = 0; nb < 2; ++nb) {
+#pragma unroll
+                for (int q = 0; q < E / 2; ++q)
+                    kq[ks % AHEAD][nb][q] = gload<u32x4_t>(kr, ko[nb] + 32 * E * ks + 16 * q);
+            }
+        };
         f32x4_t s[2][RT], small[2][RT];
 #pragma unroll
         for (int rt = 0; rt < RT; ++rt)
             s[0][rt] = s[1][rt] = small[0][rt] = small[1][rt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
+        for (int ks = 0; ks < AHEAD; ++ks) load_keys(ks);
+        __builtin_amdgcn_sched_barrier(kNoMemory);
+#pragma unroll
         for (int ks = 0; ks < KS; ++ks) {
+            float x[2][8];
 #pragma unroll
             for (int nb = 0; nb < 2; ++nb) {
-                float x[8];
-                bf16x8_t kf[kKP];
 #pragma unroll
                 for (int j = 0; j < 8; ++j) {
-                    const uint32_t d = kq[nb][ks][R16 ? 0 : j / 4][R16 ? j / 2 : j % 4];
-                    x[j] = R16 ? widen16((d >> (16 * (j % 2))) & 0xffffu, half_mask)
-                               : __uint_as_float(d);
+                    const uint32_t d = kq[ks % AHEAD][nb][R16 ? 0 : j / 4][R16 ? j / 2 : j % 4];
+                    x[nb][j] = R16 ? widen16((d >> (16 * (j % 2))) & 0xffffu, half_mask)
+                                   : __uint_as_float(d);
                 }
-                operands8<kKP>(x, kf, rows.spc);
+            }
+            if (ks + AHEAD < KS) {
+                load_keys(ks + AHEAD);
+                __builtin_amdgcn_sched_barrier(kNoMemory);
+            }
+#pragma unroll
+            for (int nb = 0; nb < 2; ++nb) {
+                bf16x8_t kf[kKP];
+                operands8<kKP>(x[nb], kf, rows.spc);
                 rows.window_keys(s[nb], small[nb], kf, ks);
             }
         }
@@ -1305,15 +1320,21 @@ __device__ bool walk_wave(const RowsLaunch& a, unsigned char* smem, const Range&
         }
         bf16x8_t pf[RT][kPP];
         rows.template weights<true>(s, hid, t0, pf);
+        uint32_t vw[2][8];
+        auto load_values = [&](int nb) {
+#pragma unroll
+            for (int j = 0; j < 8; ++j) vw[nb % 2][j] = ring_word<R16>(vr, vo[j] + 16 * E * nb);
+        };
+        load_values(0);
 #pragma unroll
         for (int nb = 0; nb < D / 16; ++nb) {
             float x[8];
             bf16x8_t vf[kVPWin];
+            if (nb + 1 < D / 16) load_values(nb + 1);
+            __builtin_amdgcn_sched_barrier(kNoMemory);
 #pragma unroll
-            for (int j = 0; j < 8; ++j) {
-                const uint32_t d = ring_word<R16>(vr, vo[j] + 16 * E * nb);
-                x[j] = R16 ? widen16(d, half_mask) : __uint_as_float(d);
-            }
+            for (int j = 0; j < 8; ++j)
+                x[j] = R16 ? widen16(vw[nb % 2][j], half_mask) : __uint_as_float(vw[nb % 2][j]);
             operands8<kVPWin>(x, vf, rows.spc);
             rows.template values<kVPWin>(vf, pf, nb);
         }

@@ -299,9 +299,13 @@ int kivi_packed_decode_attention_noalloc(
  * positions 0 .. kv_start[b]-1, quantised or in the window); each must leave
  * every query token at least one visible position (for causal queries:
  * kv_start[b] <= num_chunks*G + res_len - q_len).
- * When q_len * (q_heads / kv_heads) exceeds 8, a matrix-core store is
- * dequantised once for up to 256 query rows of a kv head at a time; a
- * plain-layout store is streamed once per 8 rows.  No reference counterpart
+ * When q_len * (q_heads / kv_heads) exceeds 8 rows, a matrix-core store is
+ * dequantised once for up to 32 rows of a kv head (head_dim 64 and 128, at most
+ * 64 and 32 rows), 16 (head_dim 256, at most 16 rows), or else 256 rows of
+ * queries that are all bf16 values and 128 of any others (64 at head_dim 256);
+ * a plain-layout store is streamed once per 8 rows.  The partials of such a
+ * call hold all of its rows, batch * q_len * q_heads * splits * (head_dim + 2)
+ * floats: num_splits is followed while they fit 64 MB.  No reference counterpart
  * beyond that math (the reference runs HF attention on the CPU,
  * src/kivi_sycl/cache/manager.py:251-290). */
 size_t kivi_packed_attention_workspace_size(int32_t batch, int32_t q_len, int32_t q_heads,

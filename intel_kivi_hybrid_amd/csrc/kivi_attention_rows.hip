@@ -1497,10 +1497,14 @@ int launch_rows(const RowsLaunch& a, hipStream_t st) {
 // Rows per workgroup, row blocks and splits of a call: 16 or 32 rows per
 // workgroup of the wave kernel; 128 or 256 of the shared one (64 at head_dim
 // 256).  Splits then give every CU a workgroup (two of the wave kernel) while
-// each split keeps at least 12 units of 32 tokens.
+// each split keeps at least 12 units of 32 tokens.  A caller's count is followed
+// while the splits' partials, which hold all rows of the call at once, fit 64 MB
+// (the plan's own never take more than 34; 256 splits of 512 tokens of 32
+// heads would take 2.2 GB).
 RowsPlan rows_plan(int B, int Hkv, int rows, int D, int G, int n_chunks, int res_len,
                    int splits_hint) {
     constexpr int kCUs = 256, kMinUnits = 12;
+    constexpr int64_t kMostPartials = 64 << 20;
     RowsPlan p;
     const bool few = rows <= few_rows(D);
     if (few) p.block_rows = rows > 16 && D <= 128 ? 32 : 16;
@@ -1512,6 +1516,7 @@ RowsPlan rows_plan(int B, int Hkv, int rows, int D, int G, int n_chunks, int res
     const int64_t groups = (int64_t)B * Hkv * p.row_blocks;
     int64_t s = splits_hint;
     if (s <= 0) s = min((few ? 2 : 1) * kCUs / groups, (int64_t)p.n_units / kMinUnits);
+    s = min(s, kMostPartials / ((int64_t)B * Hkv * rows * (D + 2) * (int64_t)sizeof(float)));
     s = max((int64_t)1, min(s, (int64_t)p.n_units));
     p.weight_per_split = (int)((weight + s - 1) / s);
     p.n_splits = (weight + p.weight_per_split - 1) / p.weight_per_split;

@@ -457,13 +457,19 @@ Plan make_plan(int B, int Hkv, int D, int G, int Gv, int n_chunks, int res_len,
         //     (512: two per CU) while every wave keeps >= 16 chunks, so that
         //     one wave per workgroup takes the residual window alone;
         // (b) enough splits for 256 workgroups (one per CU);
-        // and in their place (c) the splits whose workgroups fill all 512
-        // places exactly, where every wave keeps >= 9 chunks (6 with 8 query
-        // rows, whose chunk steps cost twice): an unfilled chip leaves CUs with
-        // one workgroup idle while the others finish two.  B=16 sequences
+        // and in their place (c) the 2 or 4 splits whose workgroups fill all 512
+        // places exactly (256 or 128 pairs of sequence and kv head), where
+        // every wave keeps >= 9 chunks (6 with 8 query rows, whose chunk steps
+        // cost twice): an unfilled chip leaves CUs with one workgroup idle while
+        // the others finish two.  B=16 sequences
         // (bf16 ring), us per call: 64/8 heads at 7777 tokens 46.3 -> 41.8 (3 ->
         // 4 splits), at 4000 35.2 -> 29.7 (2 -> 4); 32/8 heads at 7777 37.2 ->
-        // 33.6; B=32, 32/8 heads at 3000 39.3 -> 31.1 (1 -> 2).
+        // 33.6; B=32, 32/8 heads at 3000 39.3 -> 31.1 (1 -> 2).  Of 1, 2, 3, 4 and 8
+        // rows at 1 to 2.5 times the fewest chunks, fp32 and bf16 rings, the worst
+        // 1.6 % slower and most 2-35 % faster.  Fewer pairs come close to 512
+        // places under (a), whose waves keep one wave for the window: 64 pairs at
+        // 432 chunks and 32 at 864 took 6-8 % longer with 8 and 16 splits than
+        // with 7 and 14, at 1 to 4 rows.
         // Swept over B = 1-64 sequences at 2K-32K contexts (32/8 heads, the
         // best split count per shape against this rule's): B=12 at 8K takes
         // 4 splits (31.5 us; the 2048-wave target below took 6: 39.6 us, 576
@@ -489,7 +495,7 @@ Plan make_plan(int B, int Hkv, int D, int G, int Gv, int n_chunks, int res_len,
                         sa = s;
                 S = max(max(sa, kCUs / pairs), 1);
                 const int sc = kSlots / pairs;
-                if (sc > S && sc * pairs == kSlots &&
+                if (sc > S && sc <= 4 && sc * pairs == kSlots &&
                     n_chunks >= kWavesPerGroup * sc * (rows >= 8 ? 6 : 9))
                     S = sc;
             } else {

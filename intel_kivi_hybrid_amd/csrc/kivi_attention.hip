@@ -87,8 +87,9 @@ __device__ __forceinline__ int ring_slot(int start, int t, int cap) {
     return s >= cap ? s - cap : s;
 }
 
-// The general kernel of plain-layout stores whose value factors ([D/Gv][G]
-// per chunk) are more than kivi_attention_plain.hip keeps (256).
+// The general kernel of plain-layout stores: more value factors ([D/Gv][G] per
+// chunk) than kivi_attention_plain.hip keeps (256), and its slower sizes
+// (plain_attention_takes).
 template <int HG>
 __global__ __launch_bounds__(kAttnBlock) void attn_generic_kernel(AttnArgs a) {
     extern __shared__ float smem[];
@@ -528,18 +529,22 @@ Plan make_plan(int B, int Hkv, int D, int G, int Gv, int n_chunks, int res_len,
         p.n_splits = p.n_qsplits;
         return p;
     }
-    p.plain = plain_attention_supported(D, G, Gv);
+    p.plain = plain_attention_takes(rows, D, G, Gv, B * Hkv, n_chunks);
     if (p.plain) {
         // The most splits whose workgroups fit the chip at once while every
-        // wave keeps at least 3 chunks.  head_dim 96, 4K context, us per call:
-        // B=4, 32/32 heads (four workgroups per CU fit): 6, 8, 15 splits 26.4,
-        // 25.6, 28.5; B=16, 32/8 heads (three fit): 4, 6, 7 splits 49.7, 46.5,
-        // 60.2; B=8, 64/8 heads at 8K (two fit): 6, 8, 10 splits 102, 81, 125.
+        // wave keeps at least 3 chunks; with chunks of 48 or 64 tokens and several
+        // rows at least as many as give every CU a workgroup.  head_dim 96, 4K
+        // context, us per call: B=4, 32/32 heads (four workgroups per CU fit): 6, 8,
+        // 15 splits 26.4, 25.6, 28.5; B=16, 32/8 heads (three fit): 4, 6, 7 splits
+        // 49.7, 46.5, 60.2; B=8, 64/8 heads at 8K (two fit): 6, 8, 10 splits 102, 81,
+        // 125.  G = 64, 32/8 heads, B=4: 5, 8, 11 splits 51.5, 35.8, 35.1.
         constexpr int kWavesPerGroup = 4, kCUs = 256, kMinChunksPerWave = 3;
         int S = splits_hint;
         if (S <= 0)
             S = min(kCUs * plain_attention_groups_per_cu(rows, D, G, Gv) / (B * Hkv),
                     n_chunks / (kWavesPerGroup * kMinChunksPerWave));
+        if (splits_hint <= 0 && G > 32 && rows > 1)
+            S = max(S, min(kCUs / (B * Hkv), n_chunks / kWavesPerGroup));
         S = max(1, min(min(S, kMaxSplits), (n_chunks + kWavesPerGroup - 1) / kWavesPerGroup));
         p.chunks_per_wave = (n_chunks + kWavesPerGroup * S - 1) / (kWavesPerGroup * S);
         p.n_qsplits = n_chunks == 0 ? 1
@@ -1076,9 +1081,18 @@ int kivi_packed_decode_attention_noalloc(
         int32_t kv_heads, int32_t head_dim, int32_t group_size_k, int32_t group_size_v,
         int32_t chunk_capacity, int32_t num_chunks, int32_t res_capacity, int32_t res_start,
         int32_t res_len, float softmax_scale, int32_t num_splits, void* stream) {
-    const size_t need = kivi_packed_decode_attention_workspace_size(
-        batch, q_heads, kv_heads, head_dim, group_size_k, group_size_v, num_chunks, res_len,
-        num_splits);
+    auto bytes = [&](int32_t splits) {
+        return kivi_packed_decode_attention_workspace_size(batch, q_heads, kv_heads, head_dim,
+                                                           group_size_k, group_size_v,
+                                                           num_chunks, res_len, splits);
+    };
+    size_t need = bytes(num_splits);
+    // (the generic kernel's own count can ask for more: fewer then)
+    if (num_splits <= 0 && need > (size_t)KIVI_NOALLOC_SCRATCH_BYTES) {
+        for (num_splits = 256; num_splits > 1; num_splits /= 2)
+            if ((need = bytes(num_splits)) <= (size_t)KIVI_NOALLOC_SCRATCH_BYTES) break;
+        if (num_splits == 1) need = bytes(1);
+    }
     if (need > (size_t)KIVI_NOALLOC_SCRATCH_BYTES)
         return set_error(kErrInvalidArgument,
                          "this launch needs %zu bytes of split partials; the allocation-free "

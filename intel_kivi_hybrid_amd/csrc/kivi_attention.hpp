@@ -105,6 +105,9 @@ int launch_attention_mfma_hg8_r16(const AttnLaunch& a, hipStream_t stream);
 // 8 rows per kv head: AttnLaunch without k_new (the ring holds the token
 // already), n_splits and chunks_per_wave as for the matrix-core kernel.
 bool plain_attention_supported(int D, int G, int Gv);
+// Whether it is ahead of the generic kernel (query rows per kv head of the
+// launch; pairs of sequence and kv head).
+bool plain_attention_takes(int rows, int D, int G, int Gv, int pairs, int n_chunks);
 int launch_attention_plain(const AttnLaunch& a, hipStream_t stream);
 // Workgroups of it that a CU holds (query rows per kv head of the launch).
 int plain_attention_groups_per_cu(int rows, int D, int G, int Gv);

@@ -116,8 +116,8 @@ struct PlainLds {
 // Waves per SIMD (and so workgroups per CU) that the registers of an instance
 // allow; the split plan fills the chip with that many.
 __host__ __device__ constexpr int plain_waves(int HG, int N, int J) {
-    const int w = HG * N <= 4 ? 4 : HG * N <= 12 ? 3 : HG * N <= 32 ? 2 : 1;
-    return J == 4 && w > 1 ? w - 1 : w;
+    if (J == 4) return HG * N <= 4 ? 3 : HG * N <= 16 && N < 16 ? 2 : 1;
+    return HG * N <= 4 ? 4 : HG * N <= 12 ? 3 : HG * N <= 32 ? 2 : 1;
 }
 
 // HG query rows; N code dwords per lane and side of a chunk; J: D and D/Gv * G
@@ -459,6 +459,26 @@ int launch_rows_of(const AttnLaunch& a, hipStream_t st) {
 
 bool plain_attention_supported(int D, int G, int Gv) {
     return D % 16 == 0 && D <= 256 && G % 16 == 0 && G <= kWave && D / Gv * G <= 4 * kWave;
+}
+
+// With 1 or 2 rows, or chunks of up to 32 tokens, this kernel is ahead (the
+// generic one leaves half of its lanes idle at 32 tokens and reads every factor by
+// itself).  With 4 and more rows and chunks of 48 or 64 tokens, where a lane has a
+// whole token, the sums of all rows for its code words and the factors leave one
+// or two waves per SIMD; from 1 to 3 chunks per wave (4 rows of more than 128
+// factors), from 32 chunks in all (8 rows of 48 tokens) and up to 6 per wave (8
+// rows of 64) the generic kernel's many small workgroups win.  us per call, generic / this one (head_dim, G, Gv; B and
+// tokens at 8 kv heads): 4 rows 42.2 / 35.8 (96, 64, 96; 4, 4K), 21.2 / 24.3 (48,
+// 64, 16; 4, 4K), 35.2 / 40.7 (80, 48, 16; 4, 4K), 42.0 / 35.2 (64, 64, 16; 1, 30K); 8
+// rows 50.4 / 61 (96, 64, 32; 4, 4K), 85 / 96 (1, 30K), 257 / 165 (16, 4K), 110 / 118
+// (48, 48, 16; 16, 4K), 46 / 40 (96, 64, 32; 1, 200).
+bool plain_attention_takes(int rows, int D, int G, int Gv, int pairs, int n_chunks) {
+    if (!plain_attention_supported(D, G, Gv)) return false;
+    if (G <= 32 || rows <= 2) return true;
+    const int64_t chunks = (int64_t)pairs * n_chunks, per_wave = kPlainWaves * 256;
+    if (rows == 4)
+        return D / Gv * G <= 2 * kWave || chunks < per_wave || chunks >= 3 * per_wave;
+    return chunks <= 32 || (G > 48 && chunks >= 6 * per_wave);
 }
 
 // The instance (N, J) of a geometry.

@@ -35,6 +35,9 @@ CASES = [
     (2, 12, 1, 64, 16, 16, 32, 20, 0, "bf16"),       # no chunk yet, two head groups
     (1, 2, 2, 256, 16, 64, 64, 400, 0, "f32"),       # head_dim 256
     (1, 2, 2, 128, 32, 8, 64, 300, 0, "f32"),        # 512 value factors: the generic kernel
+    (4, 8, 1, 80, 64, 80, 128, 2000, 0, "bf16"),     # 8 rows of 64 tokens: the generic kernel
+    (4, 32, 8, 48, 48, 16, 96, 2000, 0, "f32"),      # 4 rows of 144 factors: likewise
+    (4, 32, 8, 96, 64, 96, 128, 1000, 0, "f16"),     # 4 rows, a workgroup for every CU
 ]
 
 

@@ -83,11 +83,35 @@ def test_noalloc_matches_workspace_entry_point(hip_device):
 
 
 def test_noalloc_plain_layout_and_wide_head_groups(hip_device):
-    """The generic kernel (a plain-layout store: G = 16) and more than 8
-    query heads per kv head (12: launches over head groups of 8 and 4, each
-    leaving its partials in the same scratch array before its merge), split,
-    against the workspace entry point bit for bit."""
+    """A plain-layout store (G = 16) and more than 8 query heads per kv head (12:
+    launches over head groups of 8 and 4, each leaving its partials in the same
+    scratch array before its merge), split, against the workspace entry point bit
+    for bit."""
     from intel_kivi_hybrid_amd import _native
     lib = _native.load()
     _case(lib, 2, 4, 2, 64, 16, 16, 32, 600, splits=5, seed=14)
     _case(lib, 2, 24, 2, 128, 32, 32, 64, 1500, splits=3, seed=15)
+
+
+def test_noalloc_takes_fewer_splits_where_its_own_count_does_not_fit(hip_device):
+    """The generic kernel (8 rows, G = 48) aims at 2048 workgroups, whose partials
+    exceed the scratch array at head_dim 256 and long contexts."""
+    from intel_kivi_hybrid_amd import _native
+    from intel_kivi_hybrid_amd.store import PackedKVStore
+    lib = _native.load()
+    B, Hq, Hkv, D, G, Gv, R, T = 1, 64, 8, 256, 48, 64, 96, 25000
+    print(f"[noalloc] own count: D={D} G={G} T={T}", flush=True)
+    k, v = make_kv(B, Hkv, T, D, seed=16)
+    st = PackedKVStore(B, Hkv, D, G, R, "cuda:0", group_size_v=Gv)
+    st.extend(k.cuda(), v.cuda(), flush_at=R)
+    q = seeded_q(B, Hq, D, seed=17).cuda()
+    assert st.workspace_bytes(Hq, 0) > KIVI_NOALLOC_SCRATCH_BYTES
+    out = torch.full_like(q, float("nan"))
+    head, tail = _common(st, q, out, 0)
+    _native.check(lib.kivi_packed_decode_attention_noalloc(*head, *tail),
+                  "kivi_packed_decode_attention_noalloc")
+    kh, vh = oracle_history(k, v, st.n_chunks, G, Gv)
+    q0 = st.n_chunks * G
+    err = rel_err(out.cpu().numpy(), decode_attention(q.cpu().numpy(), kh, vh, k[:, :, q0:].numpy(),
+                                                      v[:, :, q0:].numpy()))
+    assert err <= 1e-3

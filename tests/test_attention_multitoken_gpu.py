@@ -12,10 +12,10 @@ packed store (kivi_packed_attention through PackedKVStore.attention).
   attention per query and the reference's cosine > 0.85 gate against fp32
   attention over the unquantised cache.
 
-The shapes cover one launch with padding rows, several launches (q_len *
-Hq/Hkv > 8 rows), forced splits, the long-context mode where one wave takes
-the window, value groups of 128, the plain layout (generic kernel) and a
-context held only in the window.  Bar: 1e-3 relative (max |o - o_ref| /
+The shapes cover one launch with padding rows, steps of more than 8 rows (q_len
+* Hq/Hkv: the many-row kernels), forced splits, the long-context mode where one
+wave takes the window, value groups of 128, the plain layout and a context held
+only in the window.  Bar: 1e-3 relative (max |o - o_ref| /
 max |o_ref| per (batch, token, head)).
 """
 
@@ -39,17 +39,17 @@ def store_cls(hip_device):
 
 CASES = [
     # B, Hq, Hkv, D, G, Gv, R, T, L, splits
-    (2, 8, 2, 128, 32, 32, 128, 600, 3, 0),      # GQA 4: 12 rows -> 2 launches
+    (2, 8, 2, 128, 32, 32, 128, 600, 3, 0),      # GQA 4: 12 rows
     (1, 4, 4, 64, 32, 32, 64, 300, 5, 0),        # MHA: 5 tokens in one launch, 3 padding rows
-    (2, 16, 2, 128, 32, 32, 128, 900, 2, 3),     # GQA 8: one token per launch, 3 splits
-    (1, 8, 2, 128, 32, 128, 128, 2200, 8, 1),    # one split: a wave takes the window, Gv = D
-    (1, 2, 2, 64, 16, 16, 32, 100, 4, 0),        # plain layout: the generic kernel
-    (2, 8, 2, 64, 32, 32, 64, 40, 3, 0),         # no chunk yet: the window pass alone
-    (1, 4, 1, 128, 64, 64, 128, 1300, 6, 4),     # G = 64, GQA 4, 4 splits
-    (1, 6, 2, 128, 32, 32, 128, 600, 3, 0),      # GQA 3: 2 tokens per launch, 2 padding rows
-    (2, 24, 2, 64, 32, 32, 64, 300, 2, 2),       # GQA 12: head groups of 8 and 4, 2 splits
-    (1, 14, 2, 64, 16, 16, 32, 100, 3, 0),       # GQA 7, plain layout: the generic kernel
-    (1, 4, 2, 256, 64, 128, 128, 700, 3, 0),     # D=256, G=64, Gv=128: at most 4 rows per launch
+    (2, 16, 2, 128, 32, 32, 128, 900, 2, 3),     # GQA 8: 16 rows, 3 splits
+    (1, 8, 2, 128, 32, 128, 128, 2200, 8, 1),    # 32 rows, one split, Gv = D
+    (1, 2, 2, 64, 16, 16, 32, 100, 4, 0),        # plain layout
+    (2, 8, 2, 64, 32, 32, 64, 40, 3, 0),         # no chunk yet: the window alone, 12 rows
+    (1, 4, 1, 128, 64, 64, 128, 1300, 6, 4),     # G = 64, 24 rows, 4 splits
+    (1, 6, 2, 128, 32, 32, 128, 600, 3, 0),      # GQA 3: 9 rows
+    (2, 24, 2, 64, 32, 32, 64, 300, 2, 2),       # GQA 12: 24 rows, 2 splits
+    (1, 14, 2, 64, 16, 16, 32, 100, 3, 0),       # GQA 7, plain layout: one token per launch
+    (1, 4, 2, 256, 64, 128, 128, 700, 3, 0),     # D=256, G=64, Gv=128: 6 rows, at most 4 per launch
 ]
 
 

@@ -6,8 +6,10 @@ Rows per kv head sit at the edges of the row tiles (16), of the two kernels (16,
 32 or 64 by head_dim) and of the workgroups' row blocks (64, 128, 256); contexts end inside a 32-token
 unit, lie wholly in the window, and split.  Against float64 attention over the
 oracle's dequantised history, elementwise, with the bound that the arithmetic
-gives.  Weights and values are split into two bf16 pieces each (2^-18 relative)
-and their lo*lo product is dropped (2^-18): 3 * 2^-18 of sum_t p_t |v_t|.
+gives.  Weights and packed values (their offset from the middle of their group's
+range, at most 1.5 scales and so no more than the largest magnitude in the group)
+are split into two bf16 pieces each (2^-18 relative) and their lo*lo product is
+dropped (2^-18): 3 * 2^-18 of sum_t p_t |v_t|, where the data is of zero mean.
 Keys carry three pieces; a score is then a fp32 sum of 6 D/32 matrix products
 (three-piece queries), off by at most 6 D/32 * 2^-24 of sum_d |q_d k_d| *
 scale, which moves a weight and the normaliser by as much each.
@@ -17,8 +19,8 @@ import numpy as np
 import pytest
 import torch
 
-from oracle.attention import prefix_attention
-from tests.kv_helpers import make_kv, oracle_history
+from oracle.attention import decode_attention, prefix_attention
+from tests.kv_helpers import make_kv, oracle_history, rel_err
 
 pytestmark = pytest.mark.gpu
 
@@ -108,6 +110,72 @@ def test_unaligned_queries(hip_device):
     out = torch.empty(q.numel() + 1, device="cuda")[1:].view(B, L, Hq, D)
     st.attention(base[1:].view(B, L, Hq, D).transpose(1, 2), out=out)
     _check(out, q.transpose(1, 2), st, k, v, 32, 32)
+
+
+@pytest.mark.parametrize("Hq,Hkv,D,G,Gv,T,L,splits", [
+    (8, 1, 128, 32, 32, 500, 2, 0),          # 16 rows
+    (24, 2, 64, 32, 32, 300, 2, 2),          # 12 heads: groups of 8 and 4
+    (3, 1, 128, 64, 128, 700, 5, 0),         # 2 tokens per launch, 2 padding rows
+    (4, 1, 256, 64, 128, 500, 3, 0),         # at most 4 rows per launch
+])
+def test_unaligned_queries_take_the_decode_launches(hip_device, Hq, Hkv, D, G, Gv, T, L, splits):
+    """The decode kernel's launches of up to 8 rows, which buffers off the wide
+    loads' alignment take, causal and not."""
+    print(f"[rows] decode launches: Hq={Hq} Hkv={Hkv} D={D} G={G} T={T} L={L}", flush=True)
+    st, k, v = _store(hip_device, 2, Hkv, D, G, Gv, 64, T, L, "f32")
+    q = torch.randn(2, L, Hq, D, generator=torch.Generator().manual_seed(3)) * D ** -0.5
+    base = torch.empty(q.numel() + 1, device="cuda")
+    base[1:] = q.flatten().cuda()
+    kh, vh = oracle_history(k, v, st.n_chunks, G, Gv)
+    q0 = st.n_chunks * G
+    kr, vr = k[:, :, q0:].numpy(), v[:, :, q0:].numpy()
+    for causal in (True, False):
+        out = torch.empty(q.numel() + 1, device="cuda")[1:].view(2, L, Hq, D)
+        st.attention(base[1:].view(2, L, Hq, D).transpose(1, 2), out=out, causal=causal,
+                     num_splits=splits)
+        if causal:
+            ref = prefix_attention(q.numpy(), kh, vh, kr, vr)
+        else:
+            ref = np.stack([decode_attention(q[:, i].numpy(), kh, vh, kr, vr)
+                            for i in range(L)], axis=1)
+        assert rel_err(out.cpu().numpy(), ref) <= 1e-3
+
+
+@pytest.mark.parametrize("B,Hq,Hkv,D,G,Gv,R,T,L,splits,ring,half_q", [
+    (2, 4, 1, 128, 32, 32, 64, 300, 5, 2, "bf16", True),     # 20 rows
+    (1, 3, 1, 64, 64, 64, 64, 333, 30, 0, "f32", False),     # 90 rows
+    (2, 2, 1, 256, 32, 32, 64, 200, 6, 0, "f16", False),     # 12 rows
+    (1, 4, 2, 128, 32, 128, 64, 500, 70, 2, "f32", True),    # 280 rows
+    (1, 3, 1, 128, 32, 32, 64, 20, 8, 0, "bf16", False),     # the window alone
+])
+def test_full_attention_and_masks_together(hip_device, B, Hq, Hkv, D, G, Gv, R, T, L, splits, ring,
+                                           half_q):
+    """causal=False (every row sees the whole context), and a first visible
+    position together with holes, causal and not."""
+    print(f"[rows] full: D={D} G={G} Gv={Gv} T={T} L={L} splits={splits} {ring}", flush=True)
+    st, k, v = _store(hip_device, B, Hkv, D, G, Gv, R, T, L, ring)
+    g = torch.Generator().manual_seed(L + D)
+    q = torch.randn(B, Hq, L, D, generator=g)
+    if half_q:
+        q = q.bfloat16().float()
+    total = st.quantized_tokens + st.res_len
+    start = [min(41 * (b + 1), total - L) for b in range(B)]
+    vis = torch.rand(B, total, generator=g) >= 0.2
+    vis[:, total - L] = True
+    kh, vh = oracle_history(k, v, st.n_chunks, G, Gv)
+    q0 = st.n_chunks * G
+    qn, kr, vr = q.transpose(1, 2).numpy(), k[:, :, q0:].numpy(), v[:, :, q0:].numpy()
+    bound = _bound(qn, kh, kr)
+    for mask, oracle in (({}, {}),
+                         ({"kv_start": start, "key_mask": vis},
+                          {"kv_start": np.array(start), "visible": vis.numpy()})):
+        if mask:
+            _check(st.attention(q.cuda(), num_splits=splits, **mask), q, st, k, v, G, Gv, **oracle)
+        out = st.attention(q.cuda(), num_splits=splits, causal=False, **mask).cpu().numpy()
+        for i in range(L):
+            ref = decode_attention(qn[:, i], kh, vh, kr, vr, **oracle)
+            size = decode_attention(qn[:, i], kh, np.abs(vh), kr, np.abs(vr), **oracle)
+            assert (np.abs(out[:, i] - ref) <= bound * size).all()
 
 
 def test_negative_scale_and_hidden_rows(hip_device):
@@ -278,3 +346,18 @@ def test_common_part_of_the_values(hip_device, Hq, D, G, Gv, T, L, splits, ring)
     err = np.abs(out - ref) / bound
     print(f"[rows]   largest error {err.max():.2f} of the bound", flush=True)
     assert err.max() <= 1
+
+
+@pytest.mark.parametrize("Hq,D,G,Gv,T,L,splits,ring", ODD_CASES)
+def test_a_query_that_is_not_finite_stays_in_its_row(hip_device, Hq, D, G, Gv, T, L, splits, ring):
+    st, k, v = _store(hip_device, 1, 1, D, G, Gv, 64, T, L, ring)
+    q = torch.randn(1, Hq, L, D, generator=torch.Generator().manual_seed(L))
+    plain = st.attention(q.cuda(), num_splits=splits)
+    tol = 2 * _bound(q.transpose(1, 2).numpy(), k.numpy(), k.numpy()) * float(v.abs().max())
+    for x in (float("nan"), float("inf")):
+        bad = q.clone()
+        bad[0, 1, L // 2, 3] = x
+        out = st.attention(bad.cuda(), num_splits=splits)
+        assert bool(out[0, L // 2, 1].isnan().all())
+        out[0, L // 2, 1] = plain[0, L // 2, 1]
+        assert float((out - plain).abs().max()) <= tol

@@ -38,7 +38,7 @@ def test_typed_queries_give_the_converted_call_bits(hip_device, case, dtype):
     huge[0, 0, 0, 0] = 3.4e38 if dtype is not torch.float16 else float("inf")
     forms = [(token_major, {}), (token_major.contiguous(), {}),
              (token_major, {"kv_start": start}), (token_major, {"hidden": hidden}),
-             (huge, {})]                               # (not finite as bf16: rows taken singly)
+             (huge, {})]                               # (not finite as bf16)
     for x, kw in forms:
         assert _C.takes_typed_queries(x, st)
         got = _C.packed_attention_typed(x, st, **kw)

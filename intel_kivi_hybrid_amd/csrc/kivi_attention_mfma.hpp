@@ -83,19 +83,6 @@ constexpr int kBlock = kWaves * kWave;
 constexpr int kResPass = 16;              // residual tokens per pass of a wave
 constexpr float kRescaleThreshold = 8.0f;   // log2 units
 
-// Orders a wave's LDS writes before its own later LDS reads (other lanes of
-// the same wave read what a lane wrote).  A wave's LDS operations execute in
-// program order, so no wait is needed for that: the fences are at wavefront
-// scope, which keeps the compiler from moving LDS accesses across this point
-// and emits no s_waitcnt.  (Workgroup scope made every such point wait for
-// the wave's LDS writes to complete: 1.3 % slower at config 4.)  Never used
-// for data passed between waves; that takes lds_barrier().
-__device__ __forceinline__ void wave_sync() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
 // Code word -> B operand of tile M (four dwords of two bf16 each).  Element j
 // of the tile sits at bit 8M + 2(j/2) of the low (j even) or high (j odd)
 // half of the word; dword k keeps bits 2k..2k+1 of each half of the word
@@ -121,42 +108,6 @@ constexpr int kProdExp = 64;
 constexpr float kProdUnit = 0x1p-64f;      // 2^-kProdExp
 constexpr float kProdScale = 0x1p64f;      // 2^kProdExp
 static_assert(kCodeExp - kProdExp == 69, "code scale constants below");
-
-template <int CTRL>
-__device__ __forceinline__ float dpp(float v) {
-    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(
-        0, __builtin_bit_cast(int, v), CTRL, 0xF, 0xF, false));
-}
-
-// Reductions across the 16 lanes of a DPP row (row_ror 8, 4, 2, 1).
-__device__ __forceinline__ float row_max16(float v) {
-    v = fmaxf(v, dpp<0x128>(v));
-    v = fmaxf(v, dpp<0x124>(v));
-    v = fmaxf(v, dpp<0x122>(v));
-    return fmaxf(v, dpp<0x121>(v));
-}
-
-__device__ __forceinline__ float row_sum16(float v) {
-    v += dpp<0x128>(v);
-    v += dpp<0x124>(v);
-    v += dpp<0x122>(v);
-    return v + dpp<0x121>(v);
-}
-
-// Across the wave: DPP within each 16-lane row, then the four row results
-// through readlane.  (__shfl_xor compiles to ds_bpermute, a chain of six LDS
-// round trips.)
-__device__ __forceinline__ float lane_f(float v, int l) {
-    return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), l));
-}
-__device__ __forceinline__ float wave_max(float v) {
-    v = row_max16(v);
-    return fmaxf(fmaxf(lane_f(v, 0), lane_f(v, 16)), fmaxf(lane_f(v, 32), lane_f(v, 48)));
-}
-__device__ __forceinline__ float wave_sum(float v) {
-    v = row_sum16(v);
-    return (lane_f(v, 0) + lane_f(v, 16)) + (lane_f(v, 32) + lane_f(v, 48));
-}
 
 // A per-lane LDS address, computed once and kept in a VGPR (PIN).  Left to
 // itself the compiler rebuilds such addresses (a multiply and an add of the

@@ -40,36 +40,6 @@ constexpr int kPlainWaves = 4, kPlainBlock = kPlainWaves * kWave;
 constexpr int kPassTokens = 16;
 constexpr float kMaxMove = 8.0f;       // log2 units: the running maximum moves beyond this
 
-template <int CTRL>
-__device__ __forceinline__ float dpp_add(float v) {
-    return v + __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(
-                   0, __builtin_bit_cast(int, v), CTRL, 0xF, 0xF, false));
-}
-template <int CTRL>
-__device__ __forceinline__ float dpp_max(float v) {
-    return fmaxf(v, __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(
-                        0, __builtin_bit_cast(int, v), CTRL, 0xF, 0xF, false)));
-}
-__device__ __forceinline__ float row_sum(float v) {          // over 16 lanes
-    return dpp_add<0x121>(dpp_add<0x122>(dpp_add<0x124>(dpp_add<0x128>(v))));
-}
-__device__ __forceinline__ float lane_of(float v, int l) {
-    return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), l));
-}
-__device__ __forceinline__ float all_sum(float v) {
-    v = row_sum(v);
-    return (lane_of(v, 0) + lane_of(v, 16)) + (lane_of(v, 32) + lane_of(v, 48));
-}
-__device__ __forceinline__ float all_max(float v) {
-    v = dpp_max<0x121>(dpp_max<0x122>(dpp_max<0x124>(dpp_max<0x128>(v))));
-    return fmaxf(fmaxf(lane_of(v, 0), lane_of(v, 16)), fmaxf(lane_of(v, 32), lane_of(v, 48)));
-}
-__device__ __forceinline__ void wave_order() {      // a wave's LDS writes before its later reads
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
 // acc[h] += sum of the word's 16 codes times f[h][0..15]: byte b, bits 2k hold
 // element 4b + k.
 template <int HG>
@@ -209,7 +179,7 @@ __attribute__((amdgpu_waves_per_eu(plain_waves(HG, N, J)))) void attn_plain_kern
     // score is -inf).
     auto weigh = [&](int h, float s, bool on) {
         if (__builtin_amdgcn_ballot_w64(on && s > m[h] + kMaxMove)) {
-            const float top = all_max(on ? s : -INFINITY);
+            const float top = wave_max(on ? s : -INFINITY);
             const float f = exp2_fast(m[h] - top);
             m[h] = top;
             l[h] *= f;
@@ -258,8 +228,8 @@ __attribute__((amdgpu_waves_per_eu(plain_waves(HG, N, J)))) void attn_plain_kern
             }
         }
 #pragma unroll
-        for (int h = 0; h < HG; ++h) bias[h] = all_sum(bias[h]);
-        wave_order();
+        for (int h = 0; h < HG; ++h) bias[h] = wave_sum(bias[h]);
+        wave_sync();
         float s[HG];
 #pragma unroll
         for (int h = 0; h < HG; ++h) s[h] = 0.f;
@@ -274,15 +244,15 @@ __attribute__((amdgpu_waves_per_eu(plain_waves(HG, N, J)))) void attn_plain_kern
         const bool on = tok && pos >= kv_lo && !(hid_row && position_hidden(hid_row, pos));
 #pragma unroll
         for (int h = 0; h < HG; ++h) {
-            if (lpt > 1) s[h] = dpp_add<0xB1>(s[h]);           // quad_perm [1,0,3,2]
-            if (lpt > 2) s[h] = dpp_add<0x4E>(s[h]);           // quad_perm [2,3,0,1]
+            if (lpt > 1) s[h] += dpp<0xB1>(s[h]);           // quad_perm [1,0,3,2]
+            if (lpt > 2) s[h] += dpp<0x4E>(s[h]);           // quad_perm [2,3,0,1]
             const float w = weigh(h, s[h] + bias[h], on);
             if (part == 0) {
                 l[h] += w;
                 if (tok) sp[h * kWave + kt] = w;
             }
         }
-        wave_order();
+        wave_sync();
 #pragma unroll
         for (int j = 0; j < J; ++j) {
             const int e = lane + kWave * j;
@@ -291,7 +261,7 @@ __attribute__((amdgpu_waves_per_eu(plain_waves(HG, N, J)))) void attn_plain_kern
             for (int h = 0; h < HG; ++h) {
                 const float p = in ? sp[h * kWave + e_p[j]] : 0.f;
                 // 16 lanes hold the 16 tokens of one dword of the group
-                const float z = row_sum(in ? p * vz[j] : 0.f);
+                const float z = row_sum16(in ? p * vz[j] : 0.f);
                 if (in) {
                     pv[h * pv_h + e_pv[j]] = p * vs[j];
                     if (lane % 16 == 0) zc[h * zc_h + e / 16] = z;
@@ -299,7 +269,7 @@ __attribute__((amdgpu_waves_per_eu(plain_waves(HG, N, J)))) void attn_plain_kern
             }
         }
         load_keys(next);
-        wave_order();
+        wave_sync();
 #pragma unroll
         for (int i = 0; i < N; ++i) {
             float acc[HG];
@@ -347,17 +317,18 @@ __attribute__((amdgpu_waves_per_eu(plain_waves(HG, N, J)))) void attn_plain_kern
             }
             const int pos = a.n_chunks * G + t0 + tk;
             const bool seen = tk < n && pos >= kv_lo && !(hid_row && position_hidden(hid_row, pos));
-            wave_order();                  // the previous pass's weights have been read
+            wave_sync();                  // the previous pass's weights have been read
 #pragma unroll
             for (int h = 0; h < HG; ++h) {
-                s[h] = dpp_add<0x4E>(dpp_add<0xB1>(s[h]));
+                s[h] += dpp<0xB1>(s[h]);
+                s[h] += dpp<0x4E>(s[h]);
                 const float w = weigh(h, s[h], seen && t0 + tk < a.qr.visible(h, a.res_len));
                 if (qq == 0) {
                     l[h] += w;
                     sp[h * kWave + tk] = w;
                 }
             }
-            wave_order();
+            wave_sync();
             if (ts < ts_n) {
                 for (int t = ts; t < n; t += ts_n) {
                     const float4 v = wide(a.v_res, row(t) + 4 * c4);
@@ -381,9 +352,9 @@ __attribute__((amdgpu_waves_per_eu(plain_waves(HG, N, J)))) void attn_plain_kern
     }
 
     // ---- the wave's state in its LDS region: o [HG][D], m [HG], l [HG] ---------
-    wave_order();
+    wave_sync();
     for (int e = lane; e < HG * D; e += kWave) mine[e] = 0.f;
-    wave_order();
+    wave_sync();
     for (int w = 0; w < gw; ++w) {         // a channel's dwords lie in different lanes
 #pragma unroll
         for (int i = 0; i < N; ++i) {
@@ -393,7 +364,7 @@ __attribute__((amdgpu_waves_per_eu(plain_waves(HG, N, J)))) void attn_plain_kern
                 for (int h = 0; h < HG; ++h) mine[h * D + e / gw] += o[i][h];
             }
         }
-        wave_order();
+        wave_sync();
     }
     for (int s = 0; s < ts_n; ++s) {
         if (ts == s) {
@@ -403,11 +374,11 @@ __attribute__((amdgpu_waves_per_eu(plain_waves(HG, N, J)))) void attn_plain_kern
                 for (int i = 0; i < 4; ++i) mine[h * D + 4 * c4 + i] += ow[h][i];
             }
         }
-        wave_order();
+        wave_sync();
     }
 #pragma unroll
     for (int h = 0; h < HG; ++h) {
-        const float sum = all_sum(l[h]);
+        const float sum = wave_sum(l[h]);
         if (lane == 0) {
             mine[HG * D + h] = m[h];
             mine[HG * D + HG + h] = sum;

@@ -1076,14 +1076,6 @@ struct WaveShape {
     static constexpr int LDS = kWaveWaves * (STATE > META ? STATE : META);
 };
 
-// Orders a wave's LDS writes before its own later reads (a wave's LDS
-// operations execute in order, so no wait is needed).
-__device__ __forceinline__ void wave_fence() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
 // A lane's loads of one packed unit.  A key word is used as it lies (two
 // tiles).  A lane's value operand holds tokens 4gq..+3 and 16+4gq..+3, half
 // of what the words of lane groups gq/2 (va) and 2 + gq/2 (vb) hold.
@@ -1191,9 +1183,9 @@ __device__ bool walk_wave(const RowsLaunch& a, unsigned char* smem, const Range&
         for (int u = rg.begin + wave; u < rg.c_end; u += kWaveWaves) {
             const uint32_t hid = rg.hidden(u);
             const int next = min(u + kWaveWaves, rg.c_end - 1);
-            wave_fence();                      // the previous unit's reads come first
+            wave_sync();                      // the previous unit's reads come first
             unit.stage_meta(mt, lane, ng);
-            wave_fence();
+            wave_sync();
             unit.load_meta(a, bh, next, lane, ng);
             f32x4_t s[2][RT];
 #pragma unroll

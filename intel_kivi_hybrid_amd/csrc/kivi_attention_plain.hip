@@ -25,8 +25,8 @@
 // conversion), then what a wave pays once (a third of its time at 4 chunks per
 // wave).  Measured (MI355X, head_dim 96, G = 32, 4K context, B=4, 32/32 heads):
 // 112 us per call with the generic kernel, which read each factor from LDS
-// singly and kept half of the lanes idle, 30 us with this one (kernel 25 us,
-// merge 4 us; 57.7 MB, 2.2 TB/s in the kernel).
+// singly and kept half of the lanes idle, 29 us with this one (kernel 24 us,
+// merge 4.7 us; 57.7 MB, 2.4 TB/s in the kernel).
 #include <math.h>
 
 #include "kivi_attention.hpp"

@@ -29,8 +29,11 @@
 //   (~2^-24 relative); packed values' offsets take three products of two
 //   pieces (~2^-17 of p vs per token, averaged over the context), their
 //   groups' middles and window values six of three: a common part of the
-//   values, which does not average out, keeps fp32's precision.  The softmax is online in fp32, in the log2 domain; its maximum
-//   moves only when exceeded by more than 8 (weights <= 256).
+//   values, which does not average out, keeps fp32's precision (32/8 heads, 2K
+//   tokens, fp32, error relative to float64: zero-mean values 4.2e-6, with an
+//   offset of 20 sigma 1.7e-7; the decode launches 7.5e-6 and 4.9e-7).  The softmax
+//   is online in fp32, in the log2 domain; its maximum moves only when exceeded by
+//   more than 8 (weights <= 256).
 // * Elements that are not finite as bf16 have no pieces (inf - inf): every sum
 //   that they enter comes out NaN.  A workgroup whose window sums come out NaN
 //   walks its range again with the window in plain fp32 (Rows::plain_unit):
@@ -45,10 +48,10 @@
 // * attn_rows_wave_kernel (few rows): each wave takes units of its own and
 //   expands them straight into its operand registers.
 //
-// Measured (MI355X, 32/8 heads, head_dim 128, bf16 ring and queries; the decode
-// kernel's launches before, this file's after): 512 query tokens over 8.1K
-// packed tokens, B=1: 256 launches, 4.84 ms -> 229 us; 5 tokens over 4K, B=8: 3
-// launches, 85.6 -> 52.7 us.
+// Measured (MI355X, 32/8 heads, head_dim 128, us per call; the decode kernel's
+// launches before, this file's after): 512 query tokens over 8.1K packed tokens,
+// B=1: 256 launches, 4810 -> 233, fp32 queries 4740 -> 340; 5 tokens over 4K, B=8: 3
+// launches, 78 -> 45, fp32 77 -> 49.
 #include <float.h>
 #include <math.h>
 
@@ -91,9 +94,8 @@ __device__ __forceinline__ int64_t query_offset(const RowsLaunch& a, int b, int 
 
 // Queries and outputs are in the caller's type, read and written here: a bf16
 // model's step otherwise pays up to three more launches (q widened, q made
-// token-major, the output rounded).  A layer's step, 32/8 heads, head_dim 128:
-// 5 query tokens, 4K context, B=8 51.2 -> 44.0 us; 512 tokens, 8.1K, B=1
-// 227.9 -> 217.5 us.
+// token-major, the output rounded), 7 us of 51 for 5 query tokens over 4K, B=8,
+// 10 of 228 for 512 tokens over 8.1K, B=1 (32/8 heads, head_dim 128).
 // f(load) with load(i): elements i .. i + 3 of the queries, widened exactly.
 // (one branch around all loads: a branch per load would wait for each)
 template <class F>
@@ -563,14 +565,14 @@ struct Range {
 // ---------------------------------------------------------------------------
 // Many rows: units expanded into LDS by the whole workgroup.
 //
-// What bounds it: a wave's step is 96 matrix products (1536 cycles) of two row
-// tiles, ~270 vector instructions and 40 KB of LDS reads; two waves per SIMD
-// take ~6100 cycles per step, the products 3100 of them, the LDS reads 2600
-// (each 1 KB operand feeds two row tiles).  Also measured for 512 query
-// tokens (215 us kernel time): 4 waves with 128 rows and two workgroups per
-// CU 264 us; 4 waves with four row tiles each (half the LDS reads, one wave
-// per SIMD, 66 registers spilled) 295 us; a raised priority for half of the
-// waves 224 us.
+// What bounds it: a wave's step is 102 matrix products (1632 cycles) of two row
+// tiles, ~300 vector instructions and 41 KB of LDS reads; two waves per SIMD
+// take ~6400 cycles per step, the products 3260 of them (47 % of all SIMD cycles
+// with prologue and window), the LDS reads 2600 (each 1 KB operand feeds two row
+// tiles).  Also measured for 512 query tokens, before the middles' tile (215 us
+// kernel time then): 4 waves with 128 rows and two workgroups per CU 264 us; 4
+// waves with four row tiles each (half the LDS reads, one wave per SIMD, 66
+// registers spilled) 295 us; a raised priority for half of the waves 224 us.
 // ---------------------------------------------------------------------------
 template <int D>
 struct SharedShape {
@@ -959,7 +961,7 @@ __device__ bool walk_shared(const RowsLaunch& a, unsigned char* smem, const Rang
             } else {
                 // (as a loop: as plain code the compiler moves what both arms
                 // share above the branch, where it waits for unit's loads
-                // before any product: 36 rows, B=16 58 -> 68 us)
+                // before any product: 36 rows over 2K, B=16 68 us, so 61)
                 int once = 1;
                 asm volatile("" : "+s"(once));
 #pragma unroll 1
@@ -1056,10 +1058,10 @@ void attn_rows_shared_kernel(RowsLaunch a) {
 // Few rows: each wave expands units of its own into its registers, with no
 // barrier and no LDS traffic but the scales.
 //
-// What bounds it: the expansion's vector work, ~800 instructions per unit
-// (4-5.5 cycles each) against 1536 cycles of matrix products for two row tiles;
-// two workgroups per CU gain little over one (39 against 42 us at B=8, 5 query
-// tokens over 4K).
+// What bounds it: the expansion's vector work, ~1000 instructions per unit
+// (4-5.5 cycles each) against 1728 cycles of matrix products for two row tiles
+// (17 % of all SIMD cycles); two workgroups per CU gain little over one (39
+// against 42 us at B=8, 5 query tokens over 4K, with ~100 instructions less).
 // ---------------------------------------------------------------------------
 constexpr int kWaveWaves = 4, kWaveBlock = kWaveWaves * kWave;
 
@@ -1455,10 +1457,11 @@ __global__ __launch_bounds__(256) void attn_rows_merge_kernel(RowsLaunch a) {
 }
 
 // Rows per kv head that the wave kernel takes: those of one workgroup, and at
-// head_dim 64 of two.  Kernel times, wave / shared (rows, B): head_dim 128: 36
-// rows 71 / 55 us (B=8, 4K), 26 / 26 (B=1, 8K); 64 rows 70 / 58, 28 / 28;
-// head_dim 64 (B=8, 12 heads, 2K): 40 rows 36 / 46 us, 64 rows 37 / 47, 100
-// rows 59 / 54.
+// head_dim 64 of two.  us per call, wave / shared, bf16 (fp32 queries alike):
+// head_dim 128 (B=8, 4K; B=1, 8K) 32 rows 48 / 58, 31 / 32, 36 rows 67 / 60, 42 /
+// 32, 64 rows 68 / 63, 44 / 35; head_dim 64 (B=8, 12 heads, 2K) 40 rows 45 / 51, 64
+// rows 47 / 55, 80 rows 66 / 56; head_dim 256 (B=4, 4K) 16 rows 38 / 52, 24 rows
+// 63 / 55.
 int few_rows(int D) { return D <= 64 ? 64 : D <= 128 ? 32 : 16; }
 
 template <int D, bool R16>
